@@ -23,6 +23,7 @@ from ._lib import check, lib, ptr, stream_ptr
 from .constants import C_0, EPSILON_0
 
 NSTATE = 18
+TM_ARRAYS = [0, 1, 5, 6, 7, 17]   # Hx, Hy, Dz, ICEx, ICEy, IDz: the live arrays of a 2D TM run
 COMPONENTS = {'Ex': 0, 'Ey': 1, 'Ez': 2, 'Dx': 3, 'Dy': 4, 'Dz': 5, 'Hx': 6, 'Hy': 7, 'Hz': 8}
 _CODE = {torch.float32: _lib.CV_C64, torch.float64: _lib.CV_C128}  # CV_F32 == 0, CV_F64 == 1
 
@@ -136,6 +137,37 @@ class FdtdGrid:
                                    int(src_cell), ptr(amp_dev), int(t0), int(n_steps), ptr(pc), ptr(pl), npb,
                                    ptr(rec), int(rec_t0), int(config), stream_ptr()), 'fdtd run_tm')
         return state
+
+    def run_tm_checkpoints(self, state, eps, src_cell, amp_dev, n_steps, ck, probes, rec, config):
+        """run_tm from step 0 (``state`` advanced in place); returns the TM
+        arrays before every ``ck``-th step, (segments, 6, nx, ny)."""
+        nseg = -(-n_steps // ck)
+        new = lambda k: torch.empty((k, len(TM_ARRAYS), self.nx, self.ny), dtype=self.dtype, device=self.device)
+        ckpt, work = new(nseg), new(2)
+        pc, pl = probes
+        check(lib().cv_fdtd_run_tm_checkpoints(self.code, self._d(), ptr(self.sig), ptr(eps), ptr(state), ptr(work),
+                                               ptr(ckpt), int(ck), int(src_cell), ptr(amp_dev), int(n_steps), ptr(pc),
+                                               ptr(pl), int(pc.numel()), ptr(rec), int(config), stream_ptr()),
+              'fdtd run_tm_checkpoints')
+        return ckpt
+
+    def tm_adjoint(self, ckpt, ck, eps, src_cell, amp_dev, n_steps, probes, g_final, g_rec, g_amp, gmEz, config):
+        """Reverse the run of run_tm_checkpoints; returns the cotangent of the
+        TM arrays of its initial state (6, nx, ny).  g_final: that of the
+        final state's TM arrays or None."""
+        new = lambda *k: torch.empty(k + (self.nx, self.ny), dtype=self.dtype, device=self.device)
+        na = len(TM_ARRAYS)
+        work, hist, lam = new(2, na), new(min(ck, n_steps)), new(2, na)
+        if g_final is None:
+            lam[0].zero_()
+        else:
+            lam[0].copy_(g_final)
+        pc, pl = probes
+        check(lib().cv_fdtd_tm_adjoint(self.code, self._d(), ptr(self.sig), ptr(eps), ptr(ckpt), int(ck),
+                                       int(src_cell), ptr(amp_dev), int(n_steps), ptr(work), ptr(hist), ptr(lam),
+                                       ptr(gmEz), ptr(pc), ptr(pl), int(pc.numel()), ptr(g_rec), ptr(g_amp),
+                                       int(config), stream_ptr()), 'fdtd tm_adjoint')
+        return lam[0]
 
     def run_fused(self, state, other, eps, comp, src_cell, amp_dev, t0, n_steps, probes, rec, rec_t0):
         """Fused single-pass steps ping-ponging between ``state`` and ``other``;
@@ -323,6 +355,13 @@ class FdtdRun(torch.autograd.Function):
         need_grad = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
         checkpoints = []
         t = 0
+        if need_grad and isinstance(tm_config, int) and n_steps > 0:
+            # whole launches per segment: the next lower multiple of the steps
+            # a launch takes (a checkpoint is a third of a full state)
+            ts = tm_configs()[tm_config][2]
+            ck = min(ck - ck % ts if ck > ts else ck, n_steps)
+            checkpoints = grid.run_tm_checkpoints(state, eps, src[1], amp_dev, n_steps, ck, probes, rec, tm_config)
+            t = n_steps
         while t < n_steps:
             m = min(ck, n_steps - t) if need_grad else n_steps - t
             if need_grad:
@@ -341,6 +380,7 @@ class FdtdRun(torch.autograd.Function):
         ctx.state0 = state0.detach().clone()
         ctx.save_for_backward(eps)
         ctx.save_for_forward(eps)
+        ctx.set_materialize_grads(False)
         return rec, state
 
     @staticmethod
@@ -365,6 +405,12 @@ class FdtdRun(torch.autograd.Function):
     def backward(ctx, grec, gstate_final):
         (eps,) = ctx.saved_tensors
         grid, src, probes, n_steps, ck = ctx.grid, ctx.src, ctx.probes, ctx.n_steps, ctx.ck
+        tm = isinstance(ctx.tm_config, int)
+        # A TM run's TE components are zero, so their cotangents reach neither
+        # eps nor the amplitude: they matter only for the initial state's
+        # gradient when the final state has one.
+        if tm and n_steps > 0 and (gstate_final is None or not ctx.needs_input_grad[3]):
+            return FdtdRun._backward_tm(ctx, eps, grec, gstate_final)
         lam = grid.new_state()
         if gstate_final is not None:
             lam += gstate_final
@@ -378,7 +424,11 @@ class FdtdRun(torch.autograd.Function):
         for sgi in range(nseg - 1, -1, -1):
             t0 = sgi * ck
             m = min(ck, n_steps - t0)
-            st = ctx.checkpoints[sgi].clone()
+            if tm:
+                st = grid.new_state()
+                st[TM_ARRAYS] = ctx.checkpoints[sgi].unsqueeze(-1)
+            else:
+                st = ctx.checkpoints[sgi].clone()
             Dhist[0].copy_(st[3:6])
             for s in range(m):
                 if isinstance(ctx.tm_config, int):
@@ -397,13 +447,35 @@ class FdtdRun(torch.autograd.Function):
                     grid.adjoint(lam, eps, Dhist[s], gmE, src=src, g_src=ga)
             del st
         geps = grid.eps_grad(eps, gmE, torch.zeros_like(eps)) if ctx.needs_input_grad[0] else None
-        g_amp = None
-        if gamp is not None:
-            shape, dtype, dev = ctx.amp_meta
-            g_amp = torch.zeros(shape, dtype=dtype, device=dev)
-            g_amp.view(-1)[:n_steps] = gamp.to(dev, dtype)
+        g_amp = FdtdRun._amp_grad(ctx, gamp)
         # lam now holds the cotangent of the state the run started from
         gstate0 = lam if ctx.needs_input_grad[3] else None
         # the checkpoints stay with the graph: a retained graph (one backward
         # per output row of a Jacobian) runs this more than once
         return geps, g_amp, None, gstate0, None, None, None, None, None
+
+    @staticmethod
+    def _amp_grad(ctx, gamp):
+        if gamp is None:
+            return None
+        shape, dtype, dev = ctx.amp_meta
+        g_amp = torch.zeros(shape, dtype=dtype, device=dev)
+        g_amp.view(-1)[:ctx.n_steps] = gamp.to(dev, dtype)
+        return g_amp
+
+    @staticmethod
+    def _backward_tm(ctx, eps, grec, gstate_final):
+        """The whole reverse sweep of a TM run in one call."""
+        grid, n_steps = ctx.grid, ctx.n_steps
+        gmE = torch.zeros((3,) + grid.shape, dtype=grid.dtype, device=grid.device)
+        gamp = torch.zeros(n_steps, dtype=grid.dtype, device=grid.device) if ctx.needs_input_grad[1] else None
+        grec = grec.to(grid.dtype).contiguous() if grec is not None else None
+        g_final = None if gstate_final is None else gstate_final[TM_ARRAYS].squeeze(-1)
+        lam = grid.tm_adjoint(ctx.checkpoints, ctx.ck, eps, ctx.src[1], ctx.amp_dev, n_steps, ctx.probes, g_final,
+                              grec, gamp, gmE[2], ctx.tm_config)
+        geps = grid.eps_grad(eps, gmE, torch.zeros_like(eps)) if ctx.needs_input_grad[0] else None
+        gstate0 = None
+        if ctx.needs_input_grad[3]:
+            gstate0 = grid.new_state()
+            gstate0[TM_ARRAYS] = lam.unsqueeze(-1)
+        return geps, FdtdRun._amp_grad(ctx, gamp), None, gstate0, None, None, None, None, None

@@ -17,6 +17,7 @@
 
 #include <vector>
 #include <algorithm>
+#include <type_traits>
 
 namespace cv {
 
@@ -25,7 +26,7 @@ struct Fdtd {
     int nx, ny, nz;
     int64_t n;
     R inv_dL;
-    double dt, c0, eps0;
+    double dt, c0, eps0, dL;
     const R* sig;      // sigHx[nx] sigHy[ny] sigHz[nz] sigDx[nx] sigDy[ny] sigDz[nz]
     const R* eps;      // relative permittivity, n
     R* st;             // 18 * n
@@ -519,34 +520,60 @@ __global__ void __launch_bounds__(256) k_efields_grad(Fdtd<R> f, const R* __rest
 }
 
 // ================================================ 2D TM temporal blocking
-// Fused, temporally blocked Yee update for nz == 1 with only Hx, Hy, Dz live
-// (TM drive: Jz point source, TE fields zero).  One workgroup of WV waves owns
-// a region of RR = WV*RPT rows (x) by 64 columns (y, contiguous): lane =
-// column, each wave a band of RPT rows.  Cell values (Hx, Hy, Dz, 1/eps and the PML integrals
-// ICEx, ICEy, IDz) live in registers; neighbour values are exchanged through
-// LDS.  TS steps are advanced per launch; after TS steps the cells at least TS
-// away from the region edge are exact (the dependency cone of one step is one
-// cell on each side), so the owned tile is the region minus a TS-wide halo.
-// Region loads use periodic indices, which also makes small domains exact.
+// Temporally blocked Yee update for nz == 1 with only Hx, Hy, Dz live (TM
+// drive: Jz point source, TE fields zero), and its reverse-time adjoint.  One
+// workgroup of WV waves owns a region of RR = WV*RPT rows (x) by 64 columns
+// (y, contiguous): lane = column, each wave a band of RPT rows, all values of
+// a cell in registers.  A neighbour along y is the next lane (DPP wave
+// shift), a neighbour along x the next register, and only the rows where two
+// waves meet go through LDS (one row of Ez and one of Hy per wave and step).
+// TS steps are advanced per launch; after TS steps the cells at least TS away
+// from the region edge are exact (the dependency cone of one step is one cell
+// on each side, in either direction of time), so the owned tile is the region
+// minus a TS-wide halo.  Region loads use periodic indices, which also makes
+// small domains exact; what enters at the region's outer edge is zero.
+//
+// Bound: vector instructions of the region (halo included) on the one
+// workgroup a CU holds.  Tiles without PML run a loop of 10 vector operations
+// per cell and step, tiles with PML one of 18.  400 x 400 float32 in 16-step
+// launches: 18.2 us a launch (0.7 us a step over a prologue of 6.5 us; 25.8
+// us with every neighbour through LDS, 30 operations a cell and an amplitude
+// load in each step).
+struct TmProbes {
+    const int32_t* comp;       // 2 Ez, 6 Hx, 7 Hy
+    const int64_t* cell;       // flat cells
+    int n;
+};
+
+// The six arrays a TM state is made of.
+template <typename R>
+struct TmState {
+    R *hx, *hy, *dz, *icex, *icey, *idz;
+};
+
 template <typename R>
 struct TmArgs {
     int nx, ny;
     int tiles_x, tiles_y;      // tile grid
     int t0, nsteps;            // first global step of this launch, steps (<= TS)
-    int64_t src;               // flat source cell or -1
-    int np;                    // probes
-    R inv_dL;
-    R h1, h2, d1, d2;          // interior coefficients
-    double dt, c0, eps0;
+    int src_i, src_j;          // source cell, src_i = -1: none
+    R inv_dL, dL;
+    R cdt;                     // c0 dt / dL
+    R half_dt;                 // dt / (2 eps0)
     const R* sig;
     const R* eps;
-    const R* st_in;            // state at the start of the launch (18 arrays)
-    R* st_out;                 // state after the launch (a different buffer)
+    TmState<R> in, out;        // distinct buffers
     const double* amp;         // amplitude per global step
-    const int32_t* pcomp;      // probe components: 2 Ez, 6 Hx, 7 Hy
-    const int64_t* pcell;      // probe flat cells
+    TmProbes probes;
     R* rec;                    // (steps, np), row t - rec_t0
     int rec_t0;
+    R* hist;                   // Dz after step t0 + s at hist + s * n, or null
+    // adjoint only: in / out hold the cotangent of the state after / before the steps
+    const R* dz_hist;          // Dz after step t0 + s at dz_hist + s * n
+    const R* dz_before;        // Dz before step t0
+    R* gm;                     // accumulated cotangent of 1 / eps_zz
+    const R* grec;             // cotangent of rec, row t (global step), or null
+    R* gamp;                   // cotangent of the amplitude of global step t, or null
 };
 
 __host__ __device__ __forceinline__ int pmod(int a, int n) {
@@ -554,264 +581,648 @@ __host__ __device__ __forceinline__ int pmod(int a, int n) {
     return r < 0 ? r + n : r;
 }
 
+constexpr int kTmConfigs = 12;
 constexpr int kTmMaxProbes = 256;
+constexpr unsigned short kTmNoProbe = 0xffff;
+
+// The value of the lane above (lane + 1) or below (lane - 1); 0 beyond the wave.
+template <int CTRL>
+__device__ __forceinline__ float wave_shift(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double wave_shift(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+template <typename R>
+__device__ __forceinline__ R lane_above(R v) { return wave_shift<0x130>(v); }   // wave_shl:1
+template <typename R>
+__device__ __forceinline__ R lane_below(R v) { return wave_shift<0x138>(v); }   // wave_shr:1
+
+// A value that is the same in every lane, kept in scalar registers.
+__device__ __forceinline__ float uniform(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ double uniform(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// The value of lane s (uniform).
+__device__ __forceinline__ float read_lane(float v, int s) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), s));
+}
+__device__ __forceinline__ double read_lane(double v, int s) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, s);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), s);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// Probes inside a tile's region.  tm_probe_slots enters every probe whose cell
+// lies in the region (in each of its periodic copies) into s_slot[component][row][column];
+// of several probes of one component and cell the last one is entered and
+// s_next leads to the one before it.  Returns (uniformly) whether there is any.
+template <int RR, int NT>
+__device__ __forceinline__ bool tm_probe_slots(const TmProbes& pr, int nx, int ny, int i0, int j0,
+                                               unsigned short (*s_slot)[RR][64], unsigned short* s_next, int* s_any) {
+    if (pr.n == 0) return false;
+    if (threadIdx.x == 0) *s_any = 0;
+    __syncthreads();
+    int pi = 0, pj = 0;
+    bool mine = false;
+    const int p = threadIdx.x;
+    static_assert(NT >= kTmMaxProbes, "one thread per probe");
+    if (p < pr.n) {
+        const int64_t c = pr.cell[p];
+        if ((uint64_t)c <= 0xffffffffull) {   // a 64-bit division is a long sequence
+            pi = (int)((uint32_t)c / (uint32_t)ny);
+            pj = (int)((uint32_t)c - (uint32_t)pi * (uint32_t)ny);
+        } else {
+            pi = (int)(c / ny);
+            pj = (int)(c - (int64_t)pi * ny);
+        }
+        mine = pmod(pi - i0, nx) < RR && pmod(pj - j0, ny) < 64;
+        if (mine) *s_any = 1;
+    }
+    __syncthreads();
+    if (!*s_any) return false;   // uniform
+    for (int q = threadIdx.x; q < 3 * RR * 64; q += NT) (&s_slot[0][0][0])[q] = kTmNoProbe;
+    __syncthreads();
+    if (mine) {
+        const int k = pr.comp[p];
+        const int64_t c = pr.cell[p];
+        int before = kTmNoProbe;
+        bool head = true;
+        for (int m = 0; m < pr.n; ++m) {
+            if (pr.comp[m] != k || pr.cell[m] != c) continue;
+            if (m < p) before = m;
+            if (m > p) head = false;
+        }
+        s_next[p] = (unsigned short)before;
+        const int kk = k == 2 ? 0 : k - 5;
+        if (head)
+            for (int r = pmod(pi - i0, nx); r < RR; r += nx)
+                for (int col = pmod(pj - j0, ny); col < 64; col += ny) s_slot[kk][r][col] = (unsigned short)p;
+    }
+    __syncthreads();
+    return true;
+}
+
+// v modulo n for -n < v < 2 n without a division; tiles reach beyond the grid
+// by less than 64 cells, so that holds for every n >= 64.
+__device__ __forceinline__ int tm_wrap(int v, int n) {
+    if (n < 64) return pmod(v, n);   // uniform
+    v += v < 0 ? n : 0;
+    return v - (v >= n ? n : 0);
+}
+
+// 1 / v: the hardware's estimate (1 ulp) and one Newton step in float32
+__device__ __forceinline__ float tm_recip(float v) {
+    const float r = __builtin_amdgcn_rcpf(v);
+    const float s = __builtin_fmaf(__builtin_fmaf(-v, r, 1.0f), r, r);
+    return __builtin_isfinite(s) ? s : r;   // 1 / 0 and 1 / inf
+}
+__device__ __forceinline__ double tm_recip(double v) { return 1.0 / v; }
+
+// Geometry and coefficients of this thread's cells.  With b = sigma dt / (2
+// eps0) the coefficients of fdtd.py:272-311 separate by axis, 1/m0 = dt /
+// ((1 + b_b)(1 + b_c)), so two divisions per row and two per column serve
+// every cell; where sigma is zero m1 is 1 and m2 is c0 dt exactly.  The 1/dL
+// of the curls is folded into m2 and the own sigma's term is factored out:
+//   Hx = xa hx + xb (dEz_y + kx icx), xa, xb of the column, kx of the row
+//   Hy = ya hy + yb (dEz_x + ky icy), ya, yb of the row, ky of the column
+//   Dz = da dz + db dH + dc idz
+// with undivided differences dE, dH.  Rows are uniform over the wave and
+// kept in scalar registers.
+template <typename R, int RPT>
+struct TmCells {
+    int gi[RPT], gj;
+    R shx[RPT], shy, sdx[RPT], sdy;
+    R xa, xb, ky, ya[RPT], yb[RPT], kx[RPT];
+    R da[RPT], db[RPT], dc[RPT], me[RPT];
+    bool pml;   // any sigma of this thread's cells is non-zero
+
+    // base[cell]: the row is uniform over the wave, so the address is a scalar
+    // row pointer plus one vector offset for all rows
+    template <typename P>
+    __device__ __forceinline__ P& at(P* base, int q, int ny) const {
+        return (base + (int64_t)gi[q] * ny)[(uint32_t)gj];
+    }
+    __device__ __forceinline__ bool has_idz(int q) const { return sdx[q] != R(0) && sdy != R(0); }
+
+    // The prologue is paid once per launch by every wave of the CU, so it
+    // issues its loads before anything waits, wraps indices without divisions
+    // and forms the PML coefficients only where a sigma is non-zero.
+    __device__ __forceinline__ void place(const TmArgs<R>& a, int row0, int col) {
+        gj = tm_wrap(col, a.ny);
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) gi[q] = __builtin_amdgcn_readfirstlane(tm_wrap(row0 + q, a.nx));
+        // rows through scalar loads (constant address space)
+        using csig_t = const __attribute__((address_space(4))) R*;
+        const csig_t csig = (csig_t)a.sig;
+        shy = a.sig[a.nx + gj];
+        sdy = a.sig[2 * a.nx + a.ny + 1 + gj];
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            shx[q] = csig[gi[q]];
+            sdx[q] = csig[a.nx + a.ny + 1 + gi[q]];
+            me[q] = at(a.eps, q, a.ny);
+        }
+    }
+
+    __device__ __forceinline__ void init(const TmArgs<R>& a) {
+        R cy = R(0), ry = R(1);
+        xa = R(1); xb = -a.cdt; ky = R(0);
+        pml = shy != R(0) || sdy != R(0);
+        if (pml) {
+            const R by = shy * a.half_dt;
+            cy = sdy * a.half_dt;
+            ry = R(1) / (R(1) + cy);
+            const R h = R(1) / (R(1) + by);
+            xa = (R(1) - by) * h;
+            xb = -a.cdt * h;
+            ky = R(2) * by * a.dL;
+        }
+#pragma unroll
+        for (int q = 0; q < RPT; ++q) {
+            R cx_ = R(0), rx = R(1);
+            ya[q] = R(1); yb[q] = -a.cdt; kx[q] = R(0);
+            if (shx[q] != R(0) || sdx[q] != R(0)) {   // uniform
+                pml = true;
+                const R bx = shx[q] * a.half_dt;
+                cx_ = sdx[q] * a.half_dt;
+                rx = R(1) / (R(1) + cx_);
+                const R h = R(1) / (R(1) + bx);
+                ya[q] = uniform((R(1) - bx) * h);
+                yb[q] = uniform(-a.cdt * h);
+                kx[q] = uniform(R(2) * bx * a.dL);
+            }
+            const R r = rx * ry, cc = cx_ * cy;
+            da[q] = (R(1) - cx_ - cy - cc) * r;
+            db[q] = a.cdt * r;
+            dc[q] = R(-4) * cc * r;
+            me[q] = tm_recip(me[q]);
+        }
+    }
+};
+
+// Tile of this workgroup: XCD-aware order, consecutive workgroups go to
+// different XCDs, so each XCD gets a contiguous run of tiles (halos re-read
+// from its own L2).
+__device__ __forceinline__ void tm_tile(int tiles_y, int& ti, int& tj) {
+    const int nb = gridDim.x;
+    int b = blockIdx.x;
+    if ((nb & 7) == 0) b = (b & 7) * (nb >> 3) + (b >> 3);
+    ti = b / tiles_y;
+    tj = b - ti * tiles_y;
+}
 
 template <typename R, int WV, int RPT, int TS>
 __global__ void __launch_bounds__(64 * WV) k_tm_block(TmArgs<R> a) {
     constexpr int RR = WV * RPT;
     constexpr int NT = 64 * WV;
-    constexpr int RC = 64;
-    constexpr int OX = RR - 2 * TS, OY = RC - 2 * TS;  // owned tile
-    __shared__ R sEz[RR][RC];
-    __shared__ R sHx[RR][RC];
-    __shared__ R sHy[RR][RC];
-    __shared__ int s_np;
-    __shared__ int s_pidx[kTmMaxProbes];
-    __shared__ short s_pr[kTmMaxProbes], s_pc[kTmMaxProbes], s_pk[kTmMaxProbes];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    // XCD-aware tile order: consecutive workgroups go to different XCDs, so
-    // give each XCD a contiguous run of tiles (better L2 reuse of halos).
-    const int nb = gridDim.x;
-    int b = blockIdx.x;
-    if ((nb & 7) == 0) b = (b & 7) * (nb >> 3) + (b >> 3);
-    const int ti = b / a.tiles_y, tj = b - ti * a.tiles_y;
+    constexpr int OX = RR - 2 * TS, OY = 64 - 2 * TS;  // owned tile
+    __shared__ R sEz[WV + 1][64];   // Ez of each wave's first row
+    __shared__ R sHy[WV + 1][64];   // new Hy of each wave's last row, at [wave + 1]
+    __shared__ unsigned short s_slot[3][RR][64];
+    __shared__ unsigned short s_next[kTmMaxProbes];
+    __shared__ int s_any;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int ti, tj;
+    tm_tile(a.tiles_y, ti, tj);
     const int i0 = ti * OX, j0 = tj * OY;
     const int nx = a.nx, ny = a.ny;
     const int64_t n = (int64_t)nx * ny;
-    const int gj = pmod(j0 - TS + lane, ny);
-    const R* sigHx = a.sig;
-    const R* sigHy = a.sig + nx;
-    const R* sigDx = a.sig + nx + ny + 1;
-    const R* sigDy = a.sig + 2 * nx + ny + 1;
-    const R shy = sigHy[gj], sdy = sigDy[gj];
-    // Tiles read their halo from st_in and write only their owned cells to
-    // st_out: a tile that finishes early never changes what a later tile of
+    TmCells<R, RPT> g;
+    g.place(a, i0 - TS + w * RPT, j0 - TS + lane);
+    // Tiles read their halo from `in` and write only their owned cells to
+    // `out`: a tile that finishes early never changes what a later tile of
     // the same launch reads.
-    const R* Hx = a.st_in;
-    const R* Hy = a.st_in + n;
-    const R* Dz = a.st_in + 5 * n;
-    const R* ICEx = a.st_in + 6 * n;
-    const R* ICEy = a.st_in + 7 * n;
-    const R* IDz = a.st_in + 17 * n;
-    R* oHx = a.st_out;
-    R* oHy = a.st_out + n;
-    R* oDz = a.st_out + 5 * n;
-    R* oICEx = a.st_out + 6 * n;
-    R* oICEy = a.st_out + 7 * n;
-    R* oIDz = a.st_out + 17 * n;
-    const R dt = R(a.dt), c0 = R(a.c0), e0 = R(a.eps0);
-
-    if (threadIdx.x == 0) s_np = 0;
-    __syncthreads();
-    for (int p = threadIdx.x; p < a.np; p += NT) {
-        const int64_t c = a.pcell[p];
-        const int pi = (int)(c / ny), pj = (int)(c - (int64_t)pi * ny);
-        const int ri = pi - i0, rj = pj - j0;
-        if (ri >= 0 && ri < OX && rj >= 0 && rj < OY) {
-            const int slot = atomicAdd(&s_np, 1);
-            if (slot < kTmMaxProbes) {
-                s_pidx[slot] = p;
-                s_pr[slot] = (short)(ri + TS);
-                s_pc[slot] = (short)(rj + TS);
-                s_pk[slot] = (short)a.pcomp[p];
-            }
-        }
-    }
-
-    R hx[RPT], hy[RPT], dz[RPT], me[RPT], icx[RPT], icy[RPT], idz[RPT], shx[RPT], sdx[RPT];
-    // update coefficients per cell, formed once per launch (the PML cells'
-    // divisions stay out of the time loop): Hx = xa hx + xb cex + xc icx,
-    // Hy likewise, Dz = da dz + db chz + dc idz; xc / yc / dc are 0 where the
-    // auxiliary term is absent, so one code path serves every cell.
-    R xa[RPT], xb[RPT], xc[RPT], ya[RPT], yb[RPT], yc[RPT], da[RPT], db[RPT], dc[RPT];
-    int gi[RPT];
+    R hx[RPT], hy[RPT], dz[RPT], ez[RPT], icx[RPT], icy[RPT], idz[RPT];
 #pragma unroll
     for (int q = 0; q < RPT; ++q) {
-        const int r = w * RPT + q;
-        gi[q] = pmod(i0 - TS + r, nx);
-        const int64_t c = (int64_t)gi[q] * ny + gj;
-        hx[q] = Hx[c];
-        hy[q] = Hy[c];
-        dz[q] = Dz[c];
-        const R e = a.eps[c];
-        me[q] = R(1) / ((e + e) / R(2));
-        shx[q] = sigHx[gi[q]];
-        sdx[q] = sigDx[gi[q]];
-        icx[q] = shx[q] != R(0) ? ICEx[c] : R(0);
-        icy[q] = shy != R(0) ? ICEy[c] : R(0);
-        idz[q] = (sdx[q] != R(0) && sdy != R(0)) ? IDz[c] : R(0);
-        sEz[r][lane] = me[q] * dz[q];
-        if (shx[q] == R(0) && shy == R(0)) {
-            xa[q] = a.h1; xb[q] = a.h2; xc[q] = R(0);
-            ya[q] = a.h1; yb[q] = a.h2; yc[q] = R(0);
-        } else {
-            R m1, m2, m3, m4;
-            coef4<R>(shx[q], shy, R(0), dt, c0, e0, R(-1), m1, m2, m3, m4);   // Hx: own sigma sHx
-            xa[q] = m1; xb[q] = m2; xc[q] = shx[q] != R(0) ? m3 : R(0);
-            coef4<R>(shy, shx[q], R(0), dt, c0, e0, R(-1), m1, m2, m3, m4);   // Hy: own sigma sHy
-            ya[q] = m1; yb[q] = m2; yc[q] = shy != R(0) ? m3 : R(0);
-        }
-        if (sdx[q] == R(0) && sdy == R(0)) {
-            da[q] = a.d1; db[q] = a.d2; dc[q] = R(0);
-        } else {
-            R m1, m2, m3, m4;
-            coef4<R>(R(0), sdx[q], sdy, dt, c0, e0, R(1), m1, m2, m3, m4);
-            da[q] = m1; db[q] = m2; dc[q] = (sdx[q] != R(0) && sdy != R(0)) ? m4 : R(0);
-        }
+        hx[q] = g.at(a.in.hx, q, ny);
+        hy[q] = g.at(a.in.hy, q, ny);
+        dz[q] = g.at(a.in.dz, q, ny);
     }
-    const int src_i = a.src >= 0 ? (int)(a.src / ny) : -1;
-    const int src_j = a.src >= 0 ? (int)(a.src - (int64_t)src_i * ny) : -1;
-    __syncthreads();
-    const int np_tile = min(s_np, kTmMaxProbes);
-
-    for (int s = 0; s < a.nsteps; ++s) {
-        const int t = a.t0 + s;
-        // ---- H update: CEx = (Ez[j+1] - Ez)/dL, CEy = -(Ez[i+1] - Ez)/dL
-#pragma unroll
-        for (int q = 0; q < RPT; ++q) {
-            const int r = w * RPT + q;
-            const R ez = me[q] * dz[q];
-            const R ez_ip = sEz[min(r + 1, RR - 1)][lane];
-            const R ez_jp = sEz[r][min(lane + 1, RC - 1)];
-            const R cex = ((ez_jp - ez) - (R(0) - R(0))) * a.inv_dL;
-            const R cey = ((R(0) - R(0)) - (ez_ip - ez)) * a.inv_dL;
-            icx[q] += cex;
-            icy[q] += cey;
-            R v = xa[q] * hx[q] + xb[q] * cex;
-            v += xc[q] * icx[q];
-            hx[q] = v;
-            v = ya[q] * hy[q] + yb[q] * cey;
-            v += yc[q] * icy[q];
-            hy[q] = v;
-            sHx[r][lane] = hx[q];
-            sHy[r][lane] = hy[q];
-        }
-        __syncthreads();
-        // ---- D update: CHz = (Hy - Hy[i-1])/dL - (Hx - Hx[j-1])/dL
-#pragma unroll
-        for (int q = 0; q < RPT; ++q) {
-            const int r = w * RPT + q;
-            const R hy_im = sHy[max(r - 1, 0)][lane];
-            const R hx_jm = sHx[r][max(lane - 1, 0)];
-            const R chz = ((hy[q] - hy_im) - (hx[q] - hx_jm)) * a.inv_dL;
-            idz[q] += dz[q];
-            R v = da[q] * dz[q] + db[q] * chz;
-            v += dc[q] * idz[q];
-            if (gi[q] == src_i && gj == src_j) v += R(a.amp[t]);
-            dz[q] = v;
-            sEz[r][lane] = me[q] * v;
-        }
-        __syncthreads();
-        if (np_tile > 0) {   // uniform over the workgroup
-            for (int p = threadIdx.x; p < np_tile; p += NT) {
-                const int k = s_pk[p];
-                const R v =
-                    (k == 2) ? sEz[s_pr[p]][s_pc[p]] : (k == 6 ? sHx[s_pr[p]][s_pc[p]] : sHy[s_pr[p]][s_pc[p]]);
-                a.rec[(int64_t)(t - a.rec_t0) * a.np + s_pidx[p]] = v;
-            }
-            __syncthreads();   // the next H phase overwrites sHx / sHy
-        }
-    }
-    // ---- store the owned tile
+    bool own[RPT], any_own = false;
     const int oj = lane - TS;
-    if (oj >= 0 && oj < OY && j0 + oj < ny) {
 #pragma unroll
-        for (int q = 0; q < RPT; ++q) {
-            const int r = w * RPT + q;
-            const int oi = r - TS;
-            if (oi < 0 || oi >= OX || i0 + oi >= nx) continue;
-            const int64_t c = (int64_t)(i0 + oi) * ny + (j0 + oj);
-            oHx[c] = hx[q];
-            oHy[c] = hy[q];
-            oDz[c] = dz[q];
-            if (shx[q] != R(0)) oICEx[c] = icx[q];
-            if (shy != R(0)) oICEy[c] = icy[q];
-            if (sdx[q] != R(0) && sdy != R(0)) oIDz[c] = idz[q];
+    for (int q = 0; q < RPT; ++q) {
+        icx[q] = g.shx[q] != R(0) ? g.at(a.in.icex, q, ny) : R(0);
+        icy[q] = g.shy != R(0) ? g.at(a.in.icey, q, ny) : R(0);
+        idz[q] = g.has_idz(q) ? g.at(a.in.idz, q, ny) : R(0);
+        const int oi = w * RPT + q - TS;
+        own[q] = oj >= 0 && oj < OY && j0 + oj < ny && oi >= 0 && oi < OX && i0 + oi < nx;
+        any_own = any_own || own[q];
+    }
+    g.init(a);
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) ez[q] = g.me[q] * dz[q];
+    const bool probes = tm_probe_slots<RR, NT>(a.probes, nx, ny, i0 - TS, j0 - TS, s_slot, s_next, &s_any);
+    // (row, component) pairs of this wave that hold a probe of an owned cell
+    uint64_t pmask = 0;
+    if (probes) {
+#pragma unroll
+        for (int q = 0; q < RPT; ++q)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                if (!own[q]) s_slot[k][w * RPT + q][lane] = kTmNoProbe;   // this thread's entry only
+                if (__ballot(s_slot[k][w * RPT + q][lane] != kTmNoProbe)) pmask |= 1ull << (q * 3 + k);
+            }
+    }
+    const int src_i = a.src_i, src_j = a.src_j;
+    bool src_row = false;   // the source's row is one of this wave's
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) src_row = src_row || g.gi[q] == src_i;
+    // the launch's amplitudes, one per lane: a load inside the time loop would
+    // hold up every step of the source's tile
+    static_assert(TS <= 64, "one lane per step");
+    const R amps = src_row && lane < a.nsteps ? R(a.amp[a.t0 + lane]) : R(0);
+    sEz[w][lane] = ez[0];
+    if (w == 0) {
+        sEz[WV][lane] = R(0);
+        sHy[0][lane] = R(0);
+    }
+    const bool pml = __syncthreads_or(g.pml);
+
+    const R inv = a.inv_dL, cdt = a.cdt;
+    auto run = [&](auto with_pml) {
+        constexpr bool PML = decltype(with_pml)::value;
+        for (int s = 0; s < a.nsteps; ++s) {
+            const int t = a.t0 + s;
+            // ---- H update: CEx = (Ez[j+1] - Ez)/dL, CEy = -(Ez[i+1] - Ez)/dL
+            const R ez_next = sEz[w + 1][lane];
+#pragma unroll
+            for (int q = 0; q < RPT; ++q) {
+                const R dx = lane_above(ez[q]) - ez[q];
+                const R dy = ez[q] - (q + 1 < RPT ? ez[q + 1 < RPT ? q + 1 : q] : ez_next);
+                if constexpr (PML) {
+                    icx[q] += dx * inv;
+                    icy[q] += dy * inv;
+                    hx[q] = g.xa * hx[q] + g.xb * (dx + g.kx[q] * icx[q]);
+                    hy[q] = g.ya[q] * hy[q] + g.yb[q] * (dy + g.ky * icy[q]);
+                } else {
+                    hx[q] -= cdt * dx;
+                    hy[q] -= cdt * dy;
+                }
+            }
+            sHy[w + 1][lane] = hy[RPT - 1];
+            __syncthreads();
+            // ---- D update: CHz = (Hy - Hy[i-1])/dL - (Hx - Hx[j-1])/dL
+            const R hy_prev = sHy[w][lane];
+#pragma unroll
+            for (int q = 0; q < RPT; ++q) {
+                const R dh = (hy[q] - (q > 0 ? hy[q > 0 ? q - 1 : 0] : hy_prev)) - (hx[q] - lane_below(hx[q]));
+                if constexpr (PML) {
+                    idz[q] += dz[q];
+                    dz[q] = g.da[q] * dz[q] + g.db[q] * dh;
+                    dz[q] += g.dc[q] * idz[q];
+                } else {
+                    dz[q] += cdt * dh;
+                }
+            }
+            if (src_row) {
+                const R amp = read_lane(amps, s);
+#pragma unroll
+                for (int q = 0; q < RPT; ++q)
+                    if (g.gi[q] == src_i && g.gj == src_j) dz[q] += amp;
+            }
+#pragma unroll
+            for (int q = 0; q < RPT; ++q) ez[q] = g.me[q] * dz[q];
+            sEz[w][lane] = ez[0];
+            if (a.hist && any_own) {
+                R* hs = a.hist + (int64_t)s * n;
+#pragma unroll
+                for (int q = 0; q < RPT; ++q)
+                    if (own[q]) g.at(hs, q, ny) = dz[q];
+            }
+            if (pmask) {
+                R* row = a.rec + (int64_t)(t - a.rec_t0) * a.probes.n;
+#pragma unroll
+                for (int q = 0; q < RPT; ++q)
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        if (!(pmask >> (q * 3 + k) & 1)) continue;
+                        const R v = k == 0 ? ez[q] : k == 1 ? hx[q] : hy[q];
+                        for (int p = s_slot[k][w * RPT + q][lane]; p != kTmNoProbe; p = s_next[p]) row[p] = v;
+                    }
+            }
+            __syncthreads();
         }
+    };
+    if (pml) run(std::true_type{});
+    else run(std::false_type{});
+    // ---- store the owned tile
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) {
+        if (!own[q]) continue;
+        g.at(a.out.hx, q, ny) = hx[q];
+        g.at(a.out.hy, q, ny) = hy[q];
+        g.at(a.out.dz, q, ny) = dz[q];
+        if (g.shx[q] != R(0)) g.at(a.out.icex, q, ny) = icx[q];
+        if (g.shy != R(0)) g.at(a.out.icey, q, ny) = icy[q];
+        if (g.has_idz(q)) g.at(a.out.idz, q, ny) = idz[q];
     }
 }
 
-// The six arrays the TM kernel reads and writes (Hx, Hy, Dz, ICEx, ICEy, IDz).
-static const int kTmArrays[6] = {0, 1, 5, 6, 7, 17};
+// Reverse-time counterpart of k_tm_block: steps t0 + nsteps - 1 down to t0 of
+// the discrete adjoint (k_adj_a / k_adj_b restricted to Hx, Hy, Dz; the TE
+// components of a TM run are zero, so their cotangents reach neither eps nor
+// the amplitude).  Per step: the cotangents of that step's probes are added,
+// the amplitude's cotangent is read, then
+//   muCH = n2 lamD;  T = lamH + curlE(muCH);  lamICE += m3 T;  lamH = m1 T
+//   muCE = m2 T + lamICE;  q = curlH(muCE)   (muCH and muCE divided by dL)
+//   lamID += n4 lamD;  lamD = n1 lamD + lamID + mE q;  g_mE += D_{t-1} q.
+// D_{t-1} of the owned cells comes from the history that k_tm_block wrote.
+// 26 us per 16 steps at 400 x 400 float32; the whole gradient of a 2000-step
+// run takes 8.2 ms (126 ms with one-step launches of the general kernels and
+// a copy of D between them).
+template <typename R, int WV, int RPT, int TS>
+__global__ void __launch_bounds__(64 * WV) k_tm_adjoint(TmArgs<R> a) {
+    constexpr int RR = WV * RPT;
+    constexpr int NT = 64 * WV;
+    constexpr int OX = RR - 2 * TS, OY = 64 - 2 * TS;
+    __shared__ R sMz[WV + 1][64];   // muCHz of each wave's first row
+    __shared__ R sUy[WV + 1][64];   // muCEy of each wave's last row, at [wave + 1]
+    __shared__ unsigned short s_slot[3][RR][64];
+    __shared__ unsigned short s_next[kTmMaxProbes];
+    __shared__ int s_any;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int ti, tj;
+    tm_tile(a.tiles_y, ti, tj);
+    const int i0 = ti * OX, j0 = tj * OY;
+    const int nx = a.nx, ny = a.ny;
+    const int64_t n = (int64_t)nx * ny;
+    TmCells<R, RPT> g;
+    g.place(a, i0 - TS + w * RPT, j0 - TS + lane);
+    R hx[RPT], hy[RPT], dz[RPT], icx[RPT], icy[RPT], idz[RPT], gm[RPT], dn[RPT];
+    bool own[RPT], any_own = false;
+    const int oj = lane - TS;
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) {
+        hx[q] = g.at(a.in.hx, q, ny);
+        hy[q] = g.at(a.in.hy, q, ny);
+        dz[q] = g.at(a.in.dz, q, ny);
+        const int oi = w * RPT + q - TS;
+        own[q] = oj >= 0 && oj < OY && j0 + oj < ny && oi >= 0 && oi < OX && i0 + oi < nx;
+        any_own = any_own || own[q];
+        gm[q] = own[q] ? g.at(a.gm, q, ny) : R(0);
+        dn[q] = own[q] ? g.at(a.dz_hist + (int64_t)(a.nsteps - 1) * n, q, ny) : R(0);   // Dz after the last step
+    }
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) {
+        icx[q] = g.shx[q] != R(0) ? g.at(a.in.icex, q, ny) : R(0);
+        icy[q] = g.shy != R(0) ? g.at(a.in.icey, q, ny) : R(0);
+        idz[q] = g.has_idz(q) ? g.at(a.in.idz, q, ny) : R(0);
+    }
+    g.init(a);
+    // cotangents enter in the halo as well, so every cell of the region keeps its slot
+    const bool probes =
+        a.grec && tm_probe_slots<RR, NT>(a.probes, nx, ny, i0 - TS, j0 - TS, s_slot, s_next, &s_any);
+    uint64_t pmask = 0;
+    if (probes) {
+#pragma unroll
+        for (int q = 0; q < RPT; ++q)
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                if (__ballot(s_slot[k][w * RPT + q][lane] != kTmNoProbe)) pmask |= 1ull << (q * 3 + k);
+    }
+    const int src_i = a.gamp ? a.src_i : -1, src_j = a.src_j;
+    bool src_row = false;
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) src_row = src_row || g.gi[q] == src_i;
+    if (w == 0) {
+        sMz[WV][lane] = R(0);
+        sUy[0][lane] = R(0);
+    }
+    const bool pml = __syncthreads_or(g.pml);
+
+    const R inv = a.inv_dL, cdt = a.cdt;
+    auto run = [&](auto with_pml) {
+        constexpr bool PML = decltype(with_pml)::value;
+        // Ez-probe cotangent of each row's cell (its last probe), loaded a step ahead
+        R pre[RPT];
+        auto fetch = [&](int t) {
+            const R* row = a.grec + (int64_t)t * a.probes.n;
+#pragma unroll
+            for (int q = 0; q < RPT; ++q) {
+                if (!(pmask >> (3 * q) & 1)) continue;
+                const int p = s_slot[0][w * RPT + q][lane];
+                pre[q] = p != kTmNoProbe ? row[p] : R(0);
+            }
+        };
+        auto inject = [&](int t) {
+            const R* row = a.grec + (int64_t)t * a.probes.n;
+#pragma unroll
+            for (int q = 0; q < RPT; ++q) {
+                if (pmask >> (3 * q) & 1) {
+                    const int head = s_slot[0][w * RPT + q][lane];
+                    R v = pre[q];
+                    if (head != kTmNoProbe)
+                        for (int p = s_next[head]; p != kTmNoProbe; p = s_next[p]) v += row[p];
+                    dz[q] += g.me[q] * v;
+                    gm[q] += dn[q] * v;
+                }
+                if (pmask >> (3 * q + 1) & 1)
+                    for (int p = s_slot[1][w * RPT + q][lane]; p != kTmNoProbe; p = s_next[p]) hx[q] += row[p];
+                if (pmask >> (3 * q + 2) & 1)
+                    for (int p = s_slot[2][w * RPT + q][lane]; p != kTmNoProbe; p = s_next[p]) hy[q] += row[p];
+            }
+        };
+        R dp[RPT];   // Dz before the step, loaded while the step before it runs
+        auto load_dp = [&](int s) {
+            if (!any_own) return;
+            const R* hs = s > 0 ? a.dz_hist + (int64_t)(s - 1) * n : a.dz_before;
+#pragma unroll
+            for (int q = 0; q < RPT; ++q) dp[q] = own[q] ? g.at(hs, q, ny) : R(0);
+        };
+        if (pmask) fetch(a.t0 + a.nsteps - 1);
+        load_dp(a.nsteps - 1);
+        for (int s = a.nsteps - 1; s >= 0; --s) {
+            const int t = a.t0 + s;
+            if (pmask) {
+                inject(t);
+                if (s > 0) fetch(t - 1);
+            }
+            if (src_row) {
+#pragma unroll
+                for (int q = 0; q < RPT; ++q)
+                    if (own[q] && g.gi[q] == src_i && g.gj == src_j) a.gamp[t] = dz[q];
+            }
+            R mz[RPT];
+#pragma unroll
+            for (int q = 0; q < RPT; ++q) mz[q] = (PML ? g.db[q] : cdt) * dz[q];
+            sMz[w][lane] = mz[0];
+            __syncthreads();
+            const R mz_next = sMz[w + 1][lane];
+            R ux[RPT], uy[RPT];
+#pragma unroll
+            for (int q = 0; q < RPT; ++q) {
+                const R tx = hx[q] + (lane_above(mz[q]) - mz[q]);
+                const R ty = hy[q] + (mz[q] - (q + 1 < RPT ? mz[q + 1 < RPT ? q + 1 : q] : mz_next));
+                if constexpr (PML) {
+                    const R bx = g.xb * tx, by = g.yb[q] * ty;
+                    icx[q] += g.kx[q] * bx;
+                    icy[q] += g.ky * by;
+                    ux[q] = bx + icx[q] * inv;
+                    uy[q] = by + icy[q] * inv;
+                    hx[q] = g.xa * tx;
+                    hy[q] = g.ya[q] * ty;
+                } else {
+                    ux[q] = -cdt * tx;
+                    uy[q] = -cdt * ty;
+                    hx[q] = tx;
+                    hy[q] = ty;
+                }
+            }
+            sUy[w + 1][lane] = uy[RPT - 1];
+            __syncthreads();
+            const R uy_prev = sUy[w][lane];
+#pragma unroll
+            for (int q = 0; q < RPT; ++q) {
+                const R c = (uy[q] - (q > 0 ? uy[q > 0 ? q - 1 : 0] : uy_prev)) - (ux[q] - lane_below(ux[q]));
+                if constexpr (PML) {
+                    idz[q] += g.dc[q] * dz[q];
+                    dz[q] = g.da[q] * dz[q] + idz[q] + g.me[q] * c;
+                } else {
+                    dz[q] += g.me[q] * c;
+                }
+                if (any_own) {
+                    gm[q] += dp[q] * c;
+                    dn[q] = dp[q];
+                }
+            }
+            if (s > 0) load_dp(s - 1);
+        }
+    };
+    if (pml) run(std::true_type{});
+    else run(std::false_type{});
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) {
+        if (!own[q]) continue;
+        g.at(a.out.hx, q, ny) = hx[q];
+        g.at(a.out.hy, q, ny) = hy[q];
+        g.at(a.out.dz, q, ny) = dz[q];
+        if (g.shx[q] != R(0)) g.at(a.out.icex, q, ny) = icx[q];
+        if (g.shy != R(0)) g.at(a.out.icey, q, ny) = icy[q];
+        if (g.has_idz(q)) g.at(a.out.idz, q, ny) = idz[q];
+        g.at(a.gm, q, ny) = gm[q];
+    }
+}
+
+// TM arrays of an 18-array state, and of a packed buffer of the six arrays.
+template <typename R>
+static TmState<R> tm_of_state(R* st, int64_t n) {
+    return TmState<R>{st, st + n, st + 5 * n, st + 6 * n, st + 7 * n, st + 17 * n};
+}
+template <typename R>
+static TmState<R> tm_of_packed(R* p, int64_t n) {
+    return TmState<R>{p, p + n, p + 2 * n, p + 3 * n, p + 4 * n, p + 5 * n};
+}
+
+// out = in for the values a TM run reads or writes: the fields everywhere, an
+// integral where its sigma is non-zero (the rest of `out` keeps its values).
+template <typename R>
+__global__ void __launch_bounds__(256) k_tm_copy(TmArgs<R> a) {
+    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= (int64_t)a.nx * a.ny) return;
+    const int i = (int)(c / a.ny), j = (int)(c - (int64_t)i * a.ny);
+    a.out.hx[c] = a.in.hx[c];
+    a.out.hy[c] = a.in.hy[c];
+    a.out.dz[c] = a.in.dz[c];
+    if (a.sig[i] != R(0)) a.out.icex[c] = a.in.icex[c];
+    if (a.sig[a.nx + j] != R(0)) a.out.icey[c] = a.in.icey[c];
+    if (a.sig[a.nx + a.ny + 1 + i] != R(0) && a.sig[2 * a.nx + a.ny + 1 + j] != R(0)) a.out.idz[c] = a.in.idz[c];
+}
 
 template <typename R>
-static int copy_tm_arrays(R* dst, const R* src, int64_t n, hipStream_t s) {
-    for (int k = 0; k < 6; ++k)
-        CV_HIP(hipMemcpyAsync(dst + kTmArrays[k] * n, src + kTmArrays[k] * n, sizeof(R) * n,
-                              hipMemcpyDeviceToDevice, s));
-    return CV_OK;
-}
-
-template <typename R, int WV, int RPT, int TS>
-static int launch_tm(const Fdtd<R>& f, R* alt, const double* amp_dev, int64_t src, int t0, int n_steps,
-                     const int32_t* pcomp, const int64_t* pcell, int np, R* rec, int rec_t0, hipStream_t s) {
-    static_assert(WV * RPT > 2 * TS && 64 > 2 * TS, "the owned tile must not be empty");
-    TmArgs<R> a;
+static TmArgs<R> tm_args(const Fdtd<R>& f) {
+    TmArgs<R> a = {};
     a.nx = f.nx;
     a.ny = f.ny;
-    constexpr int OX = WV * RPT - 2 * TS, OY = 64 - 2 * TS;
-    a.tiles_x = (f.nx + OX - 1) / OX;
-    a.tiles_y = (f.ny + OY - 1) / OY;
-    a.src = src;
-    a.np = np;
-    a.inv_dL = f.inv_dL;
-    a.h1 = f.h1;
-    a.h2 = f.h2;
-    a.d1 = f.d1;
-    a.d2 = f.d2;
-    a.dt = f.dt;
-    a.c0 = f.c0;
-    a.eps0 = f.eps0;
+    a.src_i = -1;
+    a.inv_dL = R(1.0 / f.dL);
+    a.dL = R(f.dL);
+    a.cdt = R(f.c0 * f.dt / f.dL);
+    a.half_dt = R(f.dt / (2.0 * f.eps0));
     a.sig = f.sig;
     a.eps = f.eps;
-    a.st_in = f.st;
-    a.st_out = alt;
-    a.amp = amp_dev;
-    a.pcomp = pcomp;
-    a.pcell = pcell;
-    a.rec = rec;
-    a.rec_t0 = rec_t0;
-    const int nblocks = a.tiles_x * a.tiles_y;
-    if (n_steps <= 0) return CV_OK;
-    // alt starts equal to the state, so cells a launch does not write (PML
-    // integrals where sigma is 0) agree in both buffers
-    int rc = copy_tm_arrays<R>(alt, f.st, f.n, s);
-    if (rc != CV_OK) return rc;
-    R* cur = f.st;
-    R* nxt = alt;
-    for (int t = 0; t < n_steps; t += TS) {
-        a.t0 = t0 + t;
-        a.nsteps = (n_steps - t < TS) ? (n_steps - t) : TS;
-        a.st_in = cur;
-        a.st_out = nxt;
-        k_tm_block<R, WV, RPT, TS><<<nblocks, 64 * WV, 0, s>>>(a);
-        R* tmp = cur;
-        cur = nxt;
-        nxt = tmp;
-    }
-    if (cur != f.st) return copy_tm_arrays<R>(f.st, cur, f.n, s);
-    return CV_OK;
+    return a;
 }
 
 template <typename R>
-static int dispatch_tm(int cfg, const Fdtd<R>& f, R* alt, const double* amp_dev, int64_t src, int t0, int n_steps,
-                       const int32_t* pcomp, const int64_t* pcell, int np, R* rec, int rec_t0, hipStream_t s) {
-    switch (cfg) {
-        case 0: return launch_tm<R, 4, 4, 2>(f, alt, amp_dev, src, t0, n_steps, pcomp, pcell, np, rec, rec_t0, s);
-        case 1: return launch_tm<R, 4, 4, 4>(f, alt, amp_dev, src, t0, n_steps, pcomp, pcell, np, rec, rec_t0, s);
-        case 2: return launch_tm<R, 4, 8, 4>(f, alt, amp_dev, src, t0, n_steps, pcomp, pcell, np, rec, rec_t0, s);
-        case 3: return launch_tm<R, 4, 8, 8>(f, alt, amp_dev, src, t0, n_steps, pcomp, pcell, np, rec, rec_t0, s);
-        case 4: return launch_tm<R, 4, 16, 8>(f, alt, amp_dev, src, t0, n_steps, pcomp, pcell, np, rec, rec_t0, s);
-        case 5: return launch_tm<R, 4, 16, 4>(f, alt, amp_dev, src, t0, n_steps, pcomp, pcell, np, rec, rec_t0, s);
-        case 6: return launch_tm<R, 8, 4, 8>(f, alt, amp_dev, src, t0, n_steps, pcomp, pcell, np, rec, rec_t0, s);
-        case 7: return launch_tm<R, 16, 4, 16>(f, alt, amp_dev, src, t0, n_steps, pcomp, pcell, np, rec, rec_t0, s);
-        case 8: return launch_tm<R, 16, 2, 8>(f, alt, amp_dev, src, t0, n_steps, pcomp, pcell, np, rec, rec_t0, s);
-        case 9: return launch_tm<R, 16, 4, 8>(f, alt, amp_dev, src, t0, n_steps, pcomp, pcell, np, rec, rec_t0, s);
-        case 10: return launch_tm<R, 8, 4, 4>(f, alt, amp_dev, src, t0, n_steps, pcomp, pcell, np, rec, rec_t0, s);
-        case 11: return launch_tm<R, 16, 2, 4>(f, alt, amp_dev, src, t0, n_steps, pcomp, pcell, np, rec, rec_t0, s);
-        default: break;
+static void tm_source(TmArgs<R>& a, int64_t cell) {
+    a.src_i = cell >= 0 ? (int)(cell / a.ny) : -1;
+    a.src_j = cell >= 0 ? (int)(cell % a.ny) : -1;
+}
+
+template <typename R>
+static void tm_copy(TmArgs<R> a, TmState<R> in, TmState<R> out, hipStream_t s) {
+    a.in = in;
+    a.out = out;
+    k_tm_copy<R><<<(unsigned)(((int64_t)a.nx * a.ny + 255) / 256), 256, 0, s>>>(a);
+}
+
+// One launch sequence of a TM run over steps [a.t0, a.t0 + n_steps) from `in`:
+// the launches alternate between the buffers w0 and w1 (`in` may be one of
+// them) and the last one writes `out`, which must not be the buffer it reads
+// (null: the next of w0 and w1).  reverse: the adjoint steps, last step first, `in` the
+// cotangent after the steps; a.dz_hist and a.hist start at step a.t0.
+template <typename R, int WV, int RPT, int TS>
+static void launch_tm(TmArgs<R> a, TmState<R> in, TmState<R> out, TmState<R> w0, TmState<R> w1, int n_steps,
+                      bool reverse, hipStream_t s) {
+    static_assert(WV * RPT > 2 * TS && 64 > 2 * TS, "the owned tile must not be empty");
+    constexpr int OX = WV * RPT - 2 * TS, OY = 64 - 2 * TS;
+    a.tiles_x = (a.nx + OX - 1) / OX;
+    a.tiles_y = (a.ny + OY - 1) / OY;
+    const int64_t n = (int64_t)a.nx * a.ny;
+    const int nblocks = a.tiles_x * a.tiles_y;
+    const int t0 = a.t0;
+    R* hist = a.hist;
+    const R* dz_hist = a.dz_hist;
+    const R* dz_before = a.dz_before;
+    TmState<R> cur = in;
+    for (int done = 0; done < n_steps; done += TS) {
+        a.nsteps = std::min(TS, n_steps - done);
+        const int first = reverse ? n_steps - done - a.nsteps : done;
+        a.t0 = t0 + first;
+        a.hist = hist ? hist + (int64_t)first * n : nullptr;
+        a.dz_hist = dz_hist ? dz_hist + (int64_t)first * n : nullptr;
+        a.dz_before = first > 0 && dz_hist ? dz_hist + (int64_t)(first - 1) * n : dz_before;
+        a.in = cur;
+        a.out = done + TS >= n_steps && out.hx ? out : (cur.hx == w0.hx ? w1 : w0);
+        if (reverse) k_tm_adjoint<R, WV, RPT, TS><<<nblocks, 64 * WV, 0, s>>>(a);
+        else k_tm_block<R, WV, RPT, TS><<<nblocks, 64 * WV, 0, s>>>(a);
+        cur = a.out;
     }
-    CV_CHECK(false, "unknown TM tile configuration %d", cfg);
+}
+
+template <typename R>
+static int dispatch_tm(int cfg, const TmArgs<R>& a, TmState<R> in, TmState<R> out, TmState<R> w0, TmState<R> w1,
+                       int n_steps, bool reverse, hipStream_t s) {
+    switch (cfg) {
+        case 0: launch_tm<R, 4, 4, 2>(a, in, out, w0, w1, n_steps, reverse, s); break;
+        case 1: launch_tm<R, 4, 4, 4>(a, in, out, w0, w1, n_steps, reverse, s); break;
+        case 2: launch_tm<R, 4, 8, 4>(a, in, out, w0, w1, n_steps, reverse, s); break;
+        case 3: launch_tm<R, 4, 8, 8>(a, in, out, w0, w1, n_steps, reverse, s); break;
+        case 4: launch_tm<R, 4, 16, 8>(a, in, out, w0, w1, n_steps, reverse, s); break;
+        case 5: launch_tm<R, 4, 16, 4>(a, in, out, w0, w1, n_steps, reverse, s); break;
+        case 6: launch_tm<R, 8, 4, 8>(a, in, out, w0, w1, n_steps, reverse, s); break;
+        case 7: launch_tm<R, 16, 4, 16>(a, in, out, w0, w1, n_steps, reverse, s); break;
+        case 8: launch_tm<R, 16, 2, 8>(a, in, out, w0, w1, n_steps, reverse, s); break;
+        case 9: launch_tm<R, 16, 4, 8>(a, in, out, w0, w1, n_steps, reverse, s); break;
+        case 10: launch_tm<R, 8, 4, 4>(a, in, out, w0, w1, n_steps, reverse, s); break;
+        case 11: launch_tm<R, 16, 2, 4>(a, in, out, w0, w1, n_steps, reverse, s); break;
+        default: CV_CHECK(false, "unknown TM tile configuration %d", cfg);
+    }
+    return CV_OK;
 }
 
 // ================================================ fused single-pass 3D step
@@ -1715,6 +2126,7 @@ static int make_fdtd(const cv_fdtd_desc* d, const void* sig, const void* eps, vo
     f.dt = d->dt;
     f.c0 = d->c0;
     f.eps0 = d->eps0;
+    f.dL = d->dL;
     f.sig = (const R*)sig;
     f.eps = (const R*)eps;
     f.st = (R*)state;
@@ -1975,16 +2387,141 @@ extern "C" int cv_fdtd_efields_grad(int dtype, const cv_fdtd_desc* d, const void
 }
 
 extern "C" int cv_fdtd_tm_configs(int* rpt, int* ts, int* waves, int max_n) {
-    static const int R_[12] = {4, 4, 8, 8, 16, 16, 4, 4, 2, 4, 4, 2};
-    static const int T_[12] = {2, 4, 4, 8, 8, 4, 8, 16, 8, 8, 4, 4};
-    static const int W_[12] = {4, 4, 4, 4, 4, 4, 8, 16, 16, 16, 8, 16};
-    for (int i = 0; i < 12 && i < max_n; ++i) {
+    static const int R_[kTmConfigs] = {4, 4, 8, 8, 16, 16, 4, 4, 2, 4, 4, 2};
+    static const int T_[kTmConfigs] = {2, 4, 4, 8, 8, 4, 8, 16, 8, 8, 4, 4};
+    static const int W_[kTmConfigs] = {4, 4, 4, 4, 4, 4, 8, 16, 16, 16, 8, 16};
+    for (int i = 0; i < kTmConfigs && i < max_n; ++i) {
         if (rpt) rpt[i] = R_[i];
         if (ts) ts[i] = T_[i];
         if (waves) waves[i] = W_[i];
     }
-    return 12;
+    return kTmConfigs;
 }
+
+namespace cv {
+
+template <typename R>
+static int run_tm_impl(const cv_fdtd_desc* d, const void* sig, const void* eps, void* state, void* state_alt,
+                       int64_t src_cell, const double* amp_dev, int t0, int n_steps, TmProbes probes, void* rec,
+                       int rec_t0, int config, hipStream_t s) {
+    Fdtd<R> f;
+    int rc = make_fdtd<R>(d, sig, eps, state, f);
+    if (rc) return rc;
+    CV_CHECK(src_cell < f.n, "source cell out of range");
+    if (n_steps <= 0) return CV_OK;
+    TmArgs<R> a = tm_args(f);
+    tm_source(a, src_cell);
+    a.amp = amp_dev;
+    a.probes = probes;
+    a.rec = (R*)rec;
+    a.rec_t0 = rec_t0;
+    a.t0 = t0;
+    const TmState<R> A = tm_of_state(f.st, f.n), B = tm_of_state((R*)state_alt, f.n);
+    int ts[kTmConfigs];
+    cv_fdtd_tm_configs(nullptr, ts, nullptr, kTmConfigs);
+    // the last launch may not write the buffer it reads: an odd number of
+    // launches ends in the other one and is copied back
+    const bool odd = ((n_steps + ts[config] - 1) / ts[config]) % 2 != 0;
+    rc = dispatch_tm<R>(config, a, A, odd ? B : A, A, B, n_steps, false, s);
+    if (rc) return rc;
+    if (odd) tm_copy(a, B, A, s);
+    return CV_OK;
+}
+
+template <typename R>
+static int run_tm_checkpoints_impl(const cv_fdtd_desc* d, const void* sig, const void* eps, void* state, void* work,
+                                   void* checkpoints, int checkpoint_every, int64_t src_cell, const double* amp_dev,
+                                   int n_steps, TmProbes probes, void* rec, int config, hipStream_t s) {
+    Fdtd<R> f;
+    int rc = make_fdtd<R>(d, sig, eps, state, f);
+    if (rc) return rc;
+    CV_CHECK(src_cell < f.n, "source cell out of range");
+    if (n_steps <= 0) return CV_OK;
+    TmArgs<R> a = tm_args(f);
+    tm_source(a, src_cell);
+    a.amp = amp_dev;
+    a.probes = probes;
+    a.rec = (R*)rec;
+    const TmState<R> A = tm_of_state(f.st, f.n);
+    const TmState<R> w0 = tm_of_packed((R*)work, f.n), w1 = tm_of_packed((R*)work + 6 * f.n, f.n);
+    auto ck = [&](int k) { return tm_of_packed((R*)checkpoints + (int64_t)k * 6 * f.n, f.n); };
+    // a segment's last launch writes the next checkpoint, the run's last one the state
+    tm_copy(a, A, ck(0), s);
+    for (int k = 0, t = 0; t < n_steps; ++k, t += checkpoint_every) {
+        const int m = std::min(checkpoint_every, n_steps - t);
+        a.t0 = t;
+        rc = dispatch_tm<R>(config, a, ck(k), t + m < n_steps ? ck(k + 1) : A, w0, w1, m, false, s);
+        if (rc) return rc;
+    }
+    return CV_OK;
+}
+
+template <typename R>
+static int tm_adjoint_impl(const cv_fdtd_desc* d, const void* sig, const void* eps, const void* checkpoints,
+                           int checkpoint_every, int64_t src_cell, const double* amp_dev, int n_steps, void* work,
+                           void* dz_hist, void* lam, void* g_mEz, TmProbes probes, const void* g_rec, void* g_amp,
+                           int config, hipStream_t s) {
+    Fdtd<R> f;
+    int rc = make_fdtd<R>(d, sig, eps, lam, f);
+    if (rc) return rc;
+    CV_CHECK(src_cell < f.n, "source cell out of range");
+    const int64_t n = f.n;
+    const TmState<R> w0 = tm_of_packed((R*)work, n), w1 = tm_of_packed((R*)work + 6 * n, n);
+    const TmState<R> l0 = tm_of_packed((R*)lam, n), l1 = tm_of_packed((R*)lam + 6 * n, n);
+    R* hist = (R*)dz_hist;
+    const int nseg = n_steps > 0 ? (n_steps + checkpoint_every - 1) / checkpoint_every : 0;
+    TmState<R> cur = l0;
+    // The adjoint holds about 1.4 times the forward kernel's registers.  In
+    // float64, 16 waves of more than two rows a thread do not fit 128 of them
+    // (20 us a step with three rows, spilling, against 9.8 us with two, at
+    // 1211 x 901), so those shapes take the two-row one.
+    const int adj = sizeof(R) == 8 && (config == 7 || config == 9) ? 8 : config;
+    for (int k = nseg - 1; k >= 0; --k) {
+        const int t = k * checkpoint_every, m = std::min(checkpoint_every, n_steps - t);
+        const TmState<R> start = tm_of_packed((R*)checkpoints + (int64_t)k * 6 * n, n);
+        // the segment again, with Dz after each of its steps
+        TmArgs<R> a = tm_args(f);
+        a.t0 = t;
+        tm_source(a, src_cell);
+        a.amp = amp_dev;
+        a.hist = hist;
+        rc = dispatch_tm<R>(config, a, start, TmState<R>{}, w0, w1, m, false, s);
+        if (rc) return rc;
+        TmArgs<R> b = tm_args(f);
+        b.t0 = t;
+        tm_source(b, src_cell);
+        b.probes = probes;
+        b.grec = (const R*)g_rec;
+        b.gamp = (R*)g_amp;
+        b.gm = (R*)g_mEz;
+        b.dz_hist = hist;
+        b.dz_before = start.dz;
+        const TmState<R> other = cur.hx == l0.hx ? l1 : l0;
+        int ts[kTmConfigs];
+        cv_fdtd_tm_configs(nullptr, ts, nullptr, kTmConfigs);
+        const bool odd = ((m + ts[adj] - 1) / ts[adj]) % 2 != 0;
+        const TmState<R> end = odd ? other : cur;
+        rc = dispatch_tm<R>(adj, b, cur, end, l0, l1, m, true, s);
+        if (rc) return rc;
+        cur = end;
+    }
+    if (cur.hx != l0.hx) tm_copy(tm_args(f), cur, l0, s);
+    return CV_OK;
+}
+
+static int tm_checks(const cv_fdtd_desc* d, int n_steps, const int32_t* probe_comp, const int64_t* probe_cell,
+                     int n_probes, int64_t src_cell, const double* amp_dev, int config) {
+    CV_CHECK(d && d->nz == 1, "the TM kernel needs nz == 1");
+    CV_CHECK(n_probes >= 0 && n_probes <= kTmMaxProbes, "the TM kernel records at most %d probes", kTmMaxProbes);
+    CV_CHECK(n_steps >= 0, "bad step range");
+    CV_CHECK(n_probes == 0 || (probe_comp && probe_cell), "probes need comp and cell buffers");
+    CV_CHECK(src_cell < 0 || amp_dev, "a source needs its amplitude array");
+    CV_CHECK(config >= 0 && config < kTmConfigs,
+             "unknown TM tile configuration %d", config);
+    return CV_OK;
+}
+
+}  // namespace cv
 
 extern "C" int cv_fdtd_run_tm(int dtype, const cv_fdtd_desc* d, const void* sig, const void* eps, void* state,
                               void* state_alt, int64_t src_cell, const double* amp_dev, int t0, int n_steps,
@@ -1992,30 +2529,69 @@ extern "C" int cv_fdtd_run_tm(int dtype, const cv_fdtd_desc* d, const void* sig,
                               int rec_t0, int config, void* stream) {
     hipStream_t s = as_stream(stream);
     CV_CHECK(state && state_alt && state != state_alt, "two distinct state buffers are needed");
-    CV_CHECK(d && d->nz == 1, "the TM kernel needs nz == 1");
-    CV_CHECK(n_probes <= kTmMaxProbes, "the TM kernel records at most %d probes", kTmMaxProbes);
-    CV_CHECK(n_steps >= 0 && t0 >= 0, "bad step range");
-    CV_CHECK(n_probes == 0 || (probe_comp && probe_cell && rec), "probes need comp, cell and rec buffers");
-    CV_CHECK(src_cell < 0 || amp_dev, "a source needs its amplitude array");
-    if (dtype == CV_F32) {
-        Fdtd<float> f;
-        int rc = make_fdtd<float>(d, sig, eps, state, f);
-        if (rc) return rc;
-        CV_CHECK(src_cell < f.n, "source cell out of range");
-        rc = dispatch_tm<float>(config, f, (float*)state_alt, amp_dev, src_cell, t0, n_steps, probe_comp, probe_cell,
-                                n_probes, (float*)rec, rec_t0, s);
-        if (rc) return rc;
-    } else if (dtype == CV_F64) {
-        Fdtd<double> f;
-        int rc = make_fdtd<double>(d, sig, eps, state, f);
-        if (rc) return rc;
-        CV_CHECK(src_cell < f.n, "source cell out of range");
-        rc = dispatch_tm<double>(config, f, (double*)state_alt, amp_dev, src_cell, t0, n_steps, probe_comp,
-                                 probe_cell, n_probes, (double*)rec, rec_t0, s);
-        if (rc) return rc;
-    } else {
+    CV_CHECK(t0 >= 0, "bad step range");
+    CV_CHECK(n_probes == 0 || rec, "probes need a record buffer");
+    int rc = tm_checks(d, n_steps, probe_comp, probe_cell, n_probes, src_cell, amp_dev, config);
+    if (rc) return rc;
+    const TmProbes pr{probe_comp, probe_cell, n_probes};
+    if (dtype == CV_F32)
+        rc = run_tm_impl<float>(d, sig, eps, state, state_alt, src_cell, amp_dev, t0, n_steps, pr, rec, rec_t0, config,
+                                s);
+    else if (dtype == CV_F64)
+        rc = run_tm_impl<double>(d, sig, eps, state, state_alt, src_cell, amp_dev, t0, n_steps, pr, rec, rec_t0, config,
+                                 s);
+    else
         CV_CHECK(false, "unknown dtype %d", dtype);
-    }
+    if (rc) return rc;
+    CV_LAUNCH_CHECK();
+    return CV_OK;
+}
+
+extern "C" int cv_fdtd_run_tm_checkpoints(int dtype, const cv_fdtd_desc* d, const void* sig, const void* eps,
+                                          void* state, void* work, void* checkpoints, int checkpoint_every,
+                                          int64_t src_cell, const double* amp_dev, int n_steps,
+                                          const int32_t* probe_comp, const int64_t* probe_cell, int n_probes, void* rec,
+                                          int config, void* stream) {
+    hipStream_t s = as_stream(stream);
+    CV_CHECK(state && work && checkpoints, "null pointer argument");
+    CV_CHECK(checkpoint_every > 0, "checkpoint_every must be positive");
+    CV_CHECK(n_probes == 0 || rec, "probes need a record buffer");
+    int rc = tm_checks(d, n_steps, probe_comp, probe_cell, n_probes, src_cell, amp_dev, config);
+    if (rc) return rc;
+    const TmProbes pr{probe_comp, probe_cell, n_probes};
+    if (dtype == CV_F32)
+        rc = run_tm_checkpoints_impl<float>(d, sig, eps, state, work, checkpoints, checkpoint_every, src_cell, amp_dev,
+                                            n_steps, pr, rec, config, s);
+    else if (dtype == CV_F64)
+        rc = run_tm_checkpoints_impl<double>(d, sig, eps, state, work, checkpoints, checkpoint_every, src_cell, amp_dev,
+                                             n_steps, pr, rec, config, s);
+    else
+        CV_CHECK(false, "unknown dtype %d", dtype);
+    if (rc) return rc;
+    CV_LAUNCH_CHECK();
+    return CV_OK;
+}
+
+extern "C" int cv_fdtd_tm_adjoint(int dtype, const cv_fdtd_desc* d, const void* sig, const void* eps,
+                                  const void* checkpoints, int checkpoint_every, int64_t src_cell,
+                                  const double* amp_dev, int n_steps, void* work, void* dz_hist, void* lam,
+                                  void* g_mEz, const int32_t* probe_comp, const int64_t* probe_cell, int n_probes,
+                                  const void* g_rec, void* g_amp, int config, void* stream) {
+    hipStream_t s = as_stream(stream);
+    CV_CHECK(checkpoints && work && dz_hist && lam && g_mEz, "null pointer argument");
+    CV_CHECK(checkpoint_every > 0, "checkpoint_every must be positive");
+    int rc = tm_checks(d, n_steps, probe_comp, probe_cell, n_probes, src_cell, amp_dev, config);
+    if (rc) return rc;
+    const TmProbes pr{probe_comp, probe_cell, n_probes};
+    if (dtype == CV_F32)
+        rc = tm_adjoint_impl<float>(d, sig, eps, checkpoints, checkpoint_every, src_cell, amp_dev, n_steps, work,
+                                    dz_hist, lam, g_mEz, pr, g_rec, g_amp, config, s);
+    else if (dtype == CV_F64)
+        rc = tm_adjoint_impl<double>(d, sig, eps, checkpoints, checkpoint_every, src_cell, amp_dev, n_steps, work,
+                                     dz_hist, lam, g_mEz, pr, g_rec, g_amp, config, s);
+    else
+        CV_CHECK(false, "unknown dtype %d", dtype);
+    if (rc) return rc;
     CV_LAUNCH_CHECK();
     return CV_OK;
 }

@@ -390,6 +390,32 @@ int cv_fdtd_run_fused(int dtype, const cv_fdtd_desc* d, const void* sig, const v
  * counterpart in the reference (a tuning knob of this kernel). */
 int cv_fdtd_slab_tuning(int band_rows, int chunk, int target_workgroups, int map_bands);
 
+/* cv_fdtd_run_tm from step 0 with what its adjoint needs: `checkpoints`
+ * receives the TM state (Hx, Hy, Dz, ICEx, ICEy, IDz: 6 arrays of n) before
+ * the steps 0, checkpoint_every, 2 checkpoint_every, ..., `state` the state
+ * after the run; `work` holds 12 n values.  Integrals are stored where their
+ * sigma is non-zero (nothing reads the others). */
+int cv_fdtd_run_tm_checkpoints(int dtype, const cv_fdtd_desc* d, const void* sig, const void* eps, void* state,
+                               void* work, void* checkpoints, int checkpoint_every, int64_t src_cell,
+                               const double* amp_dev, int n_steps, const int32_t* probe_comp,
+                               const int64_t* probe_cell, int n_probes, void* rec, int config, void* stream);
+
+/* Adjoint of cv_fdtd_run_tm_checkpoints over the whole run, temporally blocked
+ * like the run itself: per segment, last first, the steps run again from their
+ * checkpoint with Dz of every step kept in dz_hist (checkpoint_every n
+ * values), then the adjoint steps.  lam (2 buffers of the 6 TM arrays): on
+ * entry the first holds the cotangent of the final state, on return that of
+ * the initial one (integrals where their sigma is non-zero; the second buffer
+ * is scratch).  g_mEz (n) += cotangent of 1 / eps_zz.  g_rec: cotangent of the
+ * records (n_steps, n_probes) or NULL; g_amp: cotangent of the amplitudes
+ * (n_steps, written) or NULL; `work` holds 12 n values.  The same sums as
+ * cv_fdtd_adjoint_step restricted to the TM components (autograd's tape over
+ * fdtd.py:74-144). */
+int cv_fdtd_tm_adjoint(int dtype, const cv_fdtd_desc* d, const void* sig, const void* eps, const void* checkpoints,
+                       int checkpoint_every, int64_t src_cell, const double* amp_dev, int n_steps, void* work,
+                       void* dz_hist, void* lam, void* g_mEz, const int32_t* probe_comp, const int64_t* probe_cell,
+                       int n_probes, const void* g_rec, void* g_amp, int config, void* stream);
+
 /* Tile configurations of cv_fdtd_run_tm: fills rpt[i], ts[i], waves[i]
  * (rows per thread, steps per launch, waves per workgroup; the region is
  * waves*rpt rows by 64 columns) for i < max_n and returns their number. */

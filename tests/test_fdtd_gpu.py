@@ -470,3 +470,40 @@ def test_forward_mode_per_step_api_matches_complex_step():
 
     h = 1e-30
     assert dS == pytest.approx(np.imag(obj_cs(eps0 + 1j * h * d)) / h, rel=1e-8)
+
+
+@pytest.mark.parametrize('cfg', range(12))
+@pytest.mark.parametrize('shape,steps,ck', [((9, 70), 21, 7), ((65, 61), 37, 16), ((130, 129), 33, 50)])
+def test_tm_adjoint_configs_match_generic(cfg, shape, steps, ck):
+    """The temporally blocked adjoint against the per-step kernels on grids
+    smaller than a tile, with remainders and several tiles, with and without
+    PML, for probes of every component, two of them equal, at corners and at
+    the source, gradients to eps, the amplitudes and through the final state.
+    Both form the same sums of O(steps) terms: steps * 2^-52 relative."""
+    import ceviche_amd as cv
+    print('tm adjoint cfg', cfg, shape, steps, ck, flush=True)
+    nx, ny = shape
+    rng = np.random.default_rng(cfg)
+    eps0 = rng.uniform(1, 12, (nx, ny, 1))
+    amp0 = rng.standard_normal(steps)
+    src = (nx // 2, ny // 2, 0)
+    probes = [('Ez', src), ('Hx', (0, 0, 0)), ('Ez', (nx - 1, ny - 1, 0)), ('Hy', (nx // 2 + 1, ny // 2, 0)),
+              ('Ez', (nx // 2 + 2, ny // 2 + 2, 0)), ('Ez', (nx // 2 + 2, ny // 2 + 2, 0)), ('Hx', src)]
+    wt = torch.from_numpy(rng.standard_normal((steps, len(probes)))).cuda()
+    npml = [min(3 + cfg % 3, nx // 3), 5, 0] if cfg % 4 else [0, 0, 0]
+    got = {}
+    for kernel in (cfg, 'generic'):
+        for final in (False, True):
+            eps = torch.tensor(eps0, requires_grad=True)
+            amp = torch.tensor(amp0, requires_grad=True)
+            F = cv.fdtd(eps, 20e-9, npml)
+            rec = F.run(steps, src, amp, probes, checkpoint_every=ck, kernel=kernel)
+            loss = (rec * wt).sum() + (rec ** 2).sum()
+            if final:
+                f = F.fields
+                loss = loss + (f['Ez'] ** 2).sum() + (f['Hx'] * f['Hy']).sum()
+            loss.backward()
+            got[kernel, final] = rec.detach(), eps.grad, amp.grad
+    for final in (False, True):
+        for x, y in zip(got[cfg, final], got['generic', final]):
+            assert float((x - y).norm()) <= 40 * steps * 2.2e-16 * float(y.norm()), (final, x.shape)
