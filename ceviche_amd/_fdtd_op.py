@@ -207,6 +207,23 @@ class FdtdGrid:
                                          ptr(D_prev), ptr(gmE), ptr(pc), ptr(pl), npb, ptr(g_probe), ptr(D_t),
                                          comp, cell, ptr(g_src), stream_ptr()), 'fdtd adjoint')
 
+    def step_history(self, state, hist, eps, src, amp_dev, n_steps):
+        """Advance ``state`` (all but its D) n_steps with D of every step kept:
+        hist[s] = D before step s, hist[n_steps] = D after the last; hist
+        (>= n_steps + 1, 3, ...)."""
+        comp, cell = (-1, 0) if src is None else (int(src[0]), int(src[1]))
+        check(lib().cv_fdtd_step_history(self.code, self._d(), ptr(self.sig), ptr(eps), ptr(state), ptr(hist), comp,
+                                         cell, ptr(amp_dev), int(n_steps), stream_ptr()), 'fdtd step_history')
+
+    def adjoint_steps(self, lam, eps, hist, gmE, probes, g_rec, src, g_amp, n_steps):
+        """Reverse the n_steps steps of step_history in place of ``lam``; g_rec
+        (n_steps, probes) and g_amp (n_steps) may be None."""
+        pc, pl = probes
+        comp, cell = (-1, 0) if src is None else (int(src[0]), int(src[1]))
+        check(lib().cv_fdtd_adjoint_steps(self.code, self._d(), ptr(self.sig), ptr(eps), ptr(lam), ptr(self.tmp()),
+                                          ptr(hist), ptr(gmE), ptr(pc), ptr(pl), int(pc.numel()), ptr(g_rec), comp,
+                                          cell, ptr(g_amp), int(n_steps), stream_ptr()), 'fdtd adjoint_steps')
+
     def eps_grad(self, eps, gmE, geps):
         check(lib().cv_fdtd_eps_grad(self.code, self._d(), ptr(self.sig), ptr(eps), ptr(gmE), ptr(geps),
                                      stream_ptr()), 'fdtd eps_grad')
@@ -338,13 +355,14 @@ class FdtdRun(torch.autograd.Function):
     @staticmethod
     def forward(ctx, eps, amp, grid, state0, src, probes, n_steps, checkpoint_every, tm_config=None):
         # The amplitude series is read by the temporally blocked and fused
-        # kernels from device memory (a float64 device tensor is used as it
-        # is, anything else is uploaded once) and by the per-step kernels from
-        # host memory (copied once, only for those).
+        # kernels and by the reverse sweep from device memory (a float64
+        # device tensor is used as it is, anything else is uploaded once) and
+        # by the per-step kernels from host memory (copied once, only for those).
         a = amp.detach()
         amp_dev = amp_h = None
-        if tm_config != 'generic':
-            amp_dev = a.to(grid.device, torch.float64).contiguous()
+        need_grad = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
+        if tm_config != 'generic' or need_grad:
+            amp_dev = a.to(grid.device, torch.float64).contiguous().reshape(-1)
         if tm_config in ('generic', 'fused'):
             amp_h = a.to('cpu', torch.float64).numpy()
         state = state0.detach().clone()
@@ -352,7 +370,6 @@ class FdtdRun(torch.autograd.Function):
         pc, pl = probes
         rec = torch.empty((n_steps, pc.numel()), dtype=grid.dtype, device=grid.device)
         ck = max(1, int(checkpoint_every))
-        need_grad = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
         checkpoints = []
         t = 0
         if need_grad and isinstance(tm_config, int) and n_steps > 0:
@@ -420,7 +437,7 @@ class FdtdRun(torch.autograd.Function):
         # cotangent of amp[t]: lam(D_src) after step t (source added to D, fdtd.py:122-124)
         gamp = torch.zeros(n_steps, dtype=grid.dtype, device=grid.device) if ctx.needs_input_grad[1] else None
         # D history of one segment: Dhist[s] = D after step (seg_start + s)
-        Dhist = torch.empty((ck + 1, 3) + grid.shape, dtype=grid.dtype, device=grid.device)
+        Dhist = torch.empty((min(ck, n_steps) + 1, 3) + grid.shape, dtype=grid.dtype, device=grid.device)
         for sgi in range(nseg - 1, -1, -1):
             t0 = sgi * ck
             m = min(ck, n_steps - t0)
@@ -429,22 +446,9 @@ class FdtdRun(torch.autograd.Function):
                 st[TM_ARRAYS] = ctx.checkpoints[sgi].unsqueeze(-1)
             else:
                 st = ctx.checkpoints[sgi].clone()
-            Dhist[0].copy_(st[3:6])
-            for s in range(m):
-                if isinstance(ctx.tm_config, int):
-                    grid.run_tm(st, eps, src[1], ctx.amp_dev, t0 + s, 1, None, None, 0, ctx.tm_config)
-                else:
-                    grid.step(st, eps, n_steps=1, src=src, amp=ctx.amp_h[t0 + s:t0 + s + 1])
-                Dhist[s + 1].copy_(st[3:6])
-            for s in range(m - 1, -1, -1):
-                t = t0 + s
-                ga = None if gamp is None else gamp[t:t + 1]
-                if grec is not None:
-                    gp = grec[t]
-                    grid.adjoint(lam, eps, Dhist[s], gmE, probes=probes, g_probe=gp, D_t=Dhist[s + 1],
-                                 src=src, g_src=ga)
-                else:
-                    grid.adjoint(lam, eps, Dhist[s], gmE, src=src, g_src=ga)
+            grid.step_history(st, Dhist, eps, src, ctx.amp_dev[t0:t0 + m], m)
+            grid.adjoint_steps(lam, eps, Dhist, gmE, probes, None if grec is None else grec[t0:t0 + m], src,
+                               None if gamp is None else gamp[t0:t0 + m], m)
             del st
         geps = grid.eps_grad(eps, gmE, torch.zeros_like(eps)) if ctx.needs_input_grad[0] else None
         g_amp = FdtdRun._amp_grad(ctx, gamp)

@@ -139,6 +139,8 @@ _SIGS = {
     'cv_fdtd_efields_tangent': (I, [I, P, P, P, P, P, P, P, P]),
     'cv_fdtd_efields_grad': (I, [I, P, P, P, P, P, P, P, P]),
     'cv_fdtd_adjoint_step': (I, [I, P, P, P, P, P, P, P, P, P, I, P, P, I, I64, P, P]),
+    'cv_fdtd_step_history': (I, [I, P, P, P, P, P, I, I64, P, I, P]),
+    'cv_fdtd_adjoint_steps': (I, [I, P, P, P, P, P, P, P, P, P, I, P, I, I64, P, I, P]),
     'cv_fdtd_eps_grad': (I, [I, P, P, P, P, P, P]),
     'cv_fdtd_run_tm': (I, [I, P, P, P, P, P, I64, P, I, I, P, P, I, P, I, I, P]),
     'cv_fdtd_run_tm_checkpoints': (I, [I, P, P, P, P, P, P, I, I64, P, I, P, P, I, P, I, P]),

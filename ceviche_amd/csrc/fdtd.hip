@@ -17,6 +17,7 @@
 
 #include <vector>
 #include <algorithm>
+#include <initializer_list>
 #include <type_traits>
 
 namespace cv {
@@ -32,6 +33,7 @@ struct Fdtd {
     R* st;             // 18 * n
     // interior coefficients (sigma = 0): m1 and m2 for H and D
     R h1, h2, d1, d2;
+    R cdt, c0dt, half_dt, dL_r;   // c0 dt / dL, c0 dt, dt / (2 eps0), dL
 };
 
 template <typename R>
@@ -42,10 +44,6 @@ template <typename R>
 __host__ __device__ __forceinline__ const R* sigD(const Fdtd<R>& f, int a) {
     return f.sig + (f.nx + f.ny + f.nz) + (a == 0 ? 0 : (a == 1 ? f.nx : f.nx + f.ny));
 }
-
-struct Coef4 {
-    double m1, m2, m3, m4;
-};
 
 // fdtd.py:272-311 for one component; sa is the component's own-axis sigma,
 // sb, sc the other two.  sign = -1 for H (mH2, mH3 negative), +1 for D.
@@ -114,9 +112,274 @@ __host__ __device__ __forceinline__ R efield_tangent(const Fdtd<R>& f, const R* 
     return inv * dD[a * f.n + c] - (deaa * inv * inv) * D[a * f.n + c];
 }
 
+// The value of the lane above (lane + 1) or below (lane - 1); 0 beyond the wave.
+template <int CTRL>
+__device__ __forceinline__ float wave_shift(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ double wave_shift(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+template <typename R>
+__device__ __forceinline__ R lane_above(R v) { return wave_shift<0x130>(v); }   // wave_shl:1
+template <typename R>
+__device__ __forceinline__ R lane_below(R v) { return wave_shift<0x138>(v); }   // wave_shr:1
+
+// A value that is the same in every lane, kept in scalar registers.
+__device__ __forceinline__ float uniform(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ double uniform(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// The value of lane s (uniform).
+__device__ __forceinline__ float read_lane(float v, int s) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), s));
+}
+__device__ __forceinline__ double read_lane(double v, int s) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, s);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), s);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// 1 / v: the hardware's estimate (1 ulp), one Newton step and the fix-up of
+// zeros, infinities and NaN in float32 (4 operations; the division takes 11)
+__device__ __forceinline__ float recip(float v) {
+    const float r = __builtin_amdgcn_rcpf(v);
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-v, r, 1.0f), r, r), v, 1.0f);
+}
+__device__ __forceinline__ double recip(double v) { return 1.0 / v; }
+
+// ========================================= two-phase step kernels
+// The per-step kernels (H phase, D phase and their adjoints) give each thread
+// V consecutive z cells of one (x, y) line, loaded and stored as one vector:
+// they are bound by memory, and a copy with 16-byte lanes reaches 6.2 TB/s
+// where one with 4-byte lanes reaches 3.8 (8.3 against 5.6 in the Infinity
+// Cache).  Neighbours along z are the next element or the next lane; lanes at
+// the end of a line or a wave read that one element from memory.  V divides
+// nz and every base pointer is aligned to it (step_width).
+template <typename R, int V>
+struct alignas(V * sizeof(R)) Vec {
+    R v[V];
+    __device__ __forceinline__ R& operator[](int q) { return v[q]; }
+    __device__ __forceinline__ const R& operator[](int q) const { return v[q]; }
+};
+
+template <typename R, int V>
+__device__ __forceinline__ Vec<R, V> ldv(const R* p) {
+    return *reinterpret_cast<const Vec<R, V>*>(p);
+}
+template <typename R, int V>
+__device__ __forceinline__ void stv(R* p, const Vec<R, V>& x) {
+    *reinterpret_cast<Vec<R, V>*>(p) = x;
+}
+
+// The cells of this thread: line (i, j), z = k0 .. k0 + V - 1.  Threads past
+// the end repeat the last group (lane shifts need every lane) and store nothing.
+template <typename R, int V>
+struct ZGroup {
+    int i, j, k0, nz, ny;
+    bool live, lo, hi;     // lo / hi: the neighbour below / above is not in the lane beside
+    int klo, khi;          // z of the cells below and above the group
+
+    __device__ __forceinline__ explicit ZGroup(const Fdtd<R>& f) : nz(f.nz), ny(f.ny) {
+        const int64_t total = f.n / V;
+        int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+        live = g < total;
+        if (!live) g = total - 1;
+        if (total <= (int64_t)0xffffffffLL) {
+            const uint32_t u = (uint32_t)g, ng = (uint32_t)(nz / V), ij = u / ng, ii = ij / (uint32_t)ny;
+            k0 = (int)(u - ij * ng) * V;
+            i = (int)ii;
+            j = (int)(ij - ii * (uint32_t)ny);
+        } else {
+            const int64_t ng = nz / V, ij = g / ng;
+            k0 = (int)(g - ij * ng) * V;
+            i = (int)(ij / ny);
+            j = (int)(ij - (int64_t)i * ny);
+        }
+        const int lane = threadIdx.x & 63;
+        lo = k0 == 0 || lane == 0;
+        hi = k0 + V == nz || lane == 63;
+        klo = k0 == 0 ? nz - 1 : k0 - 1;
+        khi = k0 + V == nz ? 0 : k0 + V;
+    }
+    __device__ __forceinline__ int64_t line(int ii, int jj) const { return ((int64_t)ii * ny + jj) * nz; }
+    // x one cell up / down along z; edge: the value where the lane beside does not hold it
+    __device__ __forceinline__ Vec<R, V> above(const Vec<R, V>& x, R edge) const {
+        Vec<R, V> y;
+        const R next = lane_above(x[0]);
+#pragma unroll
+        for (int q = 0; q + 1 < V; ++q) y[q] = x[q + 1];
+        y[V - 1] = hi ? (nz == V ? x[0] : edge) : next;
+        return y;
+    }
+    __device__ __forceinline__ Vec<R, V> below(const Vec<R, V>& x, R edge) const {
+        Vec<R, V> y;
+        const R prev = lane_below(x[V - 1]);
+#pragma unroll
+        for (int q = V - 1; q > 0; --q) y[q] = x[q - 1];
+        y[0] = lo ? (nz == V ? x[V - 1] : edge) : prev;
+        return y;
+    }
+};
+
+// E = D / eps_aa, eps_aa = (eps + eps[-e_a]) / 2
+template <typename R, int V>
+__device__ __forceinline__ Vec<R, V> e_vec(const Vec<R, V>& d, const Vec<R, V>& e, const Vec<R, V>& em) {
+    Vec<R, V> y;
+#pragma unroll
+    for (int q = 0; q < V; ++q) y[q] = recip((e[q] + em[q]) / R(2)) * d[q];
+    return y;
+}
+
+// PML profile values b = sigma dt / (2 eps0) and r = 1 / (1 + b) of an axis.
+// The coefficients of fdtd.py:272-311 separate into them: for a component
+// with own axis a and the others b, c
+//   m1 = (1 - b_b - b_c - b_b b_c) r_b r_c,  m2 = +-c0 dt r_b r_c,
+//   m3 = 2 b_a m2,  m4 = -4 b_b b_c r_b r_c,
+// and m1 = 1, m2 = +-c0 dt where sigma is zero.
+template <typename R>
+struct Pml1 {
+    R b, r;
+    __device__ __forceinline__ Pml1() {}
+    __device__ __forceinline__ Pml1(R sigma, R half_dt) : b(sigma * half_dt) { r = recip(R(1) + b); }
+};
+template <typename R, int V>
+struct PmlZ {
+    R b[V], r[V];
+    bool any;
+    __device__ __forceinline__ void load(const R* sig, R half_dt) {
+        any = false;
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            b[q] = sig[q] * half_dt;
+            any = any || b[q] != R(0);
+        }
+    }
+    __device__ __forceinline__ void recips() {
+#pragma unroll
+        for (int q = 0; q < V; ++q) r[q] = recip(R(1) + b[q]);
+    }
+};
+
+// The axes of component a: its own and the two others' b and r at element q.
+template <int A, typename R, int V>
+__device__ __forceinline__ void pml_axes(const Pml1<R>& x, const Pml1<R>& y, const PmlZ<R, V>& z, int q, R& ba, R& bb,
+                                         R& bc, R& r) {
+    ba = A == 0 ? x.b : A == 1 ? y.b : z.b[q];
+    bb = A == 0 ? y.b : x.b;
+    bc = A == 2 ? y.b : z.b[q];
+    r = (A == 0 ? y.r : x.r) * (A == 2 ? y.r : z.r[q]);
+}
+
+// One component's update in the PML: u = m1 u + m2 dc + m3 ic + m4 iu with the
+// undivided curl difference dc (1 / dL folded into cdt = +-c0 dt / dL).  ic and
+// iu (at this thread's cells) advance where their coefficient is non-zero.
+template <int A, typename R, int V>
+__device__ __forceinline__ void pml_update(const Fdtd<R>& f, const Pml1<R>& x, const Pml1<R>& y, const PmlZ<R, V>& z,
+                                           R cdt, Vec<R, V>& u, const Vec<R, V>& dc, R* ic, R* iu, bool live) {
+    const bool has_ic = A == 0 ? x.b != R(0) : A == 1 ? y.b != R(0) : z.any;
+    const bool has_iu = A == 0 ? y.b != R(0) && z.any : A == 1 ? x.b != R(0) && z.any : x.b != R(0) && y.b != R(0);
+    Vec<R, V> i1, i2;
+    if (has_ic) i1 = ldv<R, V>(ic);
+    if (has_iu) i2 = ldv<R, V>(iu);
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+        R ba, bb, bc, r;
+        pml_axes<A>(x, y, z, q, ba, bb, bc, r);
+        const R p = bb * bc;
+        R t = dc[q];
+        if (has_ic && ba != R(0)) {
+            i1[q] += dc[q] * f.inv_dL;
+            t += R(2) * ba * f.dL_r * i1[q];
+        }
+        R v = ((R(1) - bb - bc - p) * r) * u[q] + (cdt * r) * t;
+        if (has_iu && p != R(0)) {
+            i2[q] += u[q];
+            v += (R(-4) * p * r) * i2[q];
+        }
+        u[q] = v;
+    }
+    if (live && has_ic) stv(ic, i1);
+    if (live && has_iu) stv(iu, i2);
+}
+
 // ----------------------------------------------------------------- H phase
+// H += curl E (fdtd.py:77-101) with E = D / eps_aa formed from D and eps.
+template <typename R, int V>
+__global__ void __launch_bounds__(256) k_h(Fdtd<R> f, const R* __restrict__ D) {
+    const ZGroup<R, V> g(f);
+    const int64_t n = f.n;
+    const int i = g.i, j = g.j, ip = wrapp(i, f.nx), jp = wrapp(j, f.ny), im = wrapm(i, f.nx), jm = wrapm(j, f.ny);
+    const int64_t l = g.line(i, j), c = l + g.k0, l_jp = g.line(i, jp), l_ip = g.line(ip, j);
+    const R *eps = f.eps, *Dx = D, *Dy = D + n, *Dz = D + 2 * n;
+    R* H = f.st + c;
+    const Vec<R, V> e = ldv<R, V>(eps + c), e_im = ldv<R, V>(eps + g.line(im, j) + g.k0),
+                    e_jm = ldv<R, V>(eps + g.line(i, jm) + g.k0), e_jp = ldv<R, V>(eps + l_jp + g.k0),
+                    e_jpim = ldv<R, V>(eps + g.line(im, jp) + g.k0), e_ip = ldv<R, V>(eps + l_ip + g.k0),
+                    e_ipjm = ldv<R, V>(eps + g.line(ip, jm) + g.k0);
+    const Vec<R, V> dx = ldv<R, V>(Dx + c), dy = ldv<R, V>(Dy + c), dz = ldv<R, V>(Dz + c),
+                    dx_jp = ldv<R, V>(Dx + l_jp + g.k0), dz_jp = ldv<R, V>(Dz + l_jp + g.k0),
+                    dy_ip = ldv<R, V>(Dy + l_ip + g.k0), dz_ip = ldv<R, V>(Dz + l_ip + g.k0);
+    Vec<R, V> h[3] = {ldv<R, V>(H), ldv<R, V>(H + n), ldv<R, V>(H + 2 * n)};
+    R e_lo = R(0), e_jplo = R(0), e_iplo = R(0), ex_hi = R(0), ey_hi = R(0);
+    if (g.nz != V) {
+        if (g.lo) {
+            e_lo = eps[l + g.klo];
+            e_jplo = eps[l_jp + g.klo];
+            e_iplo = eps[l_ip + g.klo];
+        }
+        if (g.hi) {
+            const R eh = eps[l + g.khi];
+            ex_hi = recip((eh + eps[g.line(im, j) + g.khi]) / R(2)) * Dx[l + g.khi];
+            ey_hi = recip((eh + eps[g.line(i, jm) + g.khi]) / R(2)) * Dy[l + g.khi];
+        }
+    }
+    const Vec<R, V> ex = e_vec(dx, e, e_im), ey = e_vec(dy, e, e_jm), ez = e_vec(dz, e, g.below(e, e_lo));
+    const Vec<R, V> ex_jp = e_vec(dx_jp, e_jp, e_jpim), ez_jp = e_vec(dz_jp, e_jp, g.below(e_jp, e_jplo));
+    const Vec<R, V> ey_ip = e_vec(dy_ip, e_ip, e_ipjm), ez_ip = e_vec(dz_ip, e_ip, g.below(e_ip, e_iplo));
+    const Vec<R, V> ex_kp = g.above(ex, ex_hi), ey_kp = g.above(ey, ey_hi);
+    Vec<R, V> dc[3];   // dL curl_E, ceviche/derivatives.py:16-22 (forward differences, periodic)
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+        dc[0][q] = (ez_jp[q] - ez[q]) - (ey_kp[q] - ey[q]);
+        dc[1][q] = (ex_kp[q] - ex[q]) - (ez_ip[q] - ez[q]);
+        dc[2][q] = (ey_ip[q] - ey[q]) - (ex_jp[q] - ex[q]);
+    }
+    const R sx = sigH(f, 0)[i], sy = sigH(f, 1)[j];
+    PmlZ<R, V> z;
+    z.load(sigH(f, 2) + g.k0, f.half_dt);
+    if (sx != R(0) || sy != R(0) || z.any) {
+        z.recips();
+        const Pml1<R> x(sx, f.half_dt), y(sy, f.half_dt);
+        pml_update<0>(f, x, y, z, -f.cdt, h[0], dc[0], H + 6 * n, H + 9 * n, g.live);
+        pml_update<1>(f, x, y, z, -f.cdt, h[1], dc[1], H + 7 * n, H + 10 * n, g.live);
+        pml_update<2>(f, x, y, z, -f.cdt, h[2], dc[2], H + 8 * n, H + 11 * n, g.live);
+    } else {
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int q = 0; q < V; ++q) h[a][q] -= f.cdt * dc[a][q];
+    }
+    if (!g.live) return;
+    stv(H, h[0]);
+    stv(H + n, h[1]);
+    stv(H + 2 * n, h[2]);
+}
+
+// ------------------------------------------------- forward-mode H phase
 // H update of cell c of the state f.st with E read through `E(a, i, j, k)`
-// (the primal E of f.st, or the tangent E of a forward-mode step).
+// (the tangent E of a forward-mode step).
 template <typename R, typename EGet>
 __host__ __device__ __forceinline__ void h_cell_with(const Fdtd<R>& f, int64_t c, EGet E) {
     int i, j, k;
@@ -162,19 +425,6 @@ __host__ __device__ __forceinline__ void h_cell_with(const Fdtd<R>& f, int64_t c
     }
 }
 
-template <typename R>
-__host__ __device__ __forceinline__ void h_cell(const Fdtd<R>& f, int64_t c) {
-    const R* D = f.st + 3 * f.n;
-    h_cell_with(f, c, [&](int a, int i, int j, int k) { return efield(f, D, a, i, j, k); });
-}
-
-template <typename R>
-__global__ void __launch_bounds__(256) k_h(Fdtd<R> f) {
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= f.n) return;
-    h_cell(f, c);
-}
-
 // tangent H update: ft.st is the tangent state, D the primal D of the same step
 template <typename R>
 __global__ void __launch_bounds__(256) k_h_tangent(Fdtd<R> ft, const R* __restrict__ D, const R* __restrict__ deps) {
@@ -186,70 +436,72 @@ __global__ void __launch_bounds__(256) k_h_tangent(Fdtd<R> ft, const R* __restri
 
 // ----------------------------------------------------------------- D phase
 struct PointSrc {
-    int comp;         // 0..2 = Jx, Jy, Jz; -1 none
+    int comp;              // 0..2 = Jx, Jy, Jz; -1 none
     int64_t cell;
     double amp;
+    const double* amp_dev; // the amplitude in device memory instead, or null
 };
 
-template <typename R>
-__host__ __device__ __forceinline__ void d_cell(const Fdtd<R>& f, const R* __restrict__ Jx, const R* __restrict__ Jy,
-                                           const R* __restrict__ Jz, R jscale, PointSrc ps, int64_t c) {
-    int i, j, k;
-    decompose(f, c, i, j, k);
+// D (read at Din, written at Dout: the same array or two) += curl H + sources
+// (fdtd.py:102-132).
+template <typename R, int V>
+__global__ void __launch_bounds__(256) k_d(Fdtd<R> f, const R* Din, R* Dout, const R* __restrict__ Jx,
+                                           const R* __restrict__ Jy, const R* __restrict__ Jz, R jscale, PointSrc ps) {
+    const ZGroup<R, V> g(f);
     const int64_t n = f.n;
-    const R* H = f.st;
-    R* D = f.st + 3 * n;
-    R* ICH = f.st + 12 * n;
-    R* ID = f.st + 15 * n;
-    const int64_t cim = cell(f, wrapm(i, f.nx), j, k), cjm = cell(f, i, wrapm(j, f.ny), k),
-                  ckm = cell(f, i, j, wrapm(k, f.nz));
-    const R* Hx = H;
-    const R* Hy = H + n;
-    const R* Hz = H + 2 * n;
-    R ch[3];
-    // curl_H, ceviche/derivatives.py:24-30 (backward differences, periodic)
-    ch[0] = ((Hz[c] - Hz[cjm]) - (Hy[c] - Hy[ckm])) * f.inv_dL;
-    ch[1] = ((Hx[c] - Hx[ckm]) - (Hz[c] - Hz[cim])) * f.inv_dL;
-    ch[2] = ((Hy[c] - Hy[cim]) - (Hx[c] - Hx[cjm])) * f.inv_dL;
-    const int pos[3] = {i, j, k};
+    const int i = g.i, j = g.j;
+    const int64_t l = g.line(i, j), c = l + g.k0, c_im = g.line(wrapm(i, f.nx), j) + g.k0,
+                  c_jm = g.line(i, wrapm(j, f.ny)) + g.k0;
+    const R *Hx = f.st, *Hy = f.st + n, *Hz = f.st + 2 * n;
+    const Vec<R, V> hx = ldv<R, V>(Hx + c), hy = ldv<R, V>(Hy + c), hz = ldv<R, V>(Hz + c),
+                    hx_jm = ldv<R, V>(Hx + c_jm), hz_jm = ldv<R, V>(Hz + c_jm), hy_im = ldv<R, V>(Hy + c_im),
+                    hz_im = ldv<R, V>(Hz + c_im);
+    Vec<R, V> d[3] = {ldv<R, V>(Din + c), ldv<R, V>(Din + n + c), ldv<R, V>(Din + 2 * n + c)};
+    R hx_lo = R(0), hy_lo = R(0);
+    if (g.lo && g.nz != V) {
+        hx_lo = Hx[l + g.klo];
+        hy_lo = Hy[l + g.klo];
+    }
+    const Vec<R, V> hx_km = g.below(hx, hx_lo), hy_km = g.below(hy, hy_lo);
+    Vec<R, V> dc[3];   // dL curl_H, ceviche/derivatives.py:24-30 (backward differences, periodic)
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+        dc[0][q] = (hz[q] - hz_jm[q]) - (hy[q] - hy_km[q]);
+        dc[1][q] = (hx[q] - hx_km[q]) - (hz[q] - hz_im[q]);
+        dc[2][q] = (hy[q] - hy_im[q]) - (hx[q] - hx_jm[q]);
+    }
+    const R sx = sigD(f, 0)[i], sy = sigD(f, 1)[j];
+    PmlZ<R, V> z;
+    z.load(sigD(f, 2) + g.k0, f.half_dt);
+    if (sx != R(0) || sy != R(0) || z.any) {
+        z.recips();
+        const Pml1<R> x(sx, f.half_dt), y(sy, f.half_dt);
+        R* aux = f.st + c;
+        pml_update<0>(f, x, y, z, f.cdt, d[0], dc[0], aux + 12 * n, aux + 15 * n, g.live);
+        pml_update<1>(f, x, y, z, f.cdt, d[1], dc[1], aux + 13 * n, aux + 16 * n, g.live);
+        pml_update<2>(f, x, y, z, f.cdt, d[2], dc[2], aux + 14 * n, aux + 17 * n, g.live);
+    } else {
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int q = 0; q < V; ++q) d[a][q] += f.cdt * dc[a][q];
+    }
+    if (!g.live) return;
     const R* J[3] = {Jx, Jy, Jz};
+    const int64_t at = ps.cell - c;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        const int ax_b = (a == 0) ? 1 : 0;
-        const int ax_c = (a == 2) ? 1 : 2;
-        const R sa = sigD(f, a)[pos[a]], sb = sigD(f, ax_b)[pos[ax_b]], sc = sigD(f, ax_c)[pos[ax_c]];
-        const int64_t ca = a * n + c;
-        const R d = D[ca];
-        R dn;
-        if (sa == R(0) && sb == R(0) && sc == R(0)) {
-            dn = f.d1 * d + f.d2 * ch[a];
-        } else {
-            R m1, m2, m3, m4;
-            coef4<R>(sa, sb, sc, R(f.dt), R(f.c0), R(f.eps0), R(1), m1, m2, m3, m4);
-            dn = m1 * d + m2 * ch[a];
-            if (sa != R(0)) {
-                const R ich = ICH[ca] + ch[a];
-                ICH[ca] = ich;
-                dn += m3 * ich;
-            }
-            if (sb != R(0) && sc != R(0)) {
-                const R idv = ID[ca] + d;
-                ID[ca] = idv;
-                dn += m4 * idv;
-            }
+        if (J[a])
+#pragma unroll
+            for (int q = 0; q < V; ++q) d[a][q] += jscale * J[a][c + q];
+        if (ps.comp == a && at >= 0 && at < V) {
+            const R amp = R(ps.amp_dev ? *ps.amp_dev : ps.amp);
+#pragma unroll
+            for (int q = 0; q < V; ++q)
+                if (at == q) d[a][q] += amp;
         }
-        if (J[a]) dn += jscale * J[a][c];
-        if (ps.comp == a && ps.cell == c) dn += R(ps.amp);
-        D[ca] = dn;
+        stv(Dout + a * n + c, d[a]);
     }
-}
-
-template <typename R>
-__global__ void __launch_bounds__(256) k_d(Fdtd<R> f, const R* __restrict__ Jx, const R* __restrict__ Jy,
-                                           const R* __restrict__ Jz, R jscale, PointSrc ps) {
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= f.n) return;
-    d_cell(f, Jx, Jy, Jz, jscale, ps, c);
 }
 
 // ------------------------------------------------------------ probe record
@@ -310,7 +562,7 @@ __global__ void __launch_bounds__(256) k_efields(Fdtd<R> f, R* __restrict__ E) {
 
 // ============================================================== adjoint
 // Adjoint state lam (18 arrays, same layout) is the cotangent of the state
-// after step t; T holds lam_H_tot between the two phases (3 arrays).
+// after step t.  With the 1/dL of the curls folded into mu:
 //   phase A:  muCH = (n2+n3) lamD + lamICH           (cells c, c+e)
 //             T    = lamH + curlE(muCH)
 //             lamICE = m3 T + lamICE;  lamIH = m4 T + lamIH;  lamH = m1 T + lamIH
@@ -319,133 +571,264 @@ __global__ void __launch_bounds__(256) k_efields(Fdtd<R> f, R* __restrict__ E) {
 //             lamID = n4 lamD + lamID; lamICH = n3 lamD + lamICH
 //             lamD = n1 lamD + lamID + mE q;   g_mE += D_{t-1} q
 // (m*: H coefficients, n*: D coefficients; curl_E^T = curl_H for periodic
-// differences, so the adjoint is a time-reversed Yee step.)
-template <typename R>
-__host__ __device__ __forceinline__ void dcoef(const Fdtd<R>& f, int kind, int a, const int pos[3], R& m1, R& m2, R& m3,
-                                      R& m4, R& sa, R& sb, R& sc) {
-    const int ax_b = (a == 0) ? 1 : 0;
-    const int ax_c = (a == 2) ? 1 : 2;
-    if (kind == 0) {
-        sa = sigH(f, a)[pos[a]];
-        sb = sigH(f, ax_b)[pos[ax_b]];
-        sc = sigH(f, ax_c)[pos[ax_c]];
-    } else {
-        sa = sigD(f, a)[pos[a]];
-        sb = sigD(f, ax_b)[pos[ax_b]];
-        sc = sigD(f, ax_c)[pos[ax_c]];
-    }
-    if (sa == R(0) && sb == R(0) && sc == R(0)) {
-        m1 = kind == 0 ? f.h1 : f.d1;
-        m2 = kind == 0 ? f.h2 : f.d2;
-        m3 = R(0);
-        m4 = R(0);
-    } else {
-        coef4<R>(sa, sb, sc, R(f.dt), R(f.c0), R(f.eps0), kind == 0 ? R(-1) : R(1), m1, m2, m3, m4);
-    }
-}
+// differences, so the adjoint is a time-reversed Yee step.)  T is stored (3
+// arrays) only by groups with an H sigma; elsewhere m1 = 1 and lamH is T.
 
-template <typename R>
-__host__ __device__ __forceinline__ R mu_ch(const Fdtd<R>& f, const R* __restrict__ lam, int a, int i, int j, int k) {
-    const int pos[3] = {i, j, k};
-    R m1, m2, m3, m4, sa, sb, sc;
-    dcoef<R>(f, 1, a, pos, m1, m2, m3, m4, sa, sb, sc);
-    const int64_t c = cell(f, i, j, k);
-    const R lD = lam[(3 + a) * f.n + c];
-    R v = (m2 + m3) * lD;
-    // lamICH is only ever fed where sigmaD_a != 0 (it is zero elsewhere)
-    if (sa != R(0)) v += lam[(12 + a) * f.n + c];
-    return v;
-}
-
-template <typename R>
-__host__ __device__ __forceinline__ void adj_a_cell(const Fdtd<R>& f, R* __restrict__ lam, R* __restrict__ T, int64_t c) {
-    int i, j, k;
-    decompose(f, c, i, j, k);
-    const int ip = wrapp(i, f.nx), jp = wrapp(j, f.ny), kp = wrapp(k, f.nz);
-    const int64_t n = f.n;
-    // curl_E applied to muCH (forward differences)
-    const R mx = mu_ch(f, lam, 0, i, j, k), my = mu_ch(f, lam, 1, i, j, k), mz = mu_ch(f, lam, 2, i, j, k);
-    R ce[3];
-    ce[0] = ((mu_ch(f, lam, 2, i, jp, k) - mz) - (mu_ch(f, lam, 1, i, j, kp) - my)) * f.inv_dL;
-    ce[1] = ((mu_ch(f, lam, 0, i, j, kp) - mx) - (mu_ch(f, lam, 2, ip, j, k) - mz)) * f.inv_dL;
-    ce[2] = ((mu_ch(f, lam, 1, ip, j, k) - my) - (mu_ch(f, lam, 0, i, jp, k) - mx)) * f.inv_dL;
-    const int pos[3] = {i, j, k};
+// m2' u + own-sigma integral: mu of component A at element q (cdt = +-c0 dt / dL).
+// with_m3: the m3 u term as well (phase A; in phase B it is in the integral).
+template <int A, bool WITH_M3, typename R, int V>
+__device__ __forceinline__ Vec<R, V> mu_vec(const Fdtd<R>& f, const Pml1<R>& x, const Pml1<R>& y,
+                                            const PmlZ<R, V>& z, R cdt, const Vec<R, V>& u, const R* ic) {
+    const bool has_ic = A == 0 ? x.b != R(0) : A == 1 ? y.b != R(0) : z.any;
+    Vec<R, V> i1, m;
+    if (has_ic) i1 = ldv<R, V>(ic);
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        R m1, m2, m3, m4, sa, sb, sc;
-        dcoef<R>(f, 0, a, pos, m1, m2, m3, m4, sa, sb, sc);
-        const int64_t ca = a * n + c;
-        const R t = lam[ca] + ce[a];
-        T[ca] = t;
-        R lih = lam[(9 + a) * n + c];
-        if (sb != R(0) && sc != R(0)) {
-            lih = m4 * t + lih;
-            lam[(9 + a) * n + c] = lih;
-        }
-        if (sa != R(0)) lam[(6 + a) * n + c] = m3 * t + lam[(6 + a) * n + c];
-        lam[ca] = m1 * t + ((sb != R(0) && sc != R(0)) ? lih : R(0));
+    for (int q = 0; q < V; ++q) {
+        R ba, bb, bc, r;
+        pml_axes<A>(x, y, z, q, ba, bb, bc, r);
+        R w = cdt * r;
+        if (WITH_M3) w += w * (R(2) * ba);
+        m[q] = w * u[q];
+        // the integral is only ever fed where the component's own sigma is non-zero
+        if (has_ic && ba != R(0)) m[q] += i1[q] * f.inv_dL;
     }
+    return m;
 }
 
-template <typename R>
-__global__ void __launch_bounds__(256) k_adj_a(Fdtd<R> f, R* __restrict__ lam, R* __restrict__ T) {
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= f.n) return;
-    adj_a_cell(f, lam, T, c);
+// the same for one cell (the neighbour of a group's edge)
+template <int A, bool WITH_M3, typename R>
+__device__ __forceinline__ R mu_one(const Fdtd<R>& f, R sx, R sy, R sz, R cdt, R u, const R* ic) {
+    if (sx == R(0) && sy == R(0) && sz == R(0)) return cdt * u;
+    const Pml1<R> x(sx, f.half_dt), y(sy, f.half_dt);
+    PmlZ<R, 1> z;
+    z.load(&sz, f.half_dt);
+    z.recips();
+    Vec<R, 1> v;
+    v[0] = u;
+    return mu_vec<A, WITH_M3, R, 1>(f, x, y, z, cdt, v, ic)[0];
 }
 
-template <typename R>
-__host__ __device__ __forceinline__ R mu_ce(const Fdtd<R>& f, const R* __restrict__ lam, const R* __restrict__ T, int a,
-                                   int i, int j, int k) {
-    const int pos[3] = {i, j, k};
-    R m1, m2, m3, m4, sa, sb, sc;
-    dcoef<R>(f, 0, a, pos, m1, m2, m3, m4, sa, sb, sc);
-    const int64_t c = cell(f, i, j, k);
-    R v = m2 * T[a * f.n + c];
-    if (sa != R(0)) v += lam[(6 + a) * f.n + c];  // updated lamICE = m3 T + lamICE'
-    return v;
-}
-
-template <typename R>
-__host__ __device__ __forceinline__ void adj_b_cell(const Fdtd<R>& f, R* __restrict__ lam, const R* __restrict__ T,
-                                               const R* __restrict__ Dprev, R* __restrict__ gmE, int64_t c) {
-    int i, j, k;
-    decompose(f, c, i, j, k);
-    const int im = wrapm(i, f.nx), jm = wrapm(j, f.ny), km = wrapm(k, f.nz);
-    const int64_t n = f.n;
-    const R ux = mu_ce(f, lam, T, 0, i, j, k), uy = mu_ce(f, lam, T, 1, i, j, k), uz = mu_ce(f, lam, T, 2, i, j, k);
-    R q[3];
-    // curl_H applied to muCE (backward differences)
-    q[0] = ((uz - mu_ce(f, lam, T, 2, i, jm, k)) - (uy - mu_ce(f, lam, T, 1, i, j, km))) * f.inv_dL;
-    q[1] = ((ux - mu_ce(f, lam, T, 0, i, j, km)) - (uz - mu_ce(f, lam, T, 2, im, j, k))) * f.inv_dL;
-    q[2] = ((uy - mu_ce(f, lam, T, 1, im, j, k)) - (ux - mu_ce(f, lam, T, 0, i, jm, k))) * f.inv_dL;
-    const int pos[3] = {i, j, k};
-    const int64_t cm[3] = {cell(f, im, j, k), cell(f, i, jm, k), cell(f, i, j, km)};
+template <int A, typename R, int V>
+__device__ __forceinline__ void adj_h_update(const Pml1<R>& x, const Pml1<R>& y, const PmlZ<R, V>& z, R c0dt, Vec<R, V>& t,
+                                             R* lam_h, R* lam_ic, R* lam_iu, R* T, bool live) {
+    const bool has_ic = A == 0 ? x.b != R(0) : A == 1 ? y.b != R(0) : z.any;
+    const bool has_iu = A == 0 ? y.b != R(0) && z.any : A == 1 ? x.b != R(0) && z.any : x.b != R(0) && y.b != R(0);
+    Vec<R, V> i1, i2, h;
+    if (has_ic) i1 = ldv<R, V>(lam_ic);
+    if (has_iu) i2 = ldv<R, V>(lam_iu);
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        R m1, m2, m3, m4, sa, sb, sc;
-        dcoef<R>(f, 1, a, pos, m1, m2, m3, m4, sa, sb, sc);
-        const int64_t ca = (3 + a) * n + c;
-        const R lD = lam[ca];
-        R lid = R(0);
-        if (sb != R(0) && sc != R(0)) {
-            lid = m4 * lD + lam[(15 + a) * n + c];
-            lam[(15 + a) * n + c] = lid;
+    for (int q = 0; q < V; ++q) {
+        R ba, bb, bc, r;
+        pml_axes<A>(x, y, z, q, ba, bb, bc, r);
+        const R p = bb * bc;
+        R v = ((R(1) - bb - bc - p) * r) * t[q];
+        if (has_iu && p != R(0)) {
+            i2[q] += (R(-4) * p * r) * t[q];
+            v += i2[q];
         }
-        if (sa != R(0)) lam[(12 + a) * n + c] = m3 * lD + lam[(12 + a) * n + c];
-        const R eaa = (f.eps[c] + f.eps[cm[a]]) / R(2);
-        const R mE = R(1) / eaa;
-        lam[ca] = m1 * lD + lid + mE * q[a];
-        if (gmE) gmE[a * n + c] += Dprev[a * n + c] * q[a];
+        if (has_ic && ba != R(0)) i1[q] += (c0dt * r * (R(2) * ba)) * t[q];
+        h[q] = v;
+    }
+    if (!live) return;
+    stv(T, t);
+    stv(lam_h, h);
+    if (has_ic) stv(lam_ic, i1);
+    if (has_iu) stv(lam_iu, i2);
+}
+
+// Phase A.  g_src (may be null): lam(D_comp) at the source cell, the cotangent
+// of the amplitude added at this step.
+template <typename R, int V>
+__global__ void __launch_bounds__(256) k_adj_a(Fdtd<R> f, R* __restrict__ lam, R* __restrict__ T, int src_comp,
+                                               int64_t src_cell, R* __restrict__ g_src) {
+    const ZGroup<R, V> g(f);
+    const int64_t n = f.n;
+    const int i = g.i, j = g.j, ip = wrapp(i, f.nx), jp = wrapp(j, f.ny);
+    const int64_t l = g.line(i, j), c = l + g.k0, c_jp = g.line(i, jp) + g.k0, c_ip = g.line(ip, j) + g.k0;
+    const R *Lx = lam + 3 * n, *Ly = lam + 4 * n, *Lz = lam + 5 * n;
+    const R* ICH = lam + 12 * n;
+    const Vec<R, V> dx = ldv<R, V>(Lx + c), dy = ldv<R, V>(Ly + c), dz = ldv<R, V>(Lz + c),
+                    dx_jp = ldv<R, V>(Lx + c_jp), dz_jp = ldv<R, V>(Lz + c_jp), dy_ip = ldv<R, V>(Ly + c_ip),
+                    dz_ip = ldv<R, V>(Lz + c_ip);
+    Vec<R, V> t[3] = {ldv<R, V>(lam + c), ldv<R, V>(lam + n + c), ldv<R, V>(lam + 2 * n + c)};
+    if (g_src && g.live && src_cell >= c && src_cell < c + V) g_src[0] = lam[(3 + src_comp) * n + src_cell];
+    const R sx = sigD(f, 0)[i], sx_ip = sigD(f, 0)[ip], sy = sigD(f, 1)[j], sy_jp = sigD(f, 1)[jp];
+    const R* sz = sigD(f, 2);
+    PmlZ<R, V> z;
+    z.load(sz + g.k0, f.half_dt);
+    Vec<R, V> mx, my, mz, mx_jp, mz_jp, my_ip, mz_ip;
+    if (sx != R(0) || sx_ip != R(0) || sy != R(0) || sy_jp != R(0) || z.any) {
+        z.recips();
+        const Pml1<R> x(sx, f.half_dt), y(sy, f.half_dt), xp(sx_ip, f.half_dt), yp(sy_jp, f.half_dt);
+        mx = mu_vec<0, true>(f, x, y, z, f.cdt, dx, ICH + c);
+        my = mu_vec<1, true>(f, x, y, z, f.cdt, dy, ICH + n + c);
+        mz = mu_vec<2, true>(f, x, y, z, f.cdt, dz, ICH + 2 * n + c);
+        mx_jp = mu_vec<0, true>(f, x, yp, z, f.cdt, dx_jp, ICH + c_jp);
+        mz_jp = mu_vec<2, true>(f, x, yp, z, f.cdt, dz_jp, ICH + 2 * n + c_jp);
+        my_ip = mu_vec<1, true>(f, xp, y, z, f.cdt, dy_ip, ICH + n + c_ip);
+        mz_ip = mu_vec<2, true>(f, xp, y, z, f.cdt, dz_ip, ICH + 2 * n + c_ip);
+    } else {
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            mx[q] = f.cdt * dx[q];
+            my[q] = f.cdt * dy[q];
+            mz[q] = f.cdt * dz[q];
+            mx_jp[q] = f.cdt * dx_jp[q];
+            mz_jp[q] = f.cdt * dz_jp[q];
+            my_ip[q] = f.cdt * dy_ip[q];
+            mz_ip[q] = f.cdt * dz_ip[q];
+        }
+    }
+    R mx_hi = R(0), my_hi = R(0);
+    if (g.hi && g.nz != V) {
+        const int64_t ch = l + g.khi;
+        mx_hi = mu_one<0, true>(f, sx, sy, sz[g.khi], f.cdt, Lx[ch], ICH + ch);
+        my_hi = mu_one<1, true>(f, sx, sy, sz[g.khi], f.cdt, Ly[ch], ICH + n + ch);
+    }
+    const Vec<R, V> mx_kp = g.above(mx, mx_hi), my_kp = g.above(my, my_hi);
+#pragma unroll
+    for (int q = 0; q < V; ++q) {   // curl_E of muCH (forward differences)
+        t[0][q] += (mz_jp[q] - mz[q]) - (my_kp[q] - my[q]);
+        t[1][q] += (mx_kp[q] - mx[q]) - (mz_ip[q] - mz[q]);
+        t[2][q] += (my_ip[q] - my[q]) - (mx_jp[q] - mx[q]);
+    }
+    const R hx = sigH(f, 0)[i], hy = sigH(f, 1)[j];
+    PmlZ<R, V> hz;
+    hz.load(sigH(f, 2) + g.k0, f.half_dt);
+    if (hx != R(0) || hy != R(0) || hz.any) {
+        hz.recips();
+        const Pml1<R> x(hx, f.half_dt), y(hy, f.half_dt);
+        const R c0dt = -f.c0dt;
+        R* at = lam + c;
+        adj_h_update<0>(x, y, hz, c0dt, t[0], at, at + 6 * n, at + 9 * n, T + c, g.live);
+        adj_h_update<1>(x, y, hz, c0dt, t[1], at + n, at + 7 * n, at + 10 * n, T + n + c, g.live);
+        adj_h_update<2>(x, y, hz, c0dt, t[2], at + 2 * n, at + 8 * n, at + 11 * n, T + 2 * n + c, g.live);
+    } else if (g.live) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) stv(lam + a * n + c, t[a]);
     }
 }
 
-template <typename R>
+template <int A, typename R, int V>
+__device__ __forceinline__ void adj_d_update(const Pml1<R>& x, const Pml1<R>& y, const PmlZ<R, V>& z, R c0dt,
+                                             Vec<R, V>& u, R* lam_ic, R* lam_iu, bool live) {
+    const bool has_ic = A == 0 ? x.b != R(0) : A == 1 ? y.b != R(0) : z.any;
+    const bool has_iu = A == 0 ? y.b != R(0) && z.any : A == 1 ? x.b != R(0) && z.any : x.b != R(0) && y.b != R(0);
+    Vec<R, V> i1, i2;
+    if (has_ic) i1 = ldv<R, V>(lam_ic);
+    if (has_iu) i2 = ldv<R, V>(lam_iu);
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+        R ba, bb, bc, r;
+        pml_axes<A>(x, y, z, q, ba, bb, bc, r);
+        const R p = bb * bc;
+        R v = ((R(1) - bb - bc - p) * r) * u[q];
+        if (has_iu && p != R(0)) {
+            i2[q] += (R(-4) * p * r) * u[q];
+            v += i2[q];
+        }
+        if (has_ic && ba != R(0)) i1[q] += (c0dt * r * (R(2) * ba)) * u[q];
+        u[q] = v;
+    }
+    if (live && has_ic) stv(lam_ic, i1);
+    if (live && has_iu) stv(lam_iu, i2);
+}
+
+// Phase B.
+template <typename R, int V>
 __global__ void __launch_bounds__(256) k_adj_b(Fdtd<R> f, R* __restrict__ lam, const R* __restrict__ T,
                                                const R* __restrict__ Dprev, R* __restrict__ gmE) {
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= f.n) return;
-    adj_b_cell(f, lam, T, Dprev, gmE, c);
+    const ZGroup<R, V> g(f);
+    const int64_t n = f.n;
+    const int i = g.i, j = g.j, im = wrapm(i, f.nx), jm = wrapm(j, f.ny);
+    const int64_t l = g.line(i, j), c = l + g.k0, c_jm = g.line(i, jm) + g.k0, c_im = g.line(im, j) + g.k0;
+    const R* ICE = lam + 6 * n;
+    const R sx = sigH(f, 0)[i], sx_im = sigH(f, 0)[im], sy = sigH(f, 1)[j], sy_jm = sigH(f, 1)[jm];
+    const R* sz = sigH(f, 2);
+    PmlZ<R, V> z;
+    z.load(sz + g.k0, f.half_dt);
+    // T of a group: the stored one where it has a sigma, lamH elsewhere
+    const R* t0 = sx != R(0) || sy != R(0) || z.any ? T : lam;
+    const R* tj = sx != R(0) || sy_jm != R(0) || z.any ? T : lam;
+    const R* ti = sx_im != R(0) || sy != R(0) || z.any ? T : lam;
+    const Vec<R, V> hx = ldv<R, V>(t0 + c), hy = ldv<R, V>(t0 + n + c), hz = ldv<R, V>(t0 + 2 * n + c),
+                    hx_jm = ldv<R, V>(tj + c_jm), hz_jm = ldv<R, V>(tj + 2 * n + c_jm),
+                    hy_im = ldv<R, V>(ti + n + c_im), hz_im = ldv<R, V>(ti + 2 * n + c_im);
+    const Vec<R, V> e = ldv<R, V>(f.eps + c), e_im = ldv<R, V>(f.eps + c_im), e_jm = ldv<R, V>(f.eps + c_jm);
+    Vec<R, V> u[3] = {ldv<R, V>(lam + 3 * n + c), ldv<R, V>(lam + 4 * n + c), ldv<R, V>(lam + 5 * n + c)};
+    Vec<R, V> dp[3], gm[3];
+    if (gmE) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            dp[a] = ldv<R, V>(Dprev + a * n + c);
+            gm[a] = ldv<R, V>(gmE + a * n + c);
+        }
+    }
+    const R cdt = -f.cdt;
+    Vec<R, V> ux, uy, uz, ux_jm, uz_jm, uy_im, uz_im;
+    if (sx != R(0) || sx_im != R(0) || sy != R(0) || sy_jm != R(0) || z.any) {
+        z.recips();
+        const Pml1<R> x(sx, f.half_dt), y(sy, f.half_dt), xm(sx_im, f.half_dt), ym(sy_jm, f.half_dt);
+        ux = mu_vec<0, false>(f, x, y, z, cdt, hx, ICE + c);
+        uy = mu_vec<1, false>(f, x, y, z, cdt, hy, ICE + n + c);
+        uz = mu_vec<2, false>(f, x, y, z, cdt, hz, ICE + 2 * n + c);
+        ux_jm = mu_vec<0, false>(f, x, ym, z, cdt, hx_jm, ICE + c_jm);
+        uz_jm = mu_vec<2, false>(f, x, ym, z, cdt, hz_jm, ICE + 2 * n + c_jm);
+        uy_im = mu_vec<1, false>(f, xm, y, z, cdt, hy_im, ICE + n + c_im);
+        uz_im = mu_vec<2, false>(f, xm, y, z, cdt, hz_im, ICE + 2 * n + c_im);
+    } else {
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            ux[q] = cdt * hx[q];
+            uy[q] = cdt * hy[q];
+            uz[q] = cdt * hz[q];
+            ux_jm[q] = cdt * hx_jm[q];
+            uz_jm[q] = cdt * hz_jm[q];
+            uy_im[q] = cdt * hy_im[q];
+            uz_im[q] = cdt * hz_im[q];
+        }
+    }
+    R ux_lo = R(0), uy_lo = R(0), e_lo = R(0);
+    if (g.lo && g.nz != V) {
+        const int64_t cl = l + g.klo;
+        const R* tl = sx != R(0) || sy != R(0) || sz[g.klo] != R(0) ? T : lam;
+        ux_lo = mu_one<0, false>(f, sx, sy, sz[g.klo], cdt, tl[cl], ICE + cl);
+        uy_lo = mu_one<1, false>(f, sx, sy, sz[g.klo], cdt, tl[n + cl], ICE + n + cl);
+        e_lo = f.eps[cl];
+    }
+    const Vec<R, V> ux_km = g.below(ux, ux_lo), uy_km = g.below(uy, uy_lo), e_km = g.below(e, e_lo);
+    Vec<R, V> qv[3];   // curl_H of muCE (backward differences)
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+        qv[0][q] = (uz[q] - uz_jm[q]) - (uy[q] - uy_km[q]);
+        qv[1][q] = (ux[q] - ux_km[q]) - (uz[q] - uz_im[q]);
+        qv[2][q] = (uy[q] - uy_im[q]) - (ux[q] - ux_jm[q]);
+    }
+    const R dx = sigD(f, 0)[i], dy = sigD(f, 1)[j];
+    PmlZ<R, V> dz;
+    dz.load(sigD(f, 2) + g.k0, f.half_dt);
+    if (dx != R(0) || dy != R(0) || dz.any) {
+        dz.recips();
+        const Pml1<R> x(dx, f.half_dt), y(dy, f.half_dt);
+        R* at = lam + c;
+        adj_d_update<0>(x, y, dz, f.c0dt, u[0], at + 12 * n, at + 15 * n, g.live);
+        adj_d_update<1>(x, y, dz, f.c0dt, u[1], at + 13 * n, at + 16 * n, g.live);
+        adj_d_update<2>(x, y, dz, f.c0dt, u[2], at + 14 * n, at + 17 * n, g.live);
+    }
+    if (!g.live) return;
+    const Vec<R, V> em[3] = {e_im, e_jm, e_km};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const Vec<R, V> w = e_vec(qv[a], e, em[a]);
+#pragma unroll
+        for (int q = 0; q < V; ++q) u[a][q] += w[q];
+        stv(lam + (3 + a) * n + c, u[a]);
+        if (gmE) {
+#pragma unroll
+            for (int q = 0; q < V; ++q) gm[a][q] += dp[a][q] * qv[a][q];
+            stv(gmE + a * n + c, gm[a]);
+        }
+    }
 }
 
 // Probe cotangent injection: lam(comp, cell) += g[p]; for E probes also
@@ -585,45 +968,6 @@ constexpr int kTmConfigs = 12;
 constexpr int kTmMaxProbes = 256;
 constexpr unsigned short kTmNoProbe = 0xffff;
 
-// The value of the lane above (lane + 1) or below (lane - 1); 0 beyond the wave.
-template <int CTRL>
-__device__ __forceinline__ float wave_shift(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-}
-template <int CTRL>
-__device__ __forceinline__ double wave_shift(double v) {
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, true);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
-    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
-template <typename R>
-__device__ __forceinline__ R lane_above(R v) { return wave_shift<0x130>(v); }   // wave_shl:1
-template <typename R>
-__device__ __forceinline__ R lane_below(R v) { return wave_shift<0x138>(v); }   // wave_shr:1
-
-// A value that is the same in every lane, kept in scalar registers.
-__device__ __forceinline__ float uniform(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
-}
-__device__ __forceinline__ double uniform(double v) {
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
-    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
-
-// The value of lane s (uniform).
-__device__ __forceinline__ float read_lane(float v, int s) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), s));
-}
-__device__ __forceinline__ double read_lane(double v, int s) {
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, s);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), s);
-    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
-
 // Probes inside a tile's region.  tm_probe_slots enters every probe whose cell
 // lies in the region (in each of its periodic copies) into s_slot[component][row][column];
 // of several probes of one component and cell the last one is entered and
@@ -681,14 +1025,6 @@ __device__ __forceinline__ int tm_wrap(int v, int n) {
     v += v < 0 ? n : 0;
     return v - (v >= n ? n : 0);
 }
-
-// 1 / v: the hardware's estimate (1 ulp) and one Newton step in float32
-__device__ __forceinline__ float tm_recip(float v) {
-    const float r = __builtin_amdgcn_rcpf(v);
-    const float s = __builtin_fmaf(__builtin_fmaf(-v, r, 1.0f), r, r);
-    return __builtin_isfinite(s) ? s : r;   // 1 / 0 and 1 / inf
-}
-__device__ __forceinline__ double tm_recip(double v) { return 1.0 / v; }
 
 // Geometry and coefficients of this thread's cells.  With b = sigma dt / (2
 // eps0) the coefficients of fdtd.py:272-311 separate by axis, 1/m0 = dt /
@@ -767,7 +1103,7 @@ struct TmCells {
             da[q] = (R(1) - cx_ - cy - cc) * r;
             db[q] = a.cdt * r;
             dc[q] = R(-4) * cc * r;
-            me[q] = tm_recip(me[q]);
+            me[q] = recip(me[q]);
         }
     }
 };
@@ -1149,9 +1485,9 @@ static TmArgs<R> tm_args(const Fdtd<R>& f) {
     a.ny = f.ny;
     a.src_i = -1;
     a.inv_dL = R(1.0 / f.dL);
-    a.dL = R(f.dL);
-    a.cdt = R(f.c0 * f.dt / f.dL);
-    a.half_dt = R(f.dt / (2.0 * f.eps0));
+    a.dL = f.dL_r;
+    a.cdt = f.cdt;
+    a.half_dt = f.half_dt;
     a.sig = f.sig;
     a.eps = f.eps;
     return a;
@@ -2127,6 +2463,10 @@ static int make_fdtd(const cv_fdtd_desc* d, const void* sig, const void* eps, vo
     f.c0 = d->c0;
     f.eps0 = d->eps0;
     f.dL = d->dL;
+    f.cdt = R(d->c0 * d->dt / d->dL);
+    f.c0dt = R(d->c0 * d->dt);
+    f.half_dt = R(d->dt / (2.0 * d->eps0));
+    f.dL_r = R(d->dL);
     f.sig = (const R*)sig;
     f.eps = (const R*)eps;
     f.st = (R*)state;
@@ -2140,11 +2480,110 @@ static int make_fdtd(const cv_fdtd_desc* d, const void* sig, const void* eps, vo
     return CV_OK;
 }
 
+// Cells per thread of the two-phase kernels: 16 bytes (4 float32 or 2 float64)
+// where nz and every array allow aligned vectors, else the widest that does.
+template <typename R>
+static int step_width(const Fdtd<R>& f, std::initializer_list<const void*> arrays) {
+    int v = 16 / (int)sizeof(R);
+    uintptr_t bits = 0;
+    for (const void* p : arrays) bits |= (uintptr_t)p;
+    while (v > 1 && (f.nz % v != 0 || bits % (v * sizeof(R)) != 0)) v >>= 1;
+    return v;
+}
+
 static inline unsigned int nblk(int64_t n) { return (unsigned int)((n + 255) / 256); }
 
 }  // namespace cv
 
 using namespace cv;
+
+namespace cv {
+
+template <typename R>
+static void launch_h(const Fdtd<R>& f, const R* D, hipStream_t s) {
+    const int v = step_width(f, {f.st, D, f.eps});
+    if constexpr (sizeof(R) == 4)
+        if (v == 4) {
+            k_h<R, 4><<<nblk(f.n / 4), 256, 0, s>>>(f, D);
+            return;
+        }
+    if (v == 2) k_h<R, 2><<<nblk(f.n / 2), 256, 0, s>>>(f, D);
+    else k_h<R, 1><<<nblk(f.n), 256, 0, s>>>(f, D);
+}
+
+template <typename R>
+static void launch_d(const Fdtd<R>& f, const R* Din, R* Dout, const R* Jx, const R* Jy, const R* Jz, R jscale,
+                     PointSrc ps, hipStream_t s) {
+    const int v = step_width(f, {f.st, Din, Dout});
+    if constexpr (sizeof(R) == 4)
+        if (v == 4) {
+            k_d<R, 4><<<nblk(f.n / 4), 256, 0, s>>>(f, Din, Dout, Jx, Jy, Jz, jscale, ps);
+            return;
+        }
+    if (v == 2) k_d<R, 2><<<nblk(f.n / 2), 256, 0, s>>>(f, Din, Dout, Jx, Jy, Jz, jscale, ps);
+    else k_d<R, 1><<<nblk(f.n), 256, 0, s>>>(f, Din, Dout, Jx, Jy, Jz, jscale, ps);
+}
+
+template <typename R>
+static void launch_adjoint(const Fdtd<R>& f, R* lam, R* T, const R* Dprev, R* gmE, int src_comp, int64_t src_cell,
+                           R* g_src, hipStream_t s) {
+    const int v = step_width(f, {lam, T, Dprev, gmE, f.eps});
+    if constexpr (sizeof(R) == 4)
+        if (v == 4) {
+            k_adj_a<R, 4><<<nblk(f.n / 4), 256, 0, s>>>(f, lam, T, src_comp, src_cell, g_src);
+            k_adj_b<R, 4><<<nblk(f.n / 4), 256, 0, s>>>(f, lam, T, Dprev, gmE);
+            return;
+        }
+    if (v == 2) {
+        k_adj_a<R, 2><<<nblk(f.n / 2), 256, 0, s>>>(f, lam, T, src_comp, src_cell, g_src);
+        k_adj_b<R, 2><<<nblk(f.n / 2), 256, 0, s>>>(f, lam, T, Dprev, gmE);
+    } else {
+        k_adj_a<R, 1><<<nblk(f.n), 256, 0, s>>>(f, lam, T, src_comp, src_cell, g_src);
+        k_adj_b<R, 1><<<nblk(f.n), 256, 0, s>>>(f, lam, T, Dprev, gmE);
+    }
+}
+
+template <typename R>
+static int step_impl(const cv_fdtd_desc* d, const void* sig, const void* eps, void* state, const void* Jx,
+                     const void* Jy, const void* Jz, double jscale, int src_comp, int64_t src_cell, const double* amp,
+                     int n_steps, const int32_t* probe_comp, const int64_t* probe_cell, int n_probes, void* rec,
+                     hipStream_t s) {
+    Fdtd<R> f;
+    int rc = make_fdtd<R>(d, sig, eps, state, f);
+    if (rc) return rc;
+    CV_CHECK(src_comp < 0 || (src_cell >= 0 && src_cell < f.n), "source cell out of range");
+    R* D = f.st + 3 * f.n;
+    for (int t = 0; t < n_steps; ++t) {
+        const PointSrc ps{src_comp, src_cell, (src_comp >= 0 && amp) ? amp[t] : 0.0, nullptr};
+        launch_h(f, D, s);
+        launch_d(f, D, D, (const R*)Jx, (const R*)Jy, (const R*)Jz, R(jscale), ps, s);
+        if (n_probes > 0)
+            k_record<R><<<(n_probes + 63) / 64, 64, 0, s>>>(f, probe_comp, probe_cell, n_probes,
+                                                            (R*)rec + (int64_t)t * n_probes);
+    }
+    CV_LAUNCH_CHECK();
+    return CV_OK;
+}
+
+template <typename R>
+static int step_history_impl(const cv_fdtd_desc* d, const void* sig, const void* eps, void* state, void* D_hist,
+                             int src_comp, int64_t src_cell, const double* amp_dev, int n_steps, hipStream_t s) {
+    Fdtd<R> f;
+    int rc = make_fdtd<R>(d, sig, eps, state, f);
+    if (rc) return rc;
+    CV_CHECK(src_comp < 0 || (src_cell >= 0 && src_cell < f.n), "source cell out of range");
+    R* D = (R*)D_hist;
+    CV_HIP(hipMemcpyAsync(D, f.st + 3 * f.n, sizeof(R) * 3 * f.n, hipMemcpyDeviceToDevice, s));
+    for (int t = 0; t < n_steps; ++t, D += 3 * f.n) {
+        const PointSrc ps{src_comp, src_cell, 0.0, src_comp >= 0 ? amp_dev + t : nullptr};
+        launch_h(f, D, s);
+        launch_d<R>(f, D, D + 3 * f.n, nullptr, nullptr, nullptr, R(1), ps, s);
+    }
+    CV_LAUNCH_CHECK();
+    return CV_OK;
+}
+
+}  // namespace cv
 
 extern "C" int cv_fdtd_step(int dtype, const cv_fdtd_desc* d, const void* sig, const void* eps, void* state,
                             const void* Jx, const void* Jy, const void* Jz, double jscale, int src_comp,
@@ -2154,39 +2593,28 @@ extern "C" int cv_fdtd_step(int dtype, const cv_fdtd_desc* d, const void* sig, c
     CV_CHECK(n_steps >= 0, "n_steps < 0");
     CV_CHECK(src_comp >= -1 && src_comp < 3, "src_comp must be -1 (none) or 0..2");
     CV_CHECK(n_probes == 0 || (probe_comp && probe_cell && rec), "probes need comp, cell and rec buffers");
-    if (dtype == CV_F32) {
-        Fdtd<float> f;
-        int rc = make_fdtd<float>(d, sig, eps, state, f);
-        if (rc) return rc;
-        CV_CHECK(src_comp < 0 || (src_cell >= 0 && src_cell < f.n), "source cell out of range");
-        for (int t = 0; t < n_steps; ++t) {
-            PointSrc ps{src_comp, src_cell, (src_comp >= 0 && amp) ? amp[t] : 0.0};
-            k_h<float><<<nblk(f.n), 256, 0, s>>>(f);
-            k_d<float><<<nblk(f.n), 256, 0, s>>>(f, (const float*)Jx, (const float*)Jy, (const float*)Jz,
-                                                 float(jscale), ps);
-            if (n_probes > 0)
-                k_record<float><<<(n_probes + 63) / 64, 64, 0, s>>>(f, probe_comp, probe_cell, n_probes,
-                                                                    (float*)rec + (int64_t)t * n_probes);
-        }
-    } else if (dtype == CV_F64) {
-        Fdtd<double> f;
-        int rc = make_fdtd<double>(d, sig, eps, state, f);
-        if (rc) return rc;
-        CV_CHECK(src_comp < 0 || (src_cell >= 0 && src_cell < f.n), "source cell out of range");
-        for (int t = 0; t < n_steps; ++t) {
-            PointSrc ps{src_comp, src_cell, (src_comp >= 0 && amp) ? amp[t] : 0.0};
-            k_h<double><<<nblk(f.n), 256, 0, s>>>(f);
-            k_d<double><<<nblk(f.n), 256, 0, s>>>(f, (const double*)Jx, (const double*)Jy, (const double*)Jz,
-                                                  jscale, ps);
-            if (n_probes > 0)
-                k_record<double><<<(n_probes + 63) / 64, 64, 0, s>>>(f, probe_comp, probe_cell, n_probes,
-                                                                     (double*)rec + (int64_t)t * n_probes);
-        }
-    } else {
-        CV_CHECK(false, "unknown dtype %d", dtype);
-    }
-    CV_LAUNCH_CHECK();
-    return CV_OK;
+    if (dtype == CV_F32)
+        return step_impl<float>(d, sig, eps, state, Jx, Jy, Jz, jscale, src_comp, src_cell, amp, n_steps, probe_comp,
+                                probe_cell, n_probes, rec, s);
+    if (dtype == CV_F64)
+        return step_impl<double>(d, sig, eps, state, Jx, Jy, Jz, jscale, src_comp, src_cell, amp, n_steps, probe_comp,
+                                 probe_cell, n_probes, rec, s);
+    CV_CHECK(false, "unknown dtype %d", dtype);
+}
+
+extern "C" int cv_fdtd_step_history(int dtype, const cv_fdtd_desc* d, const void* sig, const void* eps, void* state,
+                                    void* D_hist, int src_comp, int64_t src_cell, const double* amp_dev, int n_steps,
+                                    void* stream) {
+    hipStream_t s = as_stream(stream);
+    CV_CHECK(D_hist, "null history buffer");
+    CV_CHECK(n_steps >= 0, "n_steps < 0");
+    CV_CHECK(src_comp >= -1 && src_comp < 3, "src_comp must be -1 (none) or 0..2");
+    CV_CHECK(src_comp < 0 || amp_dev, "a source needs its amplitude array");
+    if (dtype == CV_F32)
+        return step_history_impl<float>(d, sig, eps, state, D_hist, src_comp, src_cell, amp_dev, n_steps, s);
+    if (dtype == CV_F64)
+        return step_history_impl<double>(d, sig, eps, state, D_hist, src_comp, src_cell, amp_dev, n_steps, s);
+    CV_CHECK(false, "unknown dtype %d", dtype);
 }
 
 template <typename R>
@@ -2203,12 +2631,13 @@ static int step_tangent_impl(const cv_fdtd_desc* d, const void* sig, const void*
     CV_CHECK(src_comp < 0 || (src_cell >= 0 && src_cell < f.n), "source cell out of range");
     const R* D = f.st + 3 * f.n;
     for (int t = 0; t < n_steps; ++t) {
-        PointSrc ps{src_comp, src_cell, (src_comp >= 0 && amp) ? amp[t] : 0.0};
-        PointSrc pt{src_comp, src_cell, (src_comp >= 0 && damp) ? damp[t] : 0.0};
-        k_h<R><<<nblk(f.n), 256, 0, s>>>(f);
+        PointSrc ps{src_comp, src_cell, (src_comp >= 0 && amp) ? amp[t] : 0.0, nullptr};
+        PointSrc pt{src_comp, src_cell, (src_comp >= 0 && damp) ? damp[t] : 0.0, nullptr};
+        launch_h(f, D, s);
         k_h_tangent<R><<<nblk(f.n), 256, 0, s>>>(ft, D, (const R*)deps);   // primal D still at step t
-        k_d<R><<<nblk(f.n), 256, 0, s>>>(f, (const R*)Jx, (const R*)Jy, (const R*)Jz, R(jscale), ps);
-        k_d<R><<<nblk(f.n), 256, 0, s>>>(ft, (const R*)dJx, (const R*)dJy, (const R*)dJz, R(jscale), pt);
+        R* dD = ft.st + 3 * ft.n;
+        launch_d(f, D, f.st + 3 * f.n, (const R*)Jx, (const R*)Jy, (const R*)Jz, R(jscale), ps, s);
+        launch_d(ft, dD, dD, (const R*)dJx, (const R*)dJy, (const R*)dJz, R(jscale), pt, s);
         if (n_probes > 0) {
             if (rec)
                 k_record<R><<<(n_probes + 63) / 64, 64, 0, s>>>(f, probe_comp, probe_cell, n_probes,
@@ -2299,35 +2728,33 @@ extern "C" int cv_fdtd_efields(int dtype, const cv_fdtd_desc* d, const void* sig
     return CV_OK;
 }
 
-// g_src[0] = lam(D_comp, cell): the cotangent of a point source amplitude
-// added to D at this step (the lam after the step's probe injection).
-template <typename R>
-__global__ void k_gather_src(const R* __restrict__ lam, int64_t idx, R* __restrict__ g_src) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) g_src[0] = lam[idx];
-}
+namespace cv {
 
+// n_steps adjoint steps, last first; D_hist: D before step t at D_hist + t * 3 n
 template <typename R>
-static int adjoint_step_impl(const cv_fdtd_desc* d, const void* sig, const void* eps, void* lam_, void* tmp,
-                             const void* D_prev, void* g_mE, const int32_t* probe_comp, const int64_t* probe_cell,
-                             int n_probes, const void* g_probe, const void* D_t, int src_comp, int64_t src_cell,
-                             void* g_src, hipStream_t s) {
+static int adjoint_impl(const cv_fdtd_desc* d, const void* sig, const void* eps, void* lam_, void* tmp,
+                        const void* D_prev, const void* D_after, int64_t D_stride, void* g_mE,
+                        const int32_t* probe_comp, const int64_t* probe_cell, int n_probes, const void* g_probe,
+                        int src_comp, int64_t src_cell, void* g_src, int n_steps, hipStream_t s) {
     Fdtd<R> f;
     int rc = make_fdtd<R>(d, sig, eps, lam_, f);
     if (rc) return rc;
     R* lam = (R*)lam_;
-    if (n_probes > 0)
-        k_inject<R><<<(n_probes + 255) / 256, 256, 0, s>>>(f, lam, probe_comp, probe_cell, n_probes,
-                                                           (const R*)g_probe, (const R*)D_t, (R*)g_mE);
-    if (g_src) {
-        CV_CHECK(src_comp >= 0 && src_comp < 3 && src_cell >= 0 && src_cell < f.n,
-                 "source gradient requested for an invalid source (%d, %lld)", src_comp, (long long)src_cell);
-        k_gather_src<R><<<1, 64, 0, s>>>(lam, (int64_t)(3 + src_comp) * f.n + src_cell, (R*)g_src);
+    CV_CHECK(!g_src || (src_comp >= 0 && src_comp < 3 && src_cell >= 0 && src_cell < f.n),
+             "source gradient requested for an invalid source (%d, %lld)", src_comp, (long long)src_cell);
+    for (int t = n_steps - 1; t >= 0; --t) {
+        if (n_probes > 0 && g_probe)
+            k_inject<R><<<(n_probes + 255) / 256, 256, 0, s>>>(f, lam, probe_comp, probe_cell, n_probes,
+                                                               (const R*)g_probe + (int64_t)t * n_probes,
+                                                               (const R*)D_after + t * D_stride, (R*)g_mE);
+        launch_adjoint(f, lam, (R*)tmp, (const R*)D_prev + t * D_stride, (R*)g_mE, src_comp, src_cell,
+                       g_src ? (R*)g_src + t : nullptr, s);
     }
-    k_adj_a<R><<<nblk(f.n), 256, 0, s>>>(f, lam, (R*)tmp);
-    k_adj_b<R><<<nblk(f.n), 256, 0, s>>>(f, lam, (const R*)tmp, (const R*)D_prev, (R*)g_mE);
     CV_LAUNCH_CHECK();
     return CV_OK;
 }
+
+}  // namespace cv
 
 extern "C" int cv_fdtd_adjoint_step(int dtype, const cv_fdtd_desc* d, const void* sig, const void* eps,
                                     void* lam, void* tmp, const void* D_prev, void* g_mE, const int32_t* probe_comp,
@@ -2336,11 +2763,29 @@ extern "C" int cv_fdtd_adjoint_step(int dtype, const cv_fdtd_desc* d, const void
     hipStream_t s = as_stream(stream);
     CV_CHECK(lam && tmp, "null adjoint buffers");
     if (dtype == CV_F32)
-        return adjoint_step_impl<float>(d, sig, eps, lam, tmp, D_prev, g_mE, probe_comp, probe_cell, n_probes,
-                                        g_probe, D_t, src_comp, src_cell, g_src, s);
+        return adjoint_impl<float>(d, sig, eps, lam, tmp, D_prev, D_t, 0, g_mE, probe_comp, probe_cell, n_probes,
+                                   g_probe, src_comp, src_cell, g_src, 1, s);
     if (dtype == CV_F64)
-        return adjoint_step_impl<double>(d, sig, eps, lam, tmp, D_prev, g_mE, probe_comp, probe_cell, n_probes,
-                                         g_probe, D_t, src_comp, src_cell, g_src, s);
+        return adjoint_impl<double>(d, sig, eps, lam, tmp, D_prev, D_t, 0, g_mE, probe_comp, probe_cell, n_probes,
+                                    g_probe, src_comp, src_cell, g_src, 1, s);
+    CV_CHECK(false, "unknown dtype %d", dtype);
+}
+
+extern "C" int cv_fdtd_adjoint_steps(int dtype, const cv_fdtd_desc* d, const void* sig, const void* eps, void* lam,
+                                     void* tmp, const void* D_hist, void* g_mE, const int32_t* probe_comp,
+                                     const int64_t* probe_cell, int n_probes, const void* g_rec, int src_comp,
+                                     int64_t src_cell, void* g_amp, int n_steps, void* stream) {
+    hipStream_t s = as_stream(stream);
+    CV_CHECK(d && lam && tmp && D_hist && g_mE, "null adjoint buffers");
+    CV_CHECK(n_steps >= 0, "n_steps < 0");
+    CV_CHECK(n_probes == 0 || !g_rec || (probe_comp && probe_cell), "probes need comp and cell buffers");
+    const int64_t n3 = 3 * (int64_t)d->nx * d->ny * d->nz;
+    if (dtype == CV_F32)
+        return adjoint_impl<float>(d, sig, eps, lam, tmp, D_hist, (const float*)D_hist + n3, n3, g_mE, probe_comp,
+                                   probe_cell, n_probes, g_rec, src_comp, src_cell, g_amp, n_steps, s);
+    if (dtype == CV_F64)
+        return adjoint_impl<double>(d, sig, eps, lam, tmp, D_hist, (const double*)D_hist + n3, n3, g_mE, probe_comp,
+                                    probe_cell, n_probes, g_rec, src_comp, src_cell, g_amp, n_steps, s);
     CV_CHECK(false, "unknown dtype %d", dtype);
 }
 
@@ -2613,7 +3058,7 @@ extern "C" int cv_fdtd_run_fused(int dtype, const cv_fdtd_desc* d, const void* s
         float* A = (float*)state_a;
         float* B = (float*)state_b;
         for (int t = 0; t < n_steps; ++t) {
-            PointSrc ps{comp, src_cell, 0.0};
+            PointSrc ps{comp, src_cell, 0.0, nullptr};
             int tj, chunk_s, nb_s;
             if (f.nz > 1 && slab_shape(f.nx, f.ny, f.nz, 4, tj, chunk_s, nb_s)) {
                 launch_slab<float>(f, A, B, ps, amp_dev, t0 + t, tj, chunk_s, nb_s, s);
@@ -2644,7 +3089,7 @@ extern "C" int cv_fdtd_run_fused(int dtype, const cv_fdtd_desc* d, const void* s
         double* A = (double*)state_a;
         double* B = (double*)state_b;
         for (int t = 0; t < n_steps; ++t) {
-            PointSrc ps{comp, src_cell, 0.0};
+            PointSrc ps{comp, src_cell, 0.0, nullptr};
             int tj, chunk_s, nb_s;
             if (f.nz > 1 && slab_shape(f.nx, f.ny, f.nz, 8, tj, chunk_s, nb_s)) {
                 launch_slab<double>(f, A, B, ps, amp_dev, t0 + t, tj, chunk_s, nb_s, s);

@@ -348,6 +348,21 @@ int cv_fdtd_adjoint_step(int dtype, const cv_fdtd_desc* d, const void* sig, cons
                          const void* g_probe, const void* D_t, int src_comp, int64_t src_cell,
                          void* g_src, void* stream);
 
+/* The steps of cv_fdtd_step with a point source (amplitude amp_dev[t], device
+ * float64) keeping D of every step: D before step t is D_hist + t * 3 n, D
+ * after the last one D_hist + n_steps * 3 n (row 0 is the state's D; the
+ * state's D itself is not advanced). */
+int cv_fdtd_step_history(int dtype, const cv_fdtd_desc* d, const void* sig, const void* eps, void* state,
+                         void* D_hist, int src_comp, int64_t src_cell, const double* amp_dev, int n_steps,
+                         void* stream);
+
+/* cv_fdtd_adjoint_step for the n_steps steps of cv_fdtd_step_history, last
+ * first: g_rec row t and g_amp[t] (either may be NULL) belong to step t. */
+int cv_fdtd_adjoint_steps(int dtype, const cv_fdtd_desc* d, const void* sig, const void* eps, void* lam, void* tmp,
+                          const void* D_hist, void* g_mE, const int32_t* probe_comp, const int64_t* probe_cell,
+                          int n_probes, const void* g_rec, int src_comp, int64_t src_cell, void* g_amp, int n_steps,
+                          void* stream);
+
 /* Reverse of cv_fdtd_efields for a dense cotangent gE[3][n]:
  * gD[3][n] += gE / eps_aa;  g_mE[3][n] += D * gE (g_mE may be NULL). */
 int cv_fdtd_efields_grad(int dtype, const cv_fdtd_desc* d, const void* sig, const void* eps,

@@ -507,3 +507,45 @@ def test_tm_adjoint_configs_match_generic(cfg, shape, steps, ck):
     for final in (False, True):
         for x, y in zip(got[cfg, final], got['generic', final]):
             assert float((x - y).norm()) <= 40 * steps * 2.2e-16 * float(y.norm()), (final, x.shape)
+
+
+@pytest.mark.parametrize('precision,tol', [('float64', 1e-12), ('float32', 1e-5)])
+@pytest.mark.parametrize('shape,npml', [((6, 5, 8), [1, 1, 2]), ((5, 6, 260), [1, 2, 3]), ((4, 7, 256), [0, 0, 9]),
+                                        ((7, 4, 66), [2, 0, 4]), ((9, 8, 37), [2, 2, 0]), ((5, 4, 4), [1, 1, 1]),
+                                        ((3, 130, 2), [0, 5, 0]), ((6, 70, 1), [1, 6, 0])])
+def test_step_kernels_of_every_width_match_oracle(shape, npml, precision, tol):
+    """The two-phase step and adjoint kernels where a thread holds 4, 2 or 1
+    cells along z (nz a multiple of 4, even, odd), with one group per line,
+    lines longer and shorter than a wave, a PML whose edge falls inside a
+    group and none, and an eps whose storage is not aligned to a group:
+    fields against the oracle, eps and amplitude gradients against its
+    complex step.  tol: steps * a few roundings of the precision."""
+    import ceviche_amd as cv
+    print('step widths', shape, npml, precision, flush=True)
+    rng = np.random.default_rng(sum(shape))
+    eps0 = rng.uniform(1, 6, shape)
+    steps, dL = 14, 25e-9
+    amp = rng.standard_normal(steps)
+    src = tuple(n // 2 for n in shape)
+    probes = [('Ez', src), ('Ex', (0, 0, 0)), ('Ey', tuple(n - 1 for n in shape)), ('Hx', (0, 0, shape[2] - 1)),
+              ('Hy', src), ('Hz', (shape[0] - 1, 0, 0)), ('Dz', src), ('Ez', src)]
+    wt = rng.standard_normal((steps, len(probes)))
+    dt = torch.float64 if precision == 'float64' else torch.float32
+    n = eps0.size
+    flat = torch.zeros(n + 1, dtype=dt, device='cuda')
+    flat[1:] = torch.from_numpy(eps0.ravel()).to(flat)
+    for k, base in enumerate((flat[1:].clone(), flat[1:])):      # an aligned and an unaligned eps
+        eps = base.reshape(shape).requires_grad_(True)
+        a = torch.tensor(amp, requires_grad=True)
+        F = cv.fdtd(eps, dL, npml, precision=precision)
+        rec = F.run(steps, src, a, probes, checkpoint_every=5, kernel='generic')
+        ge, ga = torch.autograd.grad((rec * torch.from_numpy(wt).to(rec)).sum(), (eps, a))
+        _, tr = _oracle_probe_energy(eps0, dL, npml, src, amp, probes)
+        assert _rel(rec.detach().cpu().numpy(), tr) <= tol
+        d, da = rng.standard_normal(shape), rng.standard_normal(steps)
+        h = 1e-30
+        _, trc = _oracle_probe_energy(eps0 + 1j * h * d, dL, npml, src, amp + 1j * h * da, probes, dtype=np.complex128)
+        want = np.sum(wt * trc.imag) / h
+        scale = float(np.abs(wt * trc.imag).sum() / h)
+        got = float((ge.detach().cpu().double().numpy() * d).sum() + (ga.numpy() * da).sum())
+        assert abs(got - want) <= 20 * tol * scale, (got, want)
