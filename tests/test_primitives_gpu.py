@@ -165,3 +165,43 @@ def test_jacobian_shapes_and_modes():
         assert np.allclose(J, A, atol=1e-5)
     with pytest.raises(ValueError):
         cv.jacobian(fn, mode='sideways')
+
+
+@pytest.mark.parametrize('n', [1, 2, 7, 16, 17, 63, 64, 65, 130, 1023, 1025, 1041, 2056, 3074])
+def test_dense_lu_blocks_and_solves(n):
+    """The blocked dense LU and its triangular solves around the edges of
+    their panels (8 and 16 columns), row capacities (1024, 2048, 3072) and
+    64-row blocks, for A, A^T and A^H and two right-hand sides, on matrices
+    whose pivots come from far below the diagonal; backward error within
+    50 n^(1/2) roundings (growth of partial pivoting on random matrices is
+    about n^(1/2) at most)."""
+    from ceviche_amd._lib import lib, ptr, stream_ptr, check
+    print('dense lu', n, flush=True)
+    g = torch.Generator().manual_seed(n)
+    A = torch.randn(n, n, generator=g, dtype=torch.complex128)
+    A[torch.arange(n), torch.arange(n)] *= 1e-3
+    B = torch.randn(n, 2, generator=g, dtype=torch.complex128)
+    dev = A.t().contiguous().cuda()                       # column-major
+    piv = torch.empty(n, dtype=torch.int32, device='cuda')
+    info = torch.full((1,), 7, dtype=torch.int32, device='cuda')
+    check(lib().cv_dense_lu(n, ptr(dev), ptr(piv), ptr(info), stream_ptr()), 'lu')
+    assert int(info.item()) == 0
+    LU = dev.t()
+    assert float(torch.tril(LU, -1).abs().max()) <= 1.5 if n > 1 else True   # multipliers of |re| + |im| pivoting
+    for trans, M in ((0, A), (1, A.t()), (2, A.conj().t())):
+        x = B.t().contiguous().cuda()
+        check(lib().cv_dense_lu_solve(n, ptr(dev), ptr(piv), ptr(x), 2, trans, stream_ptr()), 'solve')
+        X = x.t().cpu()
+        r = (M.resolve_conj() @ X - B).norm()
+        assert float(r) <= 50 * n ** 0.5 * 2.2e-16 * float(M.norm() * X.norm()), (trans, float(r))
+
+
+def test_dense_lu_reports_the_first_zero_pivot():
+    from ceviche_amd._lib import lib, ptr, stream_ptr, check
+    A = torch.eye(40, dtype=torch.complex128)
+    A[19] = A[18]                                          # rows 18 and 19 equal: column 19 has no pivot
+    dev = A.t().contiguous().cuda()
+    piv = torch.empty(40, dtype=torch.int32, device='cuda')
+    info = torch.zeros(1, dtype=torch.int32, device='cuda')
+    check(lib().cv_dense_lu(40, ptr(dev), ptr(piv), ptr(info), stream_ptr()), 'lu')
+    assert int(info.item()) == 20
