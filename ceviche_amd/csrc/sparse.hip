@@ -110,18 +110,56 @@ __global__ void __launch_bounds__(256) k_lu_update(int n, cx<double>* __restrict
 constexpr int kLuBlockedRows = 3072;
 constexpr int kLuThreads = 1024;
 
-// |re| + |im| as a key whose order is the value's (NaN counts as 0)
-__device__ __forceinline__ uint64_t lu_key(cx<double> a) {
+// |re| + |im| (NaN counts as 0)
+__device__ __forceinline__ double lu_size(cx<double> a) {
     const double m = fabs(a.re) + fabs(a.im);
-    return m >= 0.0 ? __builtin_bit_cast(uint64_t, m) : 0;
+    return m >= 0.0 ? m : 0.0;
 }
 
-// larger key, then lower row
-__device__ __forceinline__ void lu_better(uint64_t& k, int& r, uint64_t k2, int r2) {
-    if (k2 > k || (k2 == k && r2 < r)) {
-        k = k2;
-        r = r2;
-    }
+// max of the non-negative values v over lanes, by lane exchanges inside the
+// vector unit (an LDS shuffle takes some 100 cycles a step): the lanes of a
+// row of 16 (ROW) or the whole wave
+template <int CTRL>
+__device__ __forceinline__ double lu_dpp_max(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+    return fmax(v, __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo));
+}
+__device__ __forceinline__ double lu_lane(double v, int lane) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), lane);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+template <bool ROW>
+__device__ __forceinline__ double lu_max(double v) {
+    v = lu_dpp_max<0x111>(v);   // row_shr:1
+    v = lu_dpp_max<0x112>(v);
+    v = lu_dpp_max<0x114>(v);
+    v = lu_dpp_max<0x118>(v);
+    if (ROW) return lu_lane(v, 15);
+    v = lu_dpp_max<0x142>(v);   // row_bcast:15
+    v = lu_dpp_max<0x143>(v);   // row_bcast:31
+    return lu_lane(v, 63);
+}
+
+// lowest row among the lanes of `mask`
+__device__ __forceinline__ int lu_min_row(uint64_t mask, int row) {
+    int best = __builtin_amdgcn_readlane(row, __builtin_ctzll(mask));
+    for (mask &= mask - 1; mask; mask &= mask - 1) best = min(best, __builtin_amdgcn_readlane(row, __builtin_ctzll(mask)));
+    return best;
+}
+
+// 1 / d by the hardware's estimate of 1 / |d|^2 and two Newton steps (the
+// division's 30 operations would be issued by all 16 waves for every column)
+__device__ __forceinline__ cx<double> lu_recip(cx<double> d) {
+    const double x = d.re * d.re + d.im * d.im;
+    double r = __builtin_amdgcn_rcp(x);
+    r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+    r = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+    r = __builtin_amdgcn_div_fixup(r, x, 1.0);
+    return mk(d.re * r, -d.im * r);
 }
 
 // LU with partial pivoting of the m x w panel at P (rows k .. k + m - 1 of the
@@ -132,7 +170,7 @@ __device__ __forceinline__ void lu_better(uint64_t& k, int& r, uint64_t k2, int 
 template <int NB, int RPT>
 __global__ void __launch_bounds__(kLuThreads)
 k_lu_panel_z(int n, cx<double>* __restrict__ A, int k, int w, int32_t* __restrict__ piv, int32_t* __restrict__ info) {
-    __shared__ uint64_t s_key[2][kLuThreads / 64];
+    __shared__ double s_max[2][kLuThreads / 64];
     __shared__ int s_row[2][kLuThreads / 64];
     __shared__ cx<double> s_piv[2][NB], s_top[2][NB];
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -149,36 +187,32 @@ k_lu_panel_z(int n, cx<double>* __restrict__ A, int k, int w, int32_t* __restric
     for (int c = 0; c < NB; ++c) {
         if (c < w) {   // uniform
         const int sl = c & 1;
-        uint64_t key = 0;
-        int row = m;
+        double best = 0.0;
+        int row = c;
 #pragma unroll
-        for (int q = 0; q < RPT; ++q) {
+        for (int q = RPT - 1; q >= 0; --q) {
             const int r = t + q * kLuThreads;
-            if (r >= c && r < m) lu_better(key, row, lu_key(a[q][c]), r);
+            const double v = r >= c && r < m ? lu_size(a[q][c]) : -1.0;
+            if (v >= best) {   // of equal values the lower row
+                best = v;
+                row = r;
+            }
         }
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-            const uint64_t k2 = __shfl_xor((unsigned long long)key, off, 64);
-            const int r2 = __shfl_xor(row, off, 64);
-            lu_better(key, row, k2, r2);
-        }
+        // a wave without a non-zero candidate proposes row c (not taken unless all are zero)
+        const double wmax = lu_max<false>(best);
+        const int wrow = wmax == 0.0 ? c : lu_min_row(__ballot(best == wmax), row);
         if (lane == 0) {
-            s_key[sl][wave] = key;
-            s_row[sl][wave] = row;
+            s_max[sl][wave] = wmax;
+            s_row[sl][wave] = wrow;
         }
         __syncthreads();
-        key = s_key[sl][lane & 15];
+        best = s_max[sl][lane & 15];
         row = s_row[sl][lane & 15];
-#pragma unroll
-        for (int off = 8; off >= 1; off >>= 1) {
-            const uint64_t k2 = __shfl_xor((unsigned long long)key, off, 64);
-            const int r2 = __shfl_xor(row, off, 64);
-            lu_better(key, row, k2, r2);
-        }
-        const int p = __builtin_amdgcn_readfirstlane(row);   // c <= p < m: the candidates include row c
+        const double pmax = lu_max<true>(best);
+        const int p = pmax == 0.0 ? c : lu_min_row(__ballot(best == pmax) & 0xffff, row);   // c <= p < m
         if (t == 0) {
             piv[k + c] = k + p;
-            if (key == 0 && *info == 0) *info = k + c + 1;
+            if (pmax == 0.0 && *info == 0) *info = k + c + 1;
         }
         // rows c and p change places; the pivot row goes to everyone
 #pragma unroll
@@ -194,7 +228,7 @@ k_lu_panel_z(int n, cx<double>* __restrict__ A, int k, int w, int32_t* __restric
         __syncthreads();
         const cx<double> d = s_piv[sl][c];
         const bool zero = d.re == 0.0 && d.im == 0.0;
-        const cx<double> inv = zero ? czero<double>() : cdiv(cone<double>(), d);
+        const cx<double> inv = zero ? czero<double>() : lu_recip(d);
 #pragma unroll
         for (int q = 0; q < RPT; ++q) {
             const int r = t + q * kLuThreads;
@@ -363,10 +397,11 @@ k_lu_tri(int n, const cx<double>* __restrict__ LU, cx<double>* __restrict__ B, i
     if (w != 0) return;
     cx<double> inv = cone<double>();
     if (!kUnit) inv = row < n ? cdiv(cone<double>(), s_t[lane][lane]) : cone<double>();
+#pragma unroll 8
     for (int s = 0; s < kTri; ++s) {
         const int j = kForward ? s : kTri - 1 - s;
         const cx<double> x = kUnit ? v : v * inv;
-        const cx<double> xj = mk(__shfl(x.re, j, 64), __shfl(x.im, j, 64));
+        const cx<double> xj = mk(lu_lane(x.re, j), lu_lane(x.im, j));
         if (lane == j) v = xj;
         const bool rest = kForward ? lane > j : lane < j;
         if (rest) v = v - (kTrans ? s_t[lane][j] : s_t[j][lane]) * xj;
@@ -388,13 +423,28 @@ k_lu_permute(int n, const int32_t* __restrict__ piv, cx<double>* __restrict__ B,
         s_p[i] = piv[i];
     }
     __syncthreads();
-    if (threadIdx.x == 0)
-        for (int q = 0; q < n; ++q) {
-            const int i = forward ? q : n - 1 - q, p = s_p[i];
-            const int a = s_idx[i], c = s_idx[p];
-            s_idx[i] = c;
-            s_idx[p] = a;
+    // one wave, 64 interchanges at a time: each lane traces what ends up in one
+    // of the block's rows and in its partner
+    if (threadIdx.x < 64) {
+        const int lane = threadIdx.x, nblk = (n + 63) / 64;
+        for (int k = 0; k < nblk; ++k) {
+            const int first = (forward ? k : nblk - 1 - k) * 64, i = first + lane;
+            const int p = i < n ? s_p[i] : i;
+            int src1 = i, src2 = p;
+            for (int q = 0; q < 64; ++q) {
+                const int c = forward ? 63 - q : q, x = first + c, y = __builtin_amdgcn_readlane(p, c);
+                src1 = src1 == x ? y : src1 == y ? x : src1;
+                src2 = src2 == x ? y : src2 == y ? x : src2;
+            }
+            const int v1 = i < n ? s_idx[src1] : 0, v2 = i < n ? s_idx[src2] : 0;
+            __builtin_amdgcn_wave_barrier();
+            if (i < n) {
+                s_idx[i] = v1;
+                s_idx[p] = v2;
+            }
+            __builtin_amdgcn_wave_barrier();
         }
+    }
     __syncthreads();
     constexpr int kMost = kLuPermuteLds / 1024;
     cx<double> v[kMost];
