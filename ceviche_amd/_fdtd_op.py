@@ -14,6 +14,7 @@ Two differentiable paths:
     backward with the adjoint kernels).
 """
 import ctypes
+from itertools import chain
 
 import numpy as np
 import torch
@@ -334,18 +335,20 @@ def autotune_tm(grid, eps, steps=64, reps=2):
 
 
 def _probe_tensors(grid, probes):
-    comps = []
-    cells = []
-    for name, pos in probes:
-        comps.append(COMPONENTS[name] if isinstance(name, str) else int(name))
-        pos = tuple(pos) + (0,) * (3 - len(pos))
-        i, j, k = (int(v) for v in pos)
-        if not (0 <= i < grid.nx and 0 <= j < grid.ny and 0 <= k < grid.nz):
-            raise ValueError('probe position %s outside the grid %s' % (pos, grid.shape))
-        cells.append((i * grid.ny + j) * grid.nz + k)
-    pc = torch.tensor(comps, dtype=torch.int32, device=grid.device)
-    pl = torch.tensor(cells, dtype=torch.int64, device=grid.device)
-    return pc, pl
+    """(component int32, flat cell int64) device tensors of point probes."""
+    names, pos = zip(*probes) if probes else ((), ())
+    code = {c: COMPONENTS[c] if isinstance(c, str) else int(c) for c in set(names)}
+    comps = np.fromiter(map(code.__getitem__, names), np.int32, len(names))
+    if set(map(len, pos)) - {3}:
+        pos = [tuple(p) + (0,) * (3 - len(p)) for p in pos]
+        if max(map(len, pos)) > 3:
+            raise ValueError('a probe position has at most three indices')
+    xyz = np.fromiter(map(int, chain.from_iterable(pos)), np.int64, 3 * len(pos)).reshape(-1, 3)
+    bad = ((xyz < 0) | (xyz >= np.array(grid.shape))).any(axis=1)
+    if bad.any():
+        raise ValueError('probe position %s outside the grid %s' % (tuple(pos[int(bad.argmax())]), grid.shape))
+    cells = (xyz[:, 0] * grid.ny + xyz[:, 1]) * grid.nz + xyz[:, 2]
+    return torch.from_numpy(comps).to(grid.device), torch.from_numpy(cells).to(grid.device)
 
 
 class FdtdRun(torch.autograd.Function):
