@@ -41,11 +41,10 @@
 //   down: x_I = y_I - G^T x_B
 // (A^T = [[F_II^T, F_BI^T], [F_IB^T, F_BB^T]], F_IB^T F_II^-T = X^T and
 // F_II^-T F_BI^T = G^T).  Each product is one launch for all nodes of a
-// level (a workgroup per node up to 256 rows and columns, else 64 x 64 tiles
-// with partial sums added by a second launch), the input gathered from the
-// work vector.  Nodes of a level share boundary cells (the two sides of a
-// separator), so their b_B contributions are summed per cell in a fixed
-// order by one more launch.
+// level.  The up sweep is multifrontal: a node keeps what its subtree
+// subtracts from its ring cells (its own t plus its children's, at the
+// positions of its ring) and its parent gathers from its two children, so no
+// cell is written by two nodes and no launch sums them.
 #include "fdfd_stencil.h"
 
 #include <rocblas/rocblas.h>
@@ -59,7 +58,6 @@ namespace cv {
 namespace {
 
 constexpr int kLeafCells = 32;
-constexpr int kMvTile = 64;        // rows and columns of one tile of the application products
 constexpr int kNdSolveMin = 64;   // interior blocks above this size: [Q X] directly, not the inverse and a product
 constexpr int kLuPanel = 16;      // columns per panel of the blocked Gauss-Jordan
 constexpr int kLuMin = 64;        // interior blocks above this size take the blocked Gauss-Jordan ...
@@ -79,11 +77,12 @@ struct NdLevel {
     // below this node)
     std::vector<int32_t> anbr;
     std::vector<NdGroup> groups;           // children's Schur complements, extend-added slot by slot
-    // the level's boundary cells, each with its contributions e * bmax + j
-    // (several nodes of a level can border the same separator cell)
-    std::vector<int32_t> bs_cells, bs_ptr, bs_idx;
+    // per node and [I; B] position the entries of its two children's ring sums
+    // that fall on it (indices into the sums of all levels, -1: none)
+    std::vector<int32_t> up;
+    int64_t t0 = 0;                        // first ring sum of the level
     // byte offsets of the device copies (plan buffer) and of the numeric data (factor buffer)
-    int64_t off_icells = 0, off_bcells = 0, off_anbr = 0, off_bs_cells = 0, off_bs_ptr = 0, off_bs_idx = 0;
+    int64_t off_icells = 0, off_bcells = 0, off_anbr = 0, off_up = 0;
     int64_t off_F = 0, off_piv = 0, info_first = 0;
 };
 
@@ -94,7 +93,7 @@ struct cv_nd_plan {
     int nx = 0, ny = 0;
     std::vector<cv::NdLevel> L;
     int64_t plan_bytes = 0, factor_bytes = 0;
-    int64_t off_w = 0, off_part = 0, off_tb = 0, off_info = 0, off_r = 0, off_r2 = 0;
+    int64_t off_w = 0, off_t = 0, off_info = 0, off_r = 0, off_r2 = 0;
     int64_t n_nodes = 0;
     double flops = 0.0;   // real flops of one numeric factorisation (unpadded sizes)
 };
@@ -225,12 +224,15 @@ extern "C" cv_nd_plan* cv_nd_plan_create(int nx, int ny) {
     for (size_t q = 0; q < nodes.size(); ++q) members[nodes[q].height].push_back((int)q);
     // position of a cell in the current node's [I; B] ordering
     std::vector<int32_t> pos(N, -1);
+    int64_t t_total = 0;
     for (int h = 0; h <= H; ++h) {
         NdLevel& L = P->L[h];
         L.icells.assign((size_t)L.nb * L.kmax, -1);
         L.bcells.assign((size_t)L.nb * L.bmax, -1);
         L.anbr.assign((size_t)L.nb * L.kmax * 4, -1);
-        std::vector<std::pair<int32_t, int32_t>> contrib;   // (boundary cell, e * bmax + j)
+        L.up.assign(h > 0 ? (size_t)L.nb * L.m * 2 : 0, -1);
+        L.t0 = t_total;
+        t_total += (int64_t)L.nb * L.bmax;
         for (int q : members[h]) {
             const Box& b = nodes[q];
             const int e = level_index[q];
@@ -241,7 +243,6 @@ extern "C" cv_nd_plan* cv_nd_plan_create(int nx, int ny) {
             for (size_t p = 0; p < b.B.size(); ++p) {
                 L.bcells[(size_t)e * L.bmax + p] = b.B[p];
                 pos[b.B[p]] = (int32_t)(L.kmax + p);
-                contrib.emplace_back(b.B[p], (int32_t)((int64_t)e * L.bmax + p));
             }
             for (size_t p = 0; p < b.I.size(); ++p) {
                 int32_t nbv[4];
@@ -275,6 +276,8 @@ extern "C" cv_nd_plan* cv_nd_plan_create(int nx, int ny) {
                             return nullptr;
                         }
                         g->map[base + p] = ps;
+                        L.up[((size_t)e * L.m + ps) * 2 + side] =
+                            (int32_t)(CL.t0 + (int64_t)level_index[cq] * CL.bmax + (int64_t)p);
                     }
                 }
             }
@@ -285,19 +288,9 @@ extern "C" cv_nd_plan* cv_nd_plan_create(int nx, int ny) {
         std::stable_sort(L.groups.begin(), L.groups.end(), [](const NdGroup& x, const NdGroup& y) {
             return x.child_level != y.child_level ? x.child_level < y.child_level : x.slot < y.slot;
         });
-        std::sort(contrib.begin(), contrib.end());
-        L.bs_ptr.push_back(0);
-        for (size_t i = 0; i < contrib.size(); ++i) {
-            if (i == 0 || contrib[i].first != contrib[i - 1].first) {
-                if (i > 0) L.bs_ptr.push_back((int32_t)i);
-                L.bs_cells.push_back(contrib[i].first);
-            }
-            L.bs_idx.push_back(contrib[i].second);
-        }
-        if (!contrib.empty()) L.bs_ptr.push_back((int32_t)contrib.size());
     }
     // device layouts: index arrays in the plan buffer, numeric data in the factor buffer
-    int64_t po = 0, fo = 0, pmax = 0, rmax = 0, r2max = 0, tbmax = 0, info_first = 0;
+    int64_t po = 0, fo = 0, rmax = 0, r2max = 0, info_first = 0;
     auto take = [](int64_t& o, int64_t bytes) {
         const int64_t r = o;
         o += al256(bytes);
@@ -312,27 +305,19 @@ extern "C" cv_nd_plan* cv_nd_plan_create(int nx, int ny) {
             g.off_child = take(po, 4 * (int64_t)g.child.size());
             g.off_map = take(po, 4 * (int64_t)g.map.size());
         }
-        L.off_bs_cells = take(po, 4 * (int64_t)L.bs_cells.size());
-        L.off_bs_ptr = take(po, 4 * (int64_t)L.bs_ptr.size());
-        L.off_bs_idx = take(po, 4 * (int64_t)L.bs_idx.size());
+        L.off_up = take(po, 4 * (int64_t)L.up.size());
         L.off_F = take(fo, 8 * (int64_t)L.nb * L.m * L.m);
         L.off_piv = take(fo, 4 * (int64_t)L.nb * std::max(1, L.kmax));
         L.info_first = info_first;
         info_first += L.nb;
-        // partial sums of the tiled products: per node ceil(k/64) tiles of m
-        // outputs (up sweeps) or ceil(b/64) tiles of k outputs (down sweeps)
-        pmax = std::max<int64_t>(pmax, (int64_t)L.nb * std::max<int64_t>((int64_t)((L.kmax + kMvTile - 1) / kMvTile) * L.m,
-                                                                        (int64_t)((L.bmax + kMvTile - 1) / kMvTile) * L.kmax));
         rmax = std::max<int64_t>(rmax, (int64_t)L.nb * L.kmax * L.m);
         if (L.kmax > kLuMin && L.kmax <= kLuMaxRows)   // the blocked Gauss-Jordan's second buffer
             r2max = std::max<int64_t>(r2max, (int64_t)L.nb * L.kmax * (L.kmax + L.m));
-        tbmax = std::max<int64_t>(tbmax, (int64_t)L.nb * L.bmax);
     }
     P->n_nodes = info_first;
     P->off_info = take(fo, 4 * info_first);
     P->off_w = take(fo, 8 * N);
-    P->off_part = take(fo, 8 * std::max<int64_t>(1, pmax));
-    P->off_tb = take(fo, 8 * std::max<int64_t>(1, tbmax));
+    P->off_t = take(fo, 8 * std::max<int64_t>(1, t_total));
     P->off_r = take(fo, 8 * std::max<int64_t>(1, rmax));
     P->off_r2 = take(fo, 8 * std::max<int64_t>(1, r2max));
     P->plan_bytes = std::max<int64_t>(po, 256);
@@ -371,8 +356,7 @@ extern "C" int cv_nd_plan_upload(const cv_nd_plan* p, void* plan_dev, int64_t pl
     for (const auto& L : p->L) {
         int rc = CV_OK;
         if ((rc = up(L.off_icells, L.icells)) || (rc = up(L.off_bcells, L.bcells)) || (rc = up(L.off_anbr, L.anbr)) ||
-            (rc = up(L.off_bs_cells, L.bs_cells)) || (rc = up(L.off_bs_ptr, L.bs_ptr)) ||
-            (rc = up(L.off_bs_idx, L.bs_idx)))
+            (rc = up(L.off_up, L.up)))
             return rc;
         for (const auto& g : L.groups)
             if ((rc = up(g.off_parent, g.parent)) || (rc = up(g.off_child, g.child)) || (rc = up(g.off_map, g.map)))
@@ -1057,205 +1041,170 @@ k_nd_block_copy(const cx<float>* __restrict__ src, int64_t src_stride, int src_l
     dst[(int64_t)e * dst_stride + (int64_t)j * dst_ld + i] = src[(int64_t)e * src_stride + (int64_t)j * src_ld + i];
 }
 
-// One 64 x 64 tile of a per-node product over a block of F (rows row0..,
-// columns col0.., M x N, column-major with leading dimension m).  The input
-// vector is gathered from the work vector w through xcells (xn entries per
-// node, -1 = padding).  TRANS = 0: y = A x, the four waves take 16 columns
-// each, lanes the rows, the wave sums combined through LDS; partial sums per
-// column tile in part[(e * tn + tj) * M + i].  TRANS = 1: y = A^T x, lanes
-// the rows, each wave 16 output columns reduced over the lanes; partial sums
-// per row tile in part[(e * tm + ti) * N + j].  Workgroups are node-major.
-template <bool TRANS>
-__global__ void __launch_bounds__(256)
-k_nd_mv(const cx<float>* __restrict__ F, int m, int row0, int col0, int M, int N, int tm, int tn,
-        const int32_t* __restrict__ xcells, int xn, const cx<float>* __restrict__ w, cx<float>* __restrict__ part) {
-    const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int per = tm * tn;
-    const int e = blockIdx.x / per;
-    const int rem = blockIdx.x - e * per;
-    const int ti = rem / tn, tj = rem - ti * tn;
-    const int i = ti * kMvTile + lane;
-    const cx<float>* A = F + (int64_t)e * m * m + row0 + (int64_t)col0 * m;
-    const int32_t* xc = xcells + (int64_t)e * xn;
-    const int j0 = tj * kMvTile + wid * 16;
-    if (!TRANS) {
-        __shared__ cx<float> red[4][kMvTile];
-        cx<float> acc = czero<float>();
-        if (i < M) {
-#pragma unroll
-            for (int c = 0; c < 16; ++c) {
-                const int j = j0 + c;
-                if (j < N) {
-                    const int32_t cell = xc[j];
-                    const cx<float> xj = cell >= 0 ? w[cell] : czero<float>();
-                    acc = acc + A[i + (int64_t)j * m] * xj;
-                }
-            }
+// One product of the application over a block of every node's F (rows
+// row0.., columns col0..): the input is gathered into LDS, the output goes to
+// its cells and ring sums, all in one launch per level and sweep.
+//   UP:   input v at the interior cells less the children's ring sums; outputs
+//         o < k to the work vector at the interior cells (y), o >= k plus the
+//         children's sums there to the node's ring sum o - k;
+//   down: input the work vector at the ring cells (x_B); x = y - output.
+// Bound by latency: index, gather and matrix loads of a launch follow each
+// other, so the first matrix loads are issued before the gather, and the tile
+// of a workgroup is chosen (nd_product) to keep many of them in flight.  The
+// 32 partial-sum and ring-sum launches these kernels used to need took a
+// third of an application at 1024^2.
+struct NdProduct {
+    const cx<float>* F;
+    int m, row0, col0, nout, nin, k, b;
+    const int32_t *icells, *bcells, *up;   // up: null for leaves
+    const cx<float>* v;
+    cx<float> *T, *w, *z;                  // z: the solution, written with w (null: not final)
+    int64_t t0;
+};
+
+constexpr int kMvChunk = 2048;   // inputs in LDS at a time, at most
+
+template <bool UP>
+__device__ __forceinline__ cx<float> nd_input(const NdProduct& a, int e, int q) {
+    if (UP) {
+        const int32_t c = a.icells[(int64_t)e * a.k + q];
+        if (c < 0) return czero<float>();
+        cx<float> x = a.v[c];
+        if (a.up) {
+            const int32_t* u = a.up + ((int64_t)e * a.m + q) * 2;
+            const int32_t u0 = u[0], u1 = u[1];
+            cx<float> t = u0 >= 0 ? a.T[u0] : czero<float>();
+            if (u1 >= 0) t = t + a.T[u1];
+            x = x - t;
         }
-        red[wid][lane] = acc;
+        return x;
+    }
+    const int32_t c = a.bcells[(int64_t)e * a.b + q];
+    return c >= 0 ? a.w[c] : czero<float>();
+}
+
+template <bool UP>
+__device__ __forceinline__ void nd_output(const NdProduct& a, int e, int o, cx<float> acc) {
+    if (UP && o >= a.k) {
+        if (a.up) {
+            const int32_t* u = a.up + ((int64_t)e * a.m + o) * 2;
+            const int32_t u0 = u[0], u1 = u[1];
+            if (u0 >= 0) acc = acc + a.T[u0];
+            if (u1 >= 0) acc = acc + a.T[u1];
+        }
+        a.T[a.t0 + (int64_t)e * a.b + (o - a.k)] = acc;
+        return;
+    }
+    const int32_t c = a.icells[(int64_t)e * a.k + o];
+    if (c < 0) return;
+    if (!UP) acc = a.w[c] - acc;
+    a.w[c] = acc;
+    if (a.z) a.z[c] = acc;
+}
+
+// y = A x: TR output rows per workgroup (a lane per row), the inputs dealt to
+// the NT / TR slices, summed by lane exchanges within a wave and through LDS
+// across waves.
+template <bool UP, int TR, int NT>
+__global__ void __launch_bounds__(NT) k_nd_mv(NdProduct a, int tiles) {
+    // launch_mv's rule leaves at most 32 loads a thread, so 256 (1024) inputs
+    // to a workgroup of 64 (256) threads
+    constexpr int S = NT / TR, U = 8, W = NT / 64, CH = NT == 64 ? 256 : NT == 256 ? 1024 : kMvChunk;
+    __shared__ cx<float> xs[CH + U * S];
+    __shared__ cx<float> red[W][TR];
+    const int tid = threadIdx.x, r = tid % TR, sl = tid / TR;
+    const int e = blockIdx.x / tiles, o = (blockIdx.x - e * tiles) * TR + r;
+    const int64_t m = a.m;
+    const cx<float>* A = a.F + e * m * m + a.row0 + a.col0 * m + min(o, a.nout - 1);
+    cx<float> acc = czero<float>();
+    for (int q0 = 0; q0 < a.nin; q0 += CH) {
+        const int n = min(CH, a.nin - q0);
+        const cx<float>* Aq = A + q0 * m;
+        cx<float> f[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) f[u] = Aq[min(sl + u * S, n - 1) * m];
+        if (q0 > 0) __syncthreads();
+        // entries past the end are zero, so the loop needs no remainder
+        for (int q = tid; q < n + U * S; q += NT) xs[q] = q < n ? nd_input<UP>(a, e, q0 + q) : czero<float>();
         __syncthreads();
-        if (wid == 0 && i < M) {
-            const cx<float> v = red[0][lane] + red[1][lane] + red[2][lane] + red[3][lane];
-            part[((int64_t)e * tn + tj) * M + i] = v;
-        }
-    } else {
-        cx<float> xi = czero<float>();
-        if (i < M) {
-            const int32_t cell = xc[i];
-            if (cell >= 0) xi = w[cell];
-        }
+        for (int q = sl; q < n; q += U * S) {
+            cx<float> g[U];
+            const bool more = q + U * S < n;
+            if (more)
 #pragma unroll
-        for (int c = 0; c < 16; ++c) {
-            const int j = j0 + c;
-            cx<float> v = (i < M && j < N) ? A[i + (int64_t)j * m] * xi : czero<float>();
+                for (int u = 0; u < U; ++u) g[u] = Aq[min(q + (U + u) * S, n - 1) * m];
 #pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                v.re += __shfl_xor(v.re, off);
-                v.im += __shfl_xor(v.im, off);
-            }
-            if (lane == 0 && j < N) part[((int64_t)e * tm + ti) * N + j] = v;
+            for (int u = 0; u < U; ++u) acc = acc + f[u] * xs[q + u * S];
+            if (more)
+#pragma unroll
+                for (int u = 0; u < U; ++u) f[u] = g[u];
         }
     }
-}
-
-// The same product for nodes of at most kMvNode rows and columns, one
-// workgroup per node, fused with the gather and the scatter (a node's input
-// and output cells belong to that node alone within a level): the input is
-// gathered into LDS, then one thread per output, 16 independent loads in
-// flight: TRANS = 0 an output row (the loads of a wave are coalesced), TRANS
-// = 1 an output column (each thread reads its column contiguously).
-// Outputs o < k go to the interior cells (w = y when set_interior, else
-// w -= y), o >= k to the contribution buffer tb (e * b + o - k), which
-// k_nd_bsum subtracts from the boundary cells.
-constexpr int kMvNode = 256;
-template <bool TRANS>
-__global__ void __launch_bounds__(256)
-k_nd_mv_node(const cx<float>* __restrict__ F, int m, int row0, int col0, int M, int N,
-             const int32_t* __restrict__ xcells, int xn, const int32_t* __restrict__ icells, int k, int b,
-             cx<float>* __restrict__ w, cx<float>* __restrict__ tb, int set_interior) {
-    __shared__ cx<float> xs[kMvNode];
-    const int e = blockIdx.x, tid = threadIdx.x;
-    const int32_t* xc = xcells + (int64_t)e * xn;
-    for (int q = tid; q < xn; q += blockDim.x) {
-        const int32_t c = xc[q];
-        xs[q] = c >= 0 ? w[c] : czero<float>();
-    }
-    __syncthreads();
-    const int o = tid;
-    const int nout = TRANS ? N : M, nin = TRANS ? M : N;
-    if (o >= nout) return;
-    const cx<float>* A = F + (int64_t)e * m * m + row0 + (int64_t)col0 * m;
-    // element q of output o's row (TRANS = 0) or column (TRANS = 1)
-    const cx<float>* base = TRANS ? A + (int64_t)o * m : A + o;
-    const int64_t step = TRANS ? 1 : m;
-    cx<float> acc = czero<float>();
-    int q = 0;
-    for (; q + 16 <= nin; q += 16) {
-        cx<float> a[16];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) a[u] = base[(int64_t)(q + u) * step];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) acc = acc + a[u] * xs[q + u];
-    }
-    for (; q + 4 <= nin; q += 4) {
-        cx<float> a[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) a[u] = base[(int64_t)(q + u) * step];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) acc = acc + a[u] * xs[q + u];
-    }
-    for (; q < nin; ++q) acc = acc + base[(int64_t)q * step] * xs[q];
-    if (o < k) {
-        const int32_t c = icells[(int64_t)e * k + o];
-        if (c >= 0) w[c] = set_interior ? acc : w[c] - acc;
-    } else {
-        tb[(int64_t)e * b + (o - k)] = acc;
-    }
-}
-
-// The non-transposed product for nodes with at most 32 outputs (the down
-// sweep's x_I = y_I - X x_B on the small levels), one 64-thread workgroup per
-// node: output o = t mod Mp (Mp the power of two >= M) and slice t / Mp of
-// the inputs, so every lane has loads in flight; the slices are summed by
-// lane exchanges.  Outputs as in k_nd_mv_node (o < k: interior cells, else
-// the contribution buffer).
-template <int MP>
-__global__ void __launch_bounds__(64)
-k_nd_mv_node_split(const cx<float>* __restrict__ F, int m, int row0, int col0, int M, int N,
-                   const int32_t* __restrict__ xcells, int xn, const int32_t* __restrict__ icells, int k, int b,
-                   cx<float>* __restrict__ w, cx<float>* __restrict__ tb, int set_interior) {
-    constexpr int S = 64 / MP;
-    __shared__ cx<float> xs[kMvNode];
-    const int e = blockIdx.x, tid = threadIdx.x;
-    const int32_t* xc = xcells + (int64_t)e * xn;
-    for (int q = tid; q < xn; q += 64) {
-        const int32_t c = xc[q];
-        xs[q] = c >= 0 ? w[c] : czero<float>();
-    }
-    __syncthreads();
-    const int o = tid % MP, sl = tid / MP;
-    const cx<float>* A = F + (int64_t)e * m * m + row0 + (int64_t)col0 * m;
-    cx<float> acc = czero<float>();
-    if (o < M) {
-        int q = sl;
-        for (; q + 3 * S < N; q += 4 * S) {
-            cx<float> a[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) a[u] = A[o + (int64_t)(q + u * S) * m];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) acc = acc + a[u] * xs[q + u * S];
-        }
-        for (; q < N; q += S) acc = acc + A[o + (int64_t)q * m] * xs[q];
-    }
-#pragma unroll
-    for (int off = MP; off < 64; off <<= 1) {
+    for (int off = TR; off < 64; off <<= 1) {
         acc.re += __shfl_xor(acc.re, off);
         acc.im += __shfl_xor(acc.im, off);
     }
-    if (sl != 0 || o >= M) return;
-    if (o < k) {
-        const int32_t c = icells[(int64_t)e * k + o];
-        if (c >= 0) w[c] = set_interior ? acc : w[c] - acc;
-    } else {
-        tb[(int64_t)e * b + (o - k)] = acc;
+    if (W > 1) {
+        if ((tid & 63) < TR) red[tid >> 6][r] = acc;
+        __syncthreads();
+        if (tid >= TR) return;
+        acc = red[0][r];
+        for (int q = 1; q < W; ++q) acc = acc + red[q][r];
     }
+    if (tid < TR && o < a.nout) nd_output<UP>(a, e, o, acc);
 }
 
-// Sum of the nt partial-sum tiles of each output o (Mout per node): o < k
-// to the interior cells (w = sum when set_interior, else w -= sum), o >= k
-// to the contribution buffer tb (e * b + o - k).
-__global__ void __launch_bounds__(256)
-k_nd_mv_reduce(const cx<float>* __restrict__ part, int nt, int Mout, int nb, const int32_t* __restrict__ icells,
-               int k, int b, cx<float>* __restrict__ w, cx<float>* __restrict__ tb, int set_interior) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)nb * Mout) return;
-    const int e = (int)(t / Mout), o = (int)(t - (int64_t)e * Mout);
-    cx<float> sum = czero<float>();
-    for (int q = 0; q < nt; ++q) sum = sum + part[((int64_t)e * nt + q) * Mout + o];
-    if (o < k) {
-        const int32_t c = icells[(int64_t)e * k + o];
-        if (c >= 0) w[c] = set_interior ? sum : w[c] - sum;
-    } else {
-        tb[(int64_t)e * b + (o - k)] = sum;
+// sum over the lanes of a group of GS
+template <int GS>
+__device__ __forceinline__ float group_sum(float v) {
+#pragma unroll
+    for (int off = GS / 2; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+    return v;
+}
+
+// y = A^T x: a group of GS lanes per output column (the lanes along the
+// column's rows), C columns per group.
+template <bool UP, int GS, int NT, int C>
+__global__ void __launch_bounds__(NT) k_nd_mvt(NdProduct a, int tiles) {
+    constexpr int G = NT / GS, U = 4, CH = GS < 64 ? GS : kMvChunk;   // groups below a wave hold the whole input
+    __shared__ cx<float> xs[CH + U * GS];
+    const int tid = threadIdx.x, l = tid % GS, grp = tid / GS;
+    const int e = blockIdx.x / tiles, o0 = (blockIdx.x - e * tiles) * (G * C) + grp;
+    const int64_t m = a.m;
+    const cx<float>* A = a.F + e * m * m + a.row0 + a.col0 * m;
+    cx<float> acc[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) acc[c] = czero<float>();
+    for (int q0 = 0; q0 < a.nin; q0 += CH) {
+        const int n = min(CH, a.nin - q0);
+        cx<float> f[C][U];
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int u = 0; u < U; ++u) f[c][u] = A[min(o0 + c * G, a.nout - 1) * m + q0 + min(l + u * GS, n - 1)];
+        if (q0 > 0) __syncthreads();
+        for (int q = tid; q < n + U * GS; q += NT) xs[q] = q < n ? nd_input<UP>(a, e, q0 + q) : czero<float>();
+        __syncthreads();
+        for (int q = l; q < n; q += U * GS) {
+            const bool more = q + U * GS < n;
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+                const cx<float>* Ac = A + min(o0 + c * G, a.nout - 1) * m + q0;
+#pragma unroll
+                for (int u = 0; u < U; ++u) acc[c] = acc[c] + f[c][u] * xs[q + u * GS];
+                if (more)
+#pragma unroll
+                    for (int u = 0; u < U; ++u) f[c][u] = Ac[min(q + (U + u) * GS, n - 1)];
+            }
+        }
     }
-}
-
-// w[cell] -= the sum of its contributions, for each boundary cell of a level
-// (CSR over the level's nodes, fixed order)
-__global__ void __launch_bounds__(256)
-k_nd_bsum(const int32_t* __restrict__ cells, const int32_t* __restrict__ ptr, const int32_t* __restrict__ idx, int n,
-          const cx<float>* __restrict__ tb, cx<float>* __restrict__ w) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    cx<float> sum = czero<float>();
-    for (int q = ptr[t]; q < ptr[t + 1]; ++q) sum = sum + tb[idx[q]];
-    const int32_t c = cells[t];
-    w[c] = w[c] - sum;
-}
-
-__global__ void __launch_bounds__(256) k_nd_copy(const cx<float>* __restrict__ a, cx<float>* __restrict__ b, int64_t n) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) b[t] = a[t];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const cx<float> y = mk(group_sum<GS>(acc[c].re), group_sum<GS>(acc[c].im));
+        const int o = o0 + c * G;
+        if (l == 0 && o < a.nout) nd_output<UP>(a, e, o, y);
+    }
 }
 
 int nblk(int64_t n) { return (int)((n + 255) / 256); }
@@ -1303,80 +1252,103 @@ int get_handle(hipStream_t s, rocblas_handle* out) {
 
 using rc_t = rocblas_float_complex;
 
+// Tile of an A x product: a lane per output row where the level has rows
+// enough for 256 workgroups, else down to 16 rows (128-byte runs), and threads
+// for at most 32 loads each.
+template <bool UP>
+void launch_mv(const NdProduct& a, int nb, hipStream_t s) {
+    int tr = a.nout <= 8 ? 8 : a.nout <= 16 ? 16 : a.nout <= 32 ? 32 : 64;
+    while (tr > 16 && (int64_t)nb * ((a.nout + tr - 1) / tr) < 256) tr >>= 1;
+    const int64_t loads = (int64_t)tr * std::min(a.nin, kMvChunk);
+    const int nt = loads <= 64 * 32 ? 64 : loads <= 256 * 32 ? 256 : 1024;
+    const int tiles = (a.nout + tr - 1) / tr;
+    const unsigned g = (unsigned)(nb * tiles);
+#define CV_MV(TR)                                                         \
+    if (tr == TR) {                                                       \
+        if (nt == 64) k_nd_mv<UP, TR, 64><<<g, 64, 0, s>>>(a, tiles);     \
+        else if (nt == 256) k_nd_mv<UP, TR, 256><<<g, 256, 0, s>>>(a, tiles); \
+        else k_nd_mv<UP, TR, 1024><<<g, 1024, 0, s>>>(a, tiles);          \
+    }
+    CV_MV(8) CV_MV(16) CV_MV(32) CV_MV(64)
+#undef CV_MV
+}
+
+// Tile of an A^T x product: lanes along a column up to a wave, four columns a
+// group while that leaves 512 workgroups, else one.
+template <bool UP>
+void launch_mvt(const NdProduct& a, int nb, hipStream_t s) {
+    const int gs = a.nin <= 8 ? 8 : a.nin <= 16 ? 16 : a.nin <= 32 ? 32 : 64;
+    const int per = 256 / gs;
+    const bool four = (int64_t)nb * ((a.nout + 4 * per - 1) / (4 * per)) >= 512;
+    const int cols = four ? 4 * per : per, tiles = (a.nout + cols - 1) / cols;
+    const unsigned g = (unsigned)(nb * tiles);
+#define CV_MVT(GS)                                                        \
+    if (gs == GS) {                                                       \
+        if (four) k_nd_mvt<UP, GS, 256, 4><<<g, 256, 0, s>>>(a, tiles);   \
+        else k_nd_mvt<UP, GS, 256, 1><<<g, 256, 0, s>>>(a, tiles);        \
+    }
+    CV_MVT(8) CV_MVT(16) CV_MVT(32) CV_MVT(64)
+#undef CV_MVT
+}
+
+__global__ void __launch_bounds__(256)
+k_nd_cells(const int32_t* __restrict__ cells, int n, const cx<float>* __restrict__ w, cx<float>* __restrict__ z) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < n && cells[t] >= 0) z[cells[t]] = w[cells[t]];
+}
+
 }  // namespace
 
 // M^-1 v (transpose 0) or M^-T v (transpose 1) with the nested-dissection
-// factor; v and z complex64 over the grid (may alias).
+// factor; v and z complex64 over the grid (may alias: z is written from the
+// first launch of the down sweep on, when v has been read).
 int nd_apply(const cv_nd_plan* P, const void* plan_dev, const void* factor, const cx<float>* v, cx<float>* z,
              int transpose, hipStream_t s) {
     const char* pb = (const char*)plan_dev;
     char* fb = (char*)factor;
-    const int64_t N = (int64_t)P->nx * P->ny;
-    cx<float>* w = (cx<float>*)(fb + P->off_w);
-    cx<float>* part = (cx<float>*)(fb + P->off_part);
-    cx<float>* tb = (cx<float>*)(fb + P->off_tb);
-    k_nd_copy<<<nblk(N), 256, 0, s>>>(v, w, N);
-    CV_LAUNCH_CHECK();
-    auto tiles = [](int n) { return (n + kMvTile - 1) / kMvTile; };
-    // one product per level and sweep: tiles (launch 1), sum + scatter (launch 2)
-    auto product = [&](const NdLevel& L, bool trans, int row0, int col0, int M, int N, const int32_t* xcells,
-                       int xn, int Mout, int set_interior) -> int {
-        const int32_t* ic = (const int32_t*)(pb + L.off_icells);
-        const cx<float>* F = (const cx<float>*)(fb + L.off_F);
-        if (L.m <= kMvNode) {   // small nodes: one fused launch, one workgroup per node
-            if (!trans && M <= 32) {   // few outputs: the inputs split over the lanes
-                auto* kern = M <= 8 ? k_nd_mv_node_split<8> : M <= 16 ? k_nd_mv_node_split<16>
-                                                                     : k_nd_mv_node_split<32>;
-                kern<<<L.nb, 64, 0, s>>>(F, L.m, row0, col0, M, N, xcells, xn, ic, L.kmax, L.bmax, w, tb,
-                                         set_interior);
-            } else if (!trans)
-                k_nd_mv_node<false><<<L.nb, 64 * ((M + 63) / 64), 0, s>>>(F, L.m, row0, col0, M, N, xcells, xn, ic,
-                                                                         L.kmax, L.bmax, w, tb, set_interior);
-            else
-                k_nd_mv_node<true><<<L.nb, 64 * ((N + 63) / 64), 0, s>>>(F, L.m, row0, col0, M, N, xcells, xn, ic,
-                                                                        L.kmax, L.bmax, w, tb, set_interior);
-            CV_LAUNCH_CHECK();
-            return CV_OK;
-        }
-        const int tm = tiles(M), tn = tiles(N);
-        const int64_t nwg = (int64_t)L.nb * tm * tn;
-        if (!trans)
-            k_nd_mv<false><<<(unsigned)nwg, 256, 0, s>>>(F, L.m, row0, col0, M, N, tm, tn, xcells, xn, w, part);
-        else
-            k_nd_mv<true><<<(unsigned)nwg, 256, 0, s>>>(F, L.m, row0, col0, M, N, tm, tn, xcells, xn, w, part);
-        CV_LAUNCH_CHECK();
-        const int nt = trans ? tm : tn;
-        k_nd_mv_reduce<<<nblk((int64_t)L.nb * Mout), 256, 0, s>>>(part, nt, Mout, L.nb, ic, L.kmax, L.bmax, w, tb,
-                                                                   set_interior);
-        CV_LAUNCH_CHECK();
-        return CV_OK;
-    };
     const int H = (int)P->L.size();
-    for (int l = 0; l < H; ++l) {   // up the tree: [y_I; t] = [Q; G] b_I (or [Q X]^T b_I), b_B -= t
+    NdProduct a;
+    a.v = v;
+    a.T = (cx<float>*)(fb + P->off_t);
+    a.w = (cx<float>*)(fb + P->off_w);
+    auto level = [&](int l) {
         const NdLevel& L = P->L[l];
-        if (L.kmax == 0) continue;
-        const int32_t* ic = (const int32_t*)(pb + L.off_icells);
-        const int rc = !transpose ? product(L, false, 0, 0, L.m, L.kmax, ic, L.kmax, L.m, 1)
-                                  : product(L, true, 0, 0, L.kmax, L.m, ic, L.kmax, L.m, 1);
-        if (rc != CV_OK) return rc;
-        const int nbs = (int)L.bs_cells.size();
-        if (nbs > 0) {   // b_B -= t, the contributions of the level's nodes summed per boundary cell
-            k_nd_bsum<<<nblk(nbs), 256, 0, s>>>((const int32_t*)(pb + L.off_bs_cells),
-                                                (const int32_t*)(pb + L.off_bs_ptr), (const int32_t*)(pb + L.off_bs_idx),
-                                                nbs, tb, w);
+        a.F = (const cx<float>*)(fb + L.off_F);
+        a.m = L.m;
+        a.k = L.kmax;
+        a.b = L.bmax;
+        a.icells = (const int32_t*)(pb + L.off_icells);
+        a.bcells = (const int32_t*)(pb + L.off_bcells);
+        a.up = L.up.empty() ? nullptr : (const int32_t*)(pb + L.off_up);
+        a.t0 = L.t0;
+    };
+    a.z = nullptr;
+    for (int l = 0; l < H; ++l) {   // up the tree: [y_I; t] = [Q; G] b_I (or [Q X]^T b_I)
+        level(l);
+        a.row0 = a.col0 = 0;
+        a.nout = a.m;
+        a.nin = a.k;
+        if (!transpose) launch_mv<true>(a, P->L[l].nb, s);
+        else launch_mvt<true>(a, P->L[l].nb, s);
+        CV_LAUNCH_CHECK();
+    }
+    a.z = z;
+    for (int l = H - 1; l >= 0; --l) {   // down the tree: x_I = y_I - X x_B (or G^T x_B)
+        level(l);
+        const int nb = P->L[l].nb;
+        if (a.b == 0) {   // the root: x = y
+            k_nd_cells<<<nblk((int64_t)nb * a.k), 256, 0, s>>>(a.icells, nb * a.k, a.w, z);
             CV_LAUNCH_CHECK();
+            continue;
         }
+        a.nout = a.k;
+        a.nin = a.b;
+        a.row0 = transpose ? a.k : 0;
+        a.col0 = transpose ? 0 : a.k;
+        if (!transpose) launch_mv<false>(a, nb, s);
+        else launch_mvt<false>(a, nb, s);
+        CV_LAUNCH_CHECK();
     }
-    for (int l = H - 1; l >= 0; --l) {   // down the tree: x_I -= X x_B (or G^T x_B)
-        const NdLevel& L = P->L[l];
-        if (L.kmax == 0 || L.bmax == 0) continue;
-        const int32_t* bc = (const int32_t*)(pb + L.off_bcells);
-        const int rc = !transpose ? product(L, false, 0, L.kmax, L.kmax, L.bmax, bc, L.bmax, L.kmax, 0)
-                                  : product(L, true, L.kmax, 0, L.bmax, L.kmax, bc, L.bmax, L.kmax, 0);
-        if (rc != CV_OK) return rc;
-    }
-    k_nd_copy<<<nblk(N), 256, 0, s>>>(w, z, N);
-    CV_LAUNCH_CHECK();
     return CV_OK;
 }
 
