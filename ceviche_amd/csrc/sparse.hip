@@ -14,8 +14,14 @@
 namespace cv {
 
 // out[o(s)] (+)= alpha * sum_{q in [ptr[s], ptr[s+1])} opu(u[iu[q]]) * opv(v[iv[q]])
-// with o(s) = oidx ? oidx[s] : s and opu / opv optional conjugation.  One
-// thread per segment; the sum runs in storage order (deterministic).
+// with o(s) = oidx ? oidx[s] : s and opu / opv optional conjugation; without
+// ptr (UNIT) segment s is entry s alone.  One thread per segment; the sum
+// runs in storage order (deterministic).  Bound by the latency of index and
+// gather loads that follow each other, so four entries are in flight at a
+// time: 1.3 million entries in 262144 rows, 52 -> 35 us.
+constexpr int kSegBatch = 4;
+
+template <bool UNIT>
 __global__ void __launch_bounds__(256)
 k_segsum(int64_t n_seg, const int64_t* __restrict__ ptr, const int64_t* __restrict__ iu,
          const int64_t* __restrict__ iv, const cx<double>* __restrict__ u, const cx<double>* __restrict__ v,
@@ -24,12 +30,33 @@ k_segsum(int64_t n_seg, const int64_t* __restrict__ ptr, const int64_t* __restri
     const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n_seg) return;
     cx<double> acc = czero<double>();
-    for (int64_t q = ptr[s]; q < ptr[s + 1]; ++q) {
-        cx<double> a = u[iu ? iu[q] : q];
-        cx<double> b = v[iv ? iv[q] : q];
+    auto add = [&](cx<double> a, cx<double> b) {
         if (conj_u) a = conj(a);
         if (conj_v) b = conj(b);
         acc = acc + a * b;
+    };
+    if (UNIT) {
+        add(u[iu ? iu[s] : s], v[iv ? iv[s] : s]);
+    } else {
+        const int64_t end = ptr[s + 1];
+        int64_t q = ptr[s];
+        for (; q + kSegBatch <= end; q += kSegBatch) {
+            int64_t a[kSegBatch], b[kSegBatch];
+            cx<double> x[kSegBatch], y[kSegBatch];
+#pragma unroll
+            for (int e = 0; e < kSegBatch; ++e) {
+                a[e] = iu ? iu[q + e] : q + e;
+                b[e] = iv ? iv[q + e] : q + e;
+            }
+#pragma unroll
+            for (int e = 0; e < kSegBatch; ++e) {
+                x[e] = u[a[e]];
+                y[e] = v[b[e]];
+            }
+#pragma unroll
+            for (int e = 0; e < kSegBatch; ++e) add(x[e], y[e]);
+        }
+        for (; q < end; ++q) add(u[iu ? iu[q] : q], v[iv ? iv[q] : q]);
     }
     const int64_t o = oidx ? oidx[s] : s;
     acc = alpha * acc;
@@ -226,9 +253,12 @@ k_lu_panel_z(int n, cx<double>* __restrict__ A, int k, int w, int32_t* __restric
                 for (int j = 0; j < NB; ++j) s_top[sl][j] = a[q][j];
         }
         __syncthreads();
-        const cx<double> d = s_piv[sl][c];
+        const cx<double> d = s_piv[sl][c];   // uniform
         const bool zero = d.re == 0.0 && d.im == 0.0;
         const cx<double> inv = zero ? czero<double>() : lu_recip(d);
+        // the pivot row, one entry per lane, broadcast through scalar registers
+        // (an LDS read per entry and wave took half of the column's time)
+        const cx<double> mine = s_piv[sl][lane & (NB - 1)];
 #pragma unroll
         for (int q = 0; q < RPT; ++q) {
             const int r = t + q * kLuThreads;
@@ -236,11 +266,19 @@ k_lu_panel_z(int n, cx<double>* __restrict__ A, int k, int w, int32_t* __restric
 #pragma unroll
                 for (int j = 0; j < NB; ++j) a[q][j] = r == c ? s_piv[sl][j] : s_top[sl][j];
             }
-            if (r > c && !zero) {   // a column of zeros stays as it is
-                const cx<double> l = a[q][c] * inv;
-                a[q][c] = l;
+        }
+        if (!zero) {   // a column of zeros stays as it is
+            cx<double> l[RPT];
 #pragma unroll
-                for (int j = c + 1; j < NB; ++j) a[q][j] = a[q][j] - l * s_piv[sl][j];
+            for (int q = 0; q < RPT; ++q) {
+                l[q] = t + q * kLuThreads > c ? a[q][c] * inv : czero<double>();
+                if (t + q * kLuThreads > c) a[q][c] = l[q];
+            }
+#pragma unroll
+            for (int j = c + 1; j < NB; ++j) {
+                const cx<double> u = mk(lu_lane(mine.re, j), lu_lane(mine.im, j));
+#pragma unroll
+                for (int q = 0; q < RPT; ++q) a[q][j] = a[q][j] - l[q] * u;
             }
         }
         }
@@ -306,31 +344,27 @@ k_lu_swap_z(int n, cx<double>* __restrict__ A, int k, int w, const int32_t* __re
     }
 }
 
-// A22 -= L21 U12, 64 x 64 tiles: a lane per row, each wave 16 columns; the
-// rows' multipliers in registers, the columns' U12 broadcast from LDS.
+// A22 -= L21 U12: a lane per row, each of the four waves 16 of a tile's 64
+// columns; the rows' multipliers in registers, a column's U12 through scalar
+// loads (uniform over the wave; as LDS broadcasts they bound the kernel).
 template <int NB>
-__global__ void __launch_bounds__(256) k_lu_trail_z(int n, cx<double>* __restrict__ A, int k) {
-    __shared__ cx<double> s_u[64][NB];
+__global__ void __launch_bounds__(256) k_lu_trail_z(int n, cx<double>* A, int k) {
     const int first = k + NB;
-    const int row = first + blockIdx.x * 64 + (threadIdx.x & 63), col0 = first + blockIdx.y * 64;
-    for (int q = threadIdx.x; q < 64 * NB; q += 256) {
-        const int j = q / NB, c = q % NB;
-        s_u[j][c] = col0 + j < n ? A[(int64_t)(col0 + j) * n + k + c] : czero<double>();
-    }
+    const int row = first + blockIdx.x * 64 + (threadIdx.x & 63);
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col0 = first + blockIdx.y * 64 + 16 * w;
+    const int cols = min(16, n - col0);
     cx<double> l[NB];
 #pragma unroll
     for (int c = 0; c < NB; ++c) l[c] = row < n ? A[(int64_t)(k + c) * n + row] : czero<double>();
-    __syncthreads();
-    if (row >= n) return;
-    const int w = threadIdx.x >> 6;
-    cx<double>* at = A + (int64_t)(col0 + 16 * w) * n + row;
-#pragma unroll 4
-    for (int j = 0; j < 16; ++j) {
-        if (col0 + 16 * w + j >= n) return;
-        cx<double> v = at[(int64_t)j * n];
+    using cu_t = const __attribute__((address_space(4))) double*;
+    for (int j = 0; j < cols; ++j) {
+        const cu_t u = (cu_t)(A + (int64_t)(col0 + j) * n + k);
+        cx<double>* at = A + (int64_t)(col0 + j) * n + row;
+        cx<double> v = row < n ? *at : czero<double>();
 #pragma unroll
-        for (int c = 0; c < NB; ++c) v = v - l[c] * s_u[16 * w + j][c];
-        at[(int64_t)j * n] = v;
+        for (int c = 0; c < NB; ++c) v = v - l[c] * mk(u[2 * c], u[2 * c + 1]);
+        if (row < n) *at = v;
     }
 }
 
@@ -368,6 +402,13 @@ k_lu_tri(int n, const cx<double>* __restrict__ LU, cx<double>* __restrict__ B, i
         }
     };
     cx<double> v = row < n ? b[row] : czero<double>();
+    cx<double> diag[kTri / 4];   // the diagonal block of the workgroup that solves, in flight during the update
+    if (solve)
+#pragma unroll
+        for (int q = 0; q < kTri / 4; ++q) {
+            const int r = mine * kTri + lane, c = mine * kTri + w + 4 * q;
+            diag[q] = r < n && c < n ? LU[(int64_t)c * n + r] : czero<double>();
+        }
     if (update) {
         if (threadIdx.x < kTri) s_y[lane] = blk * kTri + lane < n ? b[blk * kTri + lane] : czero<double>();
         if (kTrans) load(blk, mine);
@@ -392,7 +433,12 @@ k_lu_tri(int n, const cx<double>* __restrict__ LU, cx<double>* __restrict__ B, i
         if (w == 0 && row < n) b[row] = v;
         return;
     }
-    load(mine, mine);   // after the last read of s_t above (barrier in between)
+    // after the last read of s_t above (barrier in between)
+#pragma unroll
+    for (int q = 0; q < kTri / 4; ++q) {
+        if (conjugate) diag[q].im = -diag[q].im;
+        s_t[w + 4 * q][lane] = diag[q];
+    }
     __syncthreads();
     if (w != 0) return;
     cx<double> inv = cone<double>();
@@ -482,14 +528,14 @@ extern "C" int cv_segsum(int64_t n_seg, const int64_t* ptr, const int64_t* iu, c
                          const void* v, int conj_u, int conj_v, double alpha_re, double alpha_im,
                          const int64_t* oidx, int accumulate, void* out, void* stream) {
     CV_CHECK(n_seg >= 0, "n_seg < 0");
-    CV_CHECK(ptr && u && v && out, "null pointer argument");
+    CV_CHECK(u && v && out, "null pointer argument");
     if (n_seg == 0) return CV_OK;
     const int64_t nb = (n_seg + 255) / 256;
     CV_CHECK(nb < (1ll << 31), "too many segments");
-    k_segsum<<<(unsigned)nb, 256, 0, as_stream(stream)>>>(n_seg, ptr, iu, iv, (const cx<double>*)u,
-                                                          (const cx<double>*)v, conj_u, conj_v,
-                                                          mk(alpha_re, alpha_im), oidx, accumulate,
-                                                          (cx<double>*)out);
+    auto* kern = ptr ? k_segsum<false> : k_segsum<true>;
+    kern<<<(unsigned)nb, 256, 0, as_stream(stream)>>>(n_seg, ptr, iu, iv, (const cx<double>*)u, (const cx<double>*)v,
+                                                      conj_u, conj_v, mk(alpha_re, alpha_im), oidx, accumulate,
+                                                      (cx<double>*)out);
     CV_LAUNCH_CHECK();
     return CV_OK;
 }

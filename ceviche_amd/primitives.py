@@ -93,7 +93,6 @@ class Pattern:
         self.by_col = _Groups(cols, N)
         self.cols_by_row = _i64(cols[self.by_row.order_np])
         self.rows_by_col = _i64(rows[self.by_col.order_np])
-        self.unit = _i64(np.arange(self.M + 1))
         key = rows.astype(np.int64) * N + cols
         uniq, inv = np.unique(key, return_inverse=True)
         self.uniq = _Groups(inv.ravel(), uniq.size)
@@ -138,7 +137,7 @@ def _spmv(P, e, x, transpose=False, herm=False):
 def _outer(P, a, b, conj_b=True, alpha=1.0):
     """out[k] = alpha a[row_k] conj?(b[col_k])."""
     out = torch.empty(P.M, dtype=torch.complex128, device=_dev())
-    return segsum(P.M, P.unit, P.rows, P.cols, a, b, out, conj_v=conj_b, alpha=alpha)
+    return segsum(P.M, None, P.rows, P.cols, a, b, out, conj_v=conj_b, alpha=alpha)
 
 
 def _densify(P, e):

@@ -443,7 +443,8 @@ int cv_fdtd_eps_grad(int dtype, const cv_fdtd_desc* d, const void* sig, const vo
 /* ---------------------------------------------------- generic sparse (COO) */
 /* Segmented product sum over complex128 vectors:
  *   out[o(s)] (+)= alpha * sum_{q = ptr[s]}^{ptr[s+1]-1} opu(u[iu[q]]) * opv(v[iv[q]])
- * o(s) = oidx[s] (or s when oidx is NULL), iu / iv NULL mean the identity,
+ * o(s) = oidx[s] (or s when oidx is NULL), iu / iv NULL mean the identity, ptr
+ * NULL segments of one entry (segment s holds entry s),
  * opu / opv conjugate when conj_u / conj_v.  Deterministic (storage order).
  * With host-built groupings of the COO entries this is the CSR SpMV of
  * sp_mult (primitives.py:58-72), its A^T / A^H products and the gather

@@ -205,3 +205,22 @@ def test_dense_lu_reports_the_first_zero_pivot():
     info = torch.zeros(1, dtype=torch.int32, device='cuda')
     check(lib().cv_dense_lu(40, ptr(dev), ptr(piv), ptr(info), stream_ptr()), 'lu')
     assert int(info.item()) == 20
+
+
+@pytest.mark.parametrize('lengths', [[1], [0, 3, 4, 5], [8, 0, 0, 9, 1, 2], [4] * 300, None])
+def test_segsum_batches_and_unit_segments(lengths):
+    """Segments shorter and longer than the batch of entries in flight, empty
+    ones, and (None) the form without a segment pointer; storage-order sums
+    agree to a few roundings."""
+    from ceviche_amd.primitives import segsum
+    g = torch.Generator().manual_seed(5)
+    n_seg = 515 if lengths is None else len(lengths)
+    m = n_seg if lengths is None else sum(lengths)
+    p = torch.arange(n_seg + 1) if lengths is None else torch.tensor([0] + list(np.cumsum(lengths)))
+    u, v = (torch.randn(37, generator=g, dtype=torch.complex128) for _ in range(2))
+    iu, iv = (torch.randint(0, 37, (max(m, 1),), generator=g) for _ in range(2))
+    out = torch.zeros(n_seg, dtype=torch.complex128, device='cuda')
+    segsum(n_seg, None if lengths is None else p.cuda(), iu.cuda(), iv.cuda(), u.cuda(), v.cuda(), out, conj_v=True,
+           alpha=2.0 - 1.0j)
+    want = torch.stack([(2.0 - 1.0j) * (u[iu[p[s]:p[s + 1]]] * v[iv[p[s]:p[s + 1]]].conj()).sum() for s in range(n_seg)])
+    assert float((out.cpu() - want).abs().max()) <= 1e-14 * max(1, max(lengths or [1]))
