@@ -21,20 +21,41 @@
 
 namespace cv {
 
-constexpr int kFgCPT = 4;                    // cells per thread in the vector kernels
-constexpr int kFgCells = kBlock * kFgCPT;    // cells per workgroup
 constexpr int kFgMaxM = 64;                  // longest restart cycle
+constexpr int kFgSumFirst = 4096;            // workgroups above which the norm's partials are summed apart
 
-// Sum of NV values per workgroup into partial[blockIdx.x * NV + c] via
-// wave shuffles and LDS (fixed order).
+// Cells per thread of the vector kernels: one below half a million cells,
+// where four leave most of the GPU idle and put four stencils in a row (28 us
+// against 12 for the stencil with its products at 264 000 cells), else four,
+// which keeps the partial sums few.
+static int fg_cpt(int64_t n) { return n < (int64_t)1 << 19 ? 1 : 4; }
+static int fg_wgs(int64_t n) { return (int)((n + kBlock * fg_cpt(n) - 1) / (kBlock * fg_cpt(n))); }
+
+// Sum over the wave by lane exchanges inside the vector unit (fixed order),
+// valid in every lane; an LDS shuffle takes some 100 cycles a step, which
+// bounded the products with a long basis.
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+    return v + __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    v = dpp_add<0x111>(v);   // row_shr:1, 2, 4, 8: lane 15 of each row of 16 has the row's sum
+    v = dpp_add<0x112>(v);
+    v = dpp_add<0x114>(v);
+    v = dpp_add<0x118>(v);
+    v = dpp_add<0x142>(v);   // row_bcast:15, 31: lane 63 has the wave's sum
+    v = dpp_add<0x143>(v);
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, 63);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), 63);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
 // r = b - A64 x (or A64^T x; row-major single instance), partial[wg] = {|r|^2, |b|^2}
-template <bool TRANS>
+template <bool TRANS, int CPT>
 __global__ void __launch_bounds__(kBlock)
 k_fg_resid(const cv_fdfd_desc* __restrict__ desc, const cx<double>* __restrict__ prof, const double* __restrict__ m0,
            const double* __restrict__ m1, const cx<double>* __restrict__ b, const cx<double>* __restrict__ x,
@@ -47,8 +68,8 @@ k_fg_resid(const cv_fdfd_desc* __restrict__ desc, const cx<double>* __restrict__
     auto fx = [&](int64_t k) { return x[k]; };
     double acc[2] = {0.0, 0.0};
 #pragma unroll
-    for (int q = 0; q < kFgCPT; ++q) {
-        const int64_t k = (int64_t)blockIdx.x * kFgCells + q * kBlock + threadIdx.x;
+    for (int q = 0; q < CPT; ++q) {
+        const int64_t k = (int64_t)blockIdx.x * (kBlock * CPT) + q * kBlock + threadIdx.x;
         if (k >= n) break;
         const int inst = (int)(k / n0);
         const cv_fdfd_desc d = (inst == 0) ? d0 : load_desc(desc, inst);
@@ -89,23 +110,6 @@ k_fg_start(const cx<double>* __restrict__ r, cx<float>* __restrict__ v, double i
     v[k] = mk<float>((float)(a.re * inv), (float)(a.im * inv));
 }
 
-// w = A32 z (or A32^T z)
-template <bool TRANS>
-__global__ void __launch_bounds__(kBlock)
-k_fg_apply(const cv_fdfd_desc* __restrict__ desc, const cx<float>* __restrict__ prof, const float* __restrict__ m0,
-           const float* __restrict__ m1, const cx<float>* __restrict__ z, cx<float>* __restrict__ w) {
-    const cv_fdfd_desc d0 = load_desc(desc, 0);
-    const int64_t n0 = (int64_t)d0.nx * d0.ny;
-    const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (k >= n0 * d0.nblk) return;
-    const int inst = (int)(k / n0);
-    const cv_fdfd_desc d = (inst == 0) ? d0 : load_desc(desc, inst);
-    const int64_t loc = k - (int64_t)inst * n0;
-    const int i = (int)(loc / d.ny), j = (int)(loc - (int64_t)i * d.ny);
-    auto fz = [&](int64_t q) { return z[q]; };
-    w[k] = apply_any<float, TRANS>(d, prof, m0, m1, i, j, fz, z[k]);
-}
-
 // z = v / diag(A32)
 __global__ void __launch_bounds__(kBlock)
 k_fg_jacobi(const cv_fdfd_desc* __restrict__ desc, const cx<float>* __restrict__ prof, const float* __restrict__ m0,
@@ -121,25 +125,26 @@ k_fg_jacobi(const cv_fdfd_desc* __restrict__ desc, const cx<float>* __restrict__
     z[k] = mk<float>((float)q.re, (float)q.im);
 }
 
-// partial[wg][2c .. 2c+1] = sum over the workgroup's cells of conj(V_c) w,
+// One Arnoldi step takes six launches: the new vector and its products with
+// the basis, their sum, the first Gram-Schmidt pass and the products of its
+// result, their sum, the second pass and its norm, the normalisation.  Each
+// launch is near the launch floor on the grids that a factorisation solves
+// (3-5 us at 120^2 and 301 x 219), so a step costs what its launches cost:
+// with products, updates and norm sums apart it took ten (49 us of kernels at
+// 264 000 cells, now 38; a 301 x 219 solve with its gradient 9.7 -> 9.1 ms).
+
+// partial[wg][2c .. 2c+1] = sum over the workgroup's cells (ks) of conj(V_c) w,
 // c < nvec (V_c = V + c * n)
-__global__ void __launch_bounds__(kBlock)
-k_fg_mdot(const cx<float>* __restrict__ V, int nvec, const cx<float>* __restrict__ w, int64_t n,
-          double* __restrict__ partial) {
+template <int CPT>
+__device__ __forceinline__ void fg_dots(const cx<float>* __restrict__ V, int nvec, const cx<double> (&wv)[CPT],
+                                        const int64_t (&ks)[CPT], int64_t n, double* __restrict__ partial) {
     __shared__ double lds[kWaves][2 * kFgMaxM + 2];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    cx<double> wv[kFgCPT];
-    int64_t ks[kFgCPT];
-#pragma unroll
-    for (int q = 0; q < kFgCPT; ++q) {
-        ks[q] = (int64_t)blockIdx.x * kFgCells + q * kBlock + threadIdx.x;
-        wv[q] = ks[q] < n ? ccast<double>(w[ks[q]]) : czero<double>();
-    }
     for (int c = 0; c < nvec; ++c) {
         const cx<float>* vc = V + (int64_t)c * n;
         double sr = 0.0, si = 0.0;
 #pragma unroll
-        for (int q = 0; q < kFgCPT; ++q) {
+        for (int q = 0; q < CPT; ++q) {
             if (ks[q] < n) {
                 const cx<double> a = ccast<double>(vc[ks[q]]);
                 sr += a.re * wv[q].re + a.im * wv[q].im;
@@ -162,28 +167,95 @@ k_fg_mdot(const cx<float>* __restrict__ V, int nvec, const cx<float>* __restrict
     }
 }
 
-// w -= sum_c h_c V_c  (h complex double, on the device)
+// w = A32 z (or A32^T z) and its products with V_0 .. V_{nvec-1}
+template <bool TRANS, int CPT>
 __global__ void __launch_bounds__(kBlock)
-k_fg_maxpy(const cx<float>* __restrict__ V, int nvec, const double* __restrict__ h, cx<float>* __restrict__ w,
-           int64_t n) {
-    const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (k >= n) return;
-    cx<double> acc = ccast<double>(w[k]);
-    for (int c = 0; c < nvec; ++c) {
-        const cx<double> hc = mk(h[2 * c], h[2 * c + 1]);
-        acc = acc - hc * ccast<double>(V[(int64_t)c * n + k]);
+k_fg_apply_dot(const cv_fdfd_desc* __restrict__ desc, const cx<float>* __restrict__ prof, const float* __restrict__ m0,
+               const float* __restrict__ m1, const cx<float>* __restrict__ z, cx<float>* __restrict__ w,
+               const cx<float>* __restrict__ V, int nvec, double* __restrict__ partial) {
+    const cv_fdfd_desc d0 = load_desc(desc, 0);
+    const int64_t n0 = (int64_t)d0.nx * d0.ny, n = n0 * d0.nblk;
+    cx<double> wv[CPT];
+    int64_t ks[CPT];
+    auto fz = [&](int64_t q) { return z[q]; };
+#pragma unroll
+    for (int q = 0; q < CPT; ++q) {
+        const int64_t k = ks[q] = (int64_t)blockIdx.x * (kBlock * CPT) + q * kBlock + threadIdx.x;
+        wv[q] = czero<double>();
+        if (k >= n) continue;
+        const int inst = (int)(k / n0);
+        const cv_fdfd_desc d = (inst == 0) ? d0 : load_desc(desc, inst);
+        const int64_t loc = k - (int64_t)inst * n0;
+        const int i = (int)(loc / d.ny), j = (int)(loc - (int64_t)i * d.ny);
+        const cx<float> v = apply_any<float, TRANS>(d, prof, m0, m1, i, j, fz, z[k]);
+        w[k] = v;
+        wv[q] = ccast<double>(v);
     }
-    w[k] = mk<float>((float)acc.re, (float)acc.im);
+    fg_dots(V, nvec, wv, ks, n, partial);
 }
 
-// v = w / sqrt(nrm2[0])  (in place allowed)
+// w -= sum_c h_c V_c (h complex double, on the device), rounded to complex64;
+// DOTS: then the products of the result with V_0 .. V_{nvec-1}, else
+// partial[wg] = its norm^2 over the workgroup's cells
+template <bool DOTS, int CPT>
 __global__ void __launch_bounds__(kBlock)
-k_fg_normalize(cx<float>* __restrict__ w, const double* __restrict__ nrm2, int64_t n) {
-    const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (k >= n) return;
-    const double s = nrm2[0] > 0.0 ? 1.0 / sqrt(nrm2[0]) : 0.0;
-    const cx<float> a = w[k];
-    w[k] = mk<float>((float)(a.re * s), (float)(a.im * s));
+k_fg_axpy(const cx<float>* __restrict__ V, int nvec, const double* __restrict__ h, cx<float>* __restrict__ w,
+          int64_t n, double* __restrict__ partial) {
+    cx<double> wv[CPT];
+    int64_t ks[CPT];
+#pragma unroll
+    for (int q = 0; q < CPT; ++q) {
+        ks[q] = (int64_t)blockIdx.x * (kBlock * CPT) + q * kBlock + threadIdx.x;
+        wv[q] = ks[q] < n ? ccast<double>(w[ks[q]]) : czero<double>();
+    }
+    for (int c = 0; c < nvec; ++c) {
+        const cx<double> hc = mk(h[2 * c], h[2 * c + 1]);
+        const cx<float>* vc = V + (int64_t)c * n;
+#pragma unroll
+        for (int q = 0; q < CPT; ++q)
+            if (ks[q] < n) wv[q] = wv[q] - hc * ccast<double>(vc[ks[q]]);
+    }
+    double nr[1] = {0.0};
+#pragma unroll
+    for (int q = 0; q < CPT; ++q) {
+        const cx<float> v = mk<float>((float)wv[q].re, (float)wv[q].im);
+        if (ks[q] < n) w[ks[q]] = v;
+        wv[q] = ccast<double>(v);
+        nr[0] += norm2(wv[q]);
+    }
+    if (DOTS) {
+        fg_dots(V, nvec, wv, ks, n, partial);
+    } else {
+        __shared__ double lds[kWaves];
+        block_sum<1>(nr, lds);
+        if (threadIdx.x == 0) partial[blockIdx.x] = nr[0];
+    }
+}
+
+// w /= |w|, |w|^2 the sum of the n_wg partials (every workgroup sums them in
+// the same order; the first one also leaves the sum in nrm2[0])
+template <int CPT>
+__global__ void __launch_bounds__(kBlock)
+k_fg_normalize(cx<float>* __restrict__ w, const double* __restrict__ partial, int n_wg, double* __restrict__ nrm2,
+               int64_t n) {
+    __shared__ double lds[kWaves];
+    __shared__ double total;
+    double v[1] = {0.0};
+    for (int g = threadIdx.x; g < n_wg; g += kBlock) v[0] += partial[g];
+    block_sum<1>(v, lds);
+    if (threadIdx.x == 0) {
+        total = v[0];
+        if (blockIdx.x == 0) nrm2[0] = v[0];
+    }
+    __syncthreads();
+    const double s = total > 0.0 ? 1.0 / sqrt(total) : 0.0;
+#pragma unroll
+    for (int q = 0; q < CPT; ++q) {
+        const int64_t k = (int64_t)blockIdx.x * (kBlock * CPT) + q * kBlock + threadIdx.x;
+        if (k >= n) break;
+        const cx<float> a = w[k];
+        w[k] = mk<float>((float)(a.re * s), (float)(a.im * s));
+    }
 }
 
 // x += sum_c y_c Z_c  (complex128 accumulation)
@@ -215,7 +287,7 @@ static int64_t fg_layout(int64_t n, int m, int64_t net_bytes, char* base, FgWork
         off += al256(bytes);
         return p;
     };
-    const int64_t n_wg = (n + kFgCells - 1) / kFgCells;
+    const int64_t n_wg = fg_wgs(n);
     FgWork t;
     FgWork* o = w ? w : &t;
     o->V = (cx<float>*)take(8 * n * (m + 1));
@@ -262,16 +334,16 @@ static int fgmres_core(const cv_fdfd_desc* desc, const cv_fdfd_desc& dh, const v
                        void* x, double tol, int m, int max_iter, double inner_rtol, FgWork& w, Precond&& precondition,
                        AfterCycle&& after_cycle, cv_solve_info* info, hipStream_t s) {
     const int64_t n = (int64_t)dh.nx * dh.ny * dh.nblk;
-    const int n_wg = (int)((n + kFgCells - 1) / kFgCells);
+    const int n_wg = fg_wgs(n), cpt = fg_cpt(n);
     const int gv = (int)((n + kBlock - 1) / kBlock);
     const cx<double>* b64 = (const cx<double>*)b;
     cx<double>* x64 = (cx<double>*)x;
     double* h1 = w.h;                       // first Gram-Schmidt pass, then the sum
     double* h2 = w.h + 2 * (m + 1);         // second pass
-    double* nrm = w.h + 4 * (m + 1);        // |w|^2 at [0]; |r|^2, |b|^2 at [2], [3]
+    double* nrm = w.h + 4 * (m + 1);        // |w|^2 at [0] ([1]: its sum, if apart); |r|^2, |b|^2 at [2], [3]
     auto true_resid = [&](double* rr, double* bb) -> int {
-        k_fg_resid<TRANS><<<n_wg, kBlock, 0, s>>>(desc, (const cx<double>*)prof64, (const double*)m0_64,
-                                                  (const double*)m1_64, b64, x64, w.r, w.partial);
+        (cpt == 1 ? k_fg_resid<TRANS, 1> : k_fg_resid<TRANS, 4>)<<<n_wg, kBlock, 0, s>>>(
+            desc, (const cx<double>*)prof64, (const double*)m0_64, (const double*)m1_64, b64, x64, w.r, w.partial);
         k_fg_reduce<<<2, kBlock, 0, s>>>(w.partial, n_wg, 2, nrm + 2, 0);
         CV_LAUNCH_CHECK();
         double hv[2];
@@ -305,18 +377,22 @@ static int fgmres_core(const cv_fdfd_desc* desc, const cv_fdfd_desc& dh, const v
             cx<float>* zj = w.Z + (int64_t)j * n;
             cx<float>* wv = w.V + (int64_t)(j + 1) * n;
             if ((rc = precondition(vj, zj)) != CV_OK) return rc;
-            k_fg_apply<TRANS><<<gv, kBlock, 0, s>>>(desc, (const cx<float>*)prof32, (const float*)m0_32,
-                                             (const float*)m1_32, zj, wv);
+            (cpt == 1 ? k_fg_apply_dot<TRANS, 1> : k_fg_apply_dot<TRANS, 4>)<<<n_wg, kBlock, 0, s>>>(
+                desc, (const cx<float>*)prof32, (const float*)m0_32, (const float*)m1_32, zj, wv, w.V, j + 1,
+                w.partial);
             // two passes of classical Gram-Schmidt against V_0 .. V_j
-            k_fg_mdot<<<n_wg, kBlock, 0, s>>>(w.V, j + 1, wv, n, w.partial);
             k_fg_reduce<<<2 * (j + 1), kBlock, 0, s>>>(w.partial, n_wg, 2 * (j + 1), h1, 0);
-            k_fg_maxpy<<<gv, kBlock, 0, s>>>(w.V, j + 1, h1, wv, n);
-            k_fg_mdot<<<n_wg, kBlock, 0, s>>>(w.V, j + 1, wv, n, w.partial);
+            (cpt == 1 ? k_fg_axpy<true, 1> : k_fg_axpy<true, 4>)<<<n_wg, kBlock, 0, s>>>(w.V, j + 1, h1, wv, n,
+                                                                                        w.partial);
             k_fg_reduce<<<2 * (j + 1), kBlock, 0, s>>>(w.partial, n_wg, 2 * (j + 1), h2, 0);
-            k_fg_maxpy<<<gv, kBlock, 0, s>>>(w.V, j + 1, h2, wv, n);
-            k_fg_mdot<<<n_wg, kBlock, 0, s>>>(wv, 1, wv, n, w.partial);
-            k_fg_reduce<<<1, kBlock, 0, s>>>(w.partial, n_wg, 2, nrm, 0);
-            k_fg_normalize<<<gv, kBlock, 0, s>>>(wv, nrm, n);
+            (cpt == 1 ? k_fg_axpy<false, 1> : k_fg_axpy<false, 4>)<<<n_wg, kBlock, 0, s>>>(w.V, j + 1, h2, wv, n,
+                                                                                          w.partial);
+            // each workgroup sums the partials of all: from 4096 workgroups
+            // on that would read more than the vector, so they are summed first
+            const bool sum_first = n_wg > kFgSumFirst;
+            if (sum_first) k_fg_reduce<<<1, kBlock, 0, s>>>(w.partial, n_wg, 1, nrm + 1, 0);
+            (cpt == 1 ? k_fg_normalize<1> : k_fg_normalize<4>)<<<n_wg, kBlock, 0, s>>>(
+                wv, sum_first ? nrm + 1 : w.partial, sum_first ? 1 : n_wg, nrm, n);
             CV_LAUNCH_CHECK();
             CV_HIP(hipMemcpyAsync(hbuf.data(), w.h, sizeof(double) * (4 * (m + 1) + 1), hipMemcpyDeviceToHost, s));
             CV_HIP(hipStreamSynchronize(s));

@@ -195,6 +195,31 @@ def test_fgmres_matches_direct_solve(precond):
     assert np.linalg.norm(got - ref) <= 1e-7 * np.linalg.norm(ref)
 
 
+@pytest.mark.parametrize('N', [48, 724, 725, 2100])
+def test_fgmres_steps_minimise_the_residual_at_every_vector_width(N):
+    """Three Arnoldi steps: the residual must be the least over span{b, Ab,
+    A^2 b}, which a complex128 least-squares problem gives.  One cell per
+    thread up to 724^2 < 2^19 cells, four from 725^2 on; at 2100^2 the norm's
+    partials (more than 4096) are summed by a launch of their own.  The basis
+    is complex64: each of its vectors, orthogonalised twice, is off by a few
+    2^-24 relative to the rest, and so are their images in the residual (norm
+    at most |b|), so 3 * 8 * 2^-24 < 2e-6 bounds the difference."""
+    w, pb, bs = _small_problem(N)
+    x, info = pb.fgmres(bs, tol=1e-14, restart=3, max_iter=3, precond='none')
+    K = [bs / bs.norm()]
+    for _ in range(3):
+        y = pb.op64.apply(K[-1], pb.m0_64, pb.m1_64)
+        K.append(y / y.norm())
+    A = torch.stack(K[1:], 1)
+    Q, _ = torch.linalg.qr(A.cpu())
+    b = (bs / bs.norm()).cpu()
+    least = (b - Q @ (Q.conj().T @ b)).norm().item()
+    true = ((bs - pb.op64.apply(x, pb.m0_64, pb.m1_64)).norm() / bs.norm()).item()
+    print('N', N, 'least', least, 'got', true, 'reported', info['rel_residual'], flush=True)
+    assert info['iterations'] == 3 and abs(true - info['rel_residual']) <= 1e-10
+    assert abs(true - least) <= 2e-6
+
+
 def test_training_step_gradients_and_learned_fgmres():
     """Pairs from plain BiCGSTAB runs, a short training run (loss must fall),
     then FGMRES with the network: it must reach the FP64 tolerance, and the
