@@ -54,6 +54,15 @@ __device__ __forceinline__ float lane_f(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
+// sum over the wave, in every lane
+__device__ __forceinline__ float wave_sum_f(float v) {
+    v += dpp_f<0xB1>(v);     // quad_perm [1,0,3,2]
+    v += dpp_f<0x4E>(v);     // quad_perm [2,3,0,1]
+    v += dpp_f<0x141>(v);    // row_half_mirror
+    v += dpp_f<0x140>(v);    // row_mirror
+    return (lane_f(v, 0) + lane_f(v, 16)) + (lane_f(v, 32) + lane_f(v, 48));
+}
+
 __device__ __forceinline__ cx<float> cdivf(cx<float> a, cx<float> b) {
     const float d = b.re * b.re + b.im * b.im;
     return mk<float>((a.re * b.re + a.im * b.im) / d, (a.im * b.re - a.re * b.im) / d);
@@ -421,6 +430,20 @@ k_btd_apply(const cv_fdfd_desc* __restrict__ desc, const cx<float>* __restrict__
 // D_j^-T (b_j - U_{j-1}^T x_{j-1} - L_{j+1}^T x_{j+1})).  The sequential
 // factorisation's nx dependent inversions become ceil(log2 nx) levels of
 // independent ones; every matrix is an n x n complex64 "slot".
+//
+// The first level below level 0 with at most kBcrTail blocks ends the
+// reduction of a right-hand side: the inverse G of that level's matrix is
+// formed block by block (from X, the inverse of the level below it: G = X on
+// even rows and columns, -delta X - gamma X on odd rows, -X beta - X alpha on
+// odd columns, D^-1 - delta G - gamma G on both) and applied as one dense
+// product.  The levels it replaces have too few blocks to fill the GPU and
+// cost a launch each (6.5 us) both ways: at 120 x 120 an application takes 9
+// launches instead of 15, at 1100 x 80 15 instead of 23, the tail's 6 and 5 us
+// among them.  A solve with its gradient went from 5.3 to 4.5 ms, the coupled
+// 1100 x 80 x 3 solve from 14.3 to 13.2, with the factorisation's products for
+// G (0.1 ms) counted.  More than 8 blocks would cost more products than the
+// launches that they save.
+constexpr int kBcrTail = 8;
 
 // Level 0's L_i and U_i are diagonal (stored dense); ops mark them so the
 // products and solves touch only their diagonals.
@@ -647,7 +670,7 @@ constexpr int kGemmThreads = 256;
 constexpr int kGemmK = 16;
 
 static inline int gemm_tm(int n) { return n > 96 ? 4 : (n > 80 ? 6 : (n > 64 ? 5 : 4)); }
-static inline int gemm_tiles(int n) { const int tile = 16 * gemm_tm(n); return (n + tile - 1) / tile; }
+static inline int gemm_tiles(int n, int tm) { return (n + 16 * tm - 1) / (16 * tm); }
 
 template <int TM>
 __global__ void __launch_bounds__(kGemmThreads)
@@ -761,10 +784,16 @@ k_bcr_gemm(BcrSlots B, const BcrGemmOp* __restrict__ ops, int n, int tiles, int 
 // workgroups per op); otherwise every op is a dense product (one per tile)
 static void launch_gemm(const BcrSlots& S, const BcrGemmOp* ops, int count, int cnt, int n, bool scaling,
                         hipStream_t s) {
-    const int tiles = gemm_tiles(n);
+    // Fewer workgroups than CUs: 32-wide tiles give the launch 4 to 9 times as
+    // many, one K loop's latency shared by more waves (18 us per launch against
+    // 40 at n = 120, 14 against 35 at n = 80).
+    int tm = gemm_tm(n);
+    if (!scaling && (int64_t)gemm_tiles(n, tm) * gemm_tiles(n, tm) * count * cnt < 256) tm = 2;
+    const int tiles = gemm_tiles(n, tm);
     const int per_op = scaling ? 8 : tiles * tiles;
     const dim3 grid(per_op * count, cnt);
-    switch (gemm_tm(n)) {
+    switch (tm) {
+        case 2: k_bcr_gemm<2><<<grid, kGemmThreads, 0, s>>>(S, ops, n, tiles, per_op); break;
         case 5: k_bcr_gemm<5><<<grid, kGemmThreads, 0, s>>>(S, ops, n, tiles, per_op); break;
         case 6: k_bcr_gemm<6><<<grid, kGemmThreads, 0, s>>>(S, ops, n, tiles, per_op); break;
         default: k_bcr_gemm<4><<<grid, kGemmThreads, 0, s>>>(S, ops, n, tiles, per_op); break;
@@ -928,6 +957,97 @@ k_bcr_vec(BcrVecBatch B, const BcrVecOp* __restrict__ ops, int n, int nx) {
     if (t < n) outp[t] = res[t];
 }
 
+// x_i = sum_j G_ij b_j (A^T: sum_j G_ji^T b_j) over the N blocks of the tail
+// level; tab: N x N slots of G, then N indices of b, N of x.  4 to 8 MB of
+// matrix from the cache, every load of a thread in flight at once.
+//   A:   one wave per row, 4 per workgroup, columns over the lanes;
+//   A^T: 16 columns x 64 row groups per workgroup of 1024 threads.
+constexpr int kTailCols = 16;
+
+template <bool TRANS>
+__global__ void __launch_bounds__(TRANS ? 1024 : 256)
+k_bcr_tail(BcrVecBatch B, const int* __restrict__ tab, int N, int n) {
+    __shared__ cx<float> bs[kBcrTail * kBtdMax];
+    const cx<float>* __restrict__ slots = B.slots[blockIdx.y];
+    cx<float>* const work = B.work[blockIdx.y];
+    const int64_t nn = (int64_t)n * n;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int tot = N * n;
+    if (!TRANS) {
+        const int row = blockIdx.x * 4 + wave;
+        const int i = row / n, r = row - i * n;
+        cx<float> e[kBcrTail][2];
+#pragma unroll
+        for (int j = 0; j < kBcrTail; ++j)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int c = lane + 64 * q;
+                e[j][q] = (row < tot && j < N && c < n) ? slots[tab[i * N + j] * nn + (int64_t)r * n + c]
+                                                        : czero<float>();
+            }
+        for (int k = t; k < kBcrTail * kBtdMax; k += 256) {
+            const int j = k / kBtdMax, c = k % kBtdMax;
+            bs[k] = (j < N && c < n) ? work[(int64_t)tab[N * N + j] * n + c] : czero<float>();
+        }
+        __syncthreads();
+        if (row >= tot) return;
+        cx<float> a = czero<float>();
+#pragma unroll
+        for (int j = 0; j < kBcrTail; ++j)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const cx<float> x = bs[j * kBtdMax + 64 * q + lane];
+                a.re = fmaf(e[j][q].re, x.re, fmaf(-e[j][q].im, x.im, a.re));
+                a.im = fmaf(e[j][q].re, x.im, fmaf(e[j][q].im, x.re, a.im));
+            }
+        a.re = wave_sum_f(a.re);
+        a.im = wave_sum_f(a.im);
+        if (lane == 0) work[(int64_t)tab[N * N + N + i] * n + r] = a;
+    } else {
+        __shared__ cx<float> red[16][kTailCols];
+        const int tiles = (n + kTailCols - 1) / kTailCols;
+        const int i = blockIdx.x / tiles, c = (blockIdx.x - i * tiles) * kTailCols + (t & (kTailCols - 1));
+        const int g = t / kTailCols;
+        constexpr int kRows = kBtdMax / 64;    // rows of a block per thread
+        cx<float> e[kBcrTail][kRows];
+#pragma unroll
+        for (int j = 0; j < kBcrTail; ++j)
+#pragma unroll
+            for (int q = 0; q < kRows; ++q) {
+                const int r = g + 64 * q;
+                e[j][q] = (j < N && r < n && c < n) ? slots[tab[j * N + i] * nn + (int64_t)r * n + c]
+                                                    : czero<float>();
+            }
+        for (int k = t; k < kBcrTail * kBtdMax; k += 1024) {
+            const int j = k / kBtdMax, r = k % kBtdMax;
+            bs[k] = (j < N && r < n) ? work[(int64_t)tab[N * N + j] * n + r] : czero<float>();
+        }
+        __syncthreads();
+        cx<float> a = czero<float>();
+#pragma unroll
+        for (int j = 0; j < kBcrTail; ++j)
+#pragma unroll
+            for (int q = 0; q < kRows; ++q) {
+                const cx<float> x = bs[j * kBtdMax + 64 * q + g];
+                a.re = fmaf(e[j][q].re, x.re, fmaf(-e[j][q].im, x.im, a.re));
+                a.im = fmaf(e[j][q].re, x.im, fmaf(e[j][q].im, x.re, a.im));
+            }
+#pragma unroll
+        for (int off = 16; off < 64; off <<= 1) {
+            a.re += __shfl_xor(a.re, off, 64);
+            a.im += __shfl_xor(a.im, off, 64);
+        }
+        if (lane < kTailCols) red[wave][lane] = a;
+        __syncthreads();
+        if (t < kTailCols && c < n) {
+            cx<float> v = czero<float>();
+#pragma unroll
+            for (int q = 0; q < 16; ++q) v = v + red[q][t];
+            work[(int64_t)tab[N * N + N + i] * n + c] = v;
+        }
+    }
+}
+
 }  // namespace cv
 
 using namespace cv;
@@ -1017,10 +1137,13 @@ struct BcrPlan {
     std::vector<std::vector<BcrGemmOp>> g1, g2;   // per level: products, then next-level blocks
     std::vector<std::vector<BcrVecOp>> fwd, bwd;  // per level: RHS reduction, back-substitution
     int final_slot = -1;
-    BcrVecOp final_op{};
+    BcrVecOp final_op{};                          // without a tail
+    int tail_n = 0;                               // blocks of the tail level (0: no tail)
+    std::vector<std::vector<BcrGemmOp>> tg;       // products that form the tail's inverse, in launch order
+    std::vector<int> tail;                        // its slots, right-hand side and solution vectors
     // byte offsets inside the factor buffer
-    int64_t off_dls = 0, off_final = 0, off_slots = 0, off_vecs = 0, bytes = 0;
-    std::vector<int64_t> off_inv, off_g1, off_g2, off_fwd, off_bwd;
+    int64_t off_dls = 0, off_final = 0, off_tail = 0, off_slots = 0, off_vecs = 0, bytes = 0;
+    std::vector<int64_t> off_inv, off_g1, off_g2, off_fwd, off_bwd, off_tg;
 };
 
 static int64_t al256b(int64_t x) { return (x + 255) & ~int64_t(255); }
@@ -1043,8 +1166,22 @@ static void bcr_plan(int nx, int n, BcrPlan& P) {
         P.dls[3 * j + 1] = L[j];
         P.dls[3 * j + 2] = U[j];
     }
+    struct TailLevel {
+        int N;
+        std::vector<int> D, al, be, ga, de;       // al .. de by even block
+    };
+    std::vector<TailLevel> tails;
     int N = nx;
     while (N > 1) {
+        const bool tail = N <= kBcrTail && N < nx;
+        if (tail && P.tail_n == 0) {
+            P.tail_n = N;
+            P.tail.assign((size_t)N * N, -1);
+            P.tail.insert(P.tail.end(), b.begin(), b.end());
+            P.tail.insert(P.tail.end(), x.begin(), x.end());
+        }
+        TailLevel T{N, D, std::vector<int>(N, -1), std::vector<int>(N, -1), std::vector<int>(N, -1),
+                    std::vector<int>(N, -1)};
         std::vector<int> inv, D2, L2, U2, b2, x2;
         std::vector<BcrGemmOp> g1, g2;
         std::vector<BcrVecOp> fw, bw;
@@ -1081,12 +1218,17 @@ static void bcr_plan(int nx, int n, BcrPlan& P) {
                 U2[jj] = ns++;
                 g2.push_back({U2[jj], -1, be, U[j + 1], -1, -1, -1.0f, 0.0f, dg * 2});
             }
+            T.al[j] = al;
+            T.be[j] = be;
+            T.ga[j] = ga;
+            T.de[j] = de;
+            if (tail) continue;
             b2[jj] = nv++;
             x2[jj] = nv++;
             fw.push_back({b2[jj], b[j], (j >= 1) ? b[j - 1] : -1, (j + 1 < N) ? b[j + 1] : -1, al, be, ga, de, -1, 0});
             bw.push_back({x[j], x2[jj], -1, -1, -1, -1, -1, -1, -1, 0});     // even: copy from the next level
         }
-        for (int j = 1; j < N; j += 2) {
+        for (int j = 1; j < N && !tail; j += 2) {
             const bool up = (j + 1 < N);
             bw.push_back({x[j], b[j], x2[(j - 1) / 2], up ? x2[(j + 1) / 2] : -1, L[j], up ? U[j] : -1, U[j - 1],
                           up ? L[j + 1] : -1, D[j], dg * 15});
@@ -1094,8 +1236,12 @@ static void bcr_plan(int nx, int n, BcrPlan& P) {
         P.inv.push_back(inv);
         P.g1.push_back(g1);
         P.g2.push_back(g2);
-        P.fwd.push_back(fw);
-        P.bwd.push_back(bw);
+        if (tail) {
+            tails.push_back(T);
+        } else {
+            P.fwd.push_back(fw);
+            P.bwd.push_back(bw);
+        }
         D = D2;
         L = L2;
         U = U2;
@@ -1104,10 +1250,43 @@ static void bcr_plan(int nx, int n, BcrPlan& P) {
         N = N2;
     }
     P.final_slot = D[0];
-    P.final_op = {x[0], b[0], -1, -1, -1, -1, -1, -1, D[0], 0};
+    if (P.tail_n == 0) P.final_op = {x[0], b[0], -1, -1, -1, -1, -1, -1, D[0], 0};
+    // the tail's inverse, from the last block's up
+    std::vector<int> X(1, D[0]);
+    for (size_t q = tails.size(); q-- > 0;) {
+        const TailLevel& T = tails[q];
+        const int M = T.N, M2 = (M + 1) / 2;
+        std::vector<int> G((size_t)M * M, -1);
+        std::vector<BcrGemmOp> mixed, odd;
+        for (int i = 0; i < M; i += 2)
+            for (int j = 0; j < M; j += 2) G[i * M + j] = X[(i / 2) * M2 + j / 2];
+        for (int i = 1; i < M; i += 2) {
+            const bool up = i + 1 < M;
+            for (int j = 0; j < M; j += 2) {
+                // G_ij = -delta X_(i-1)j - gamma X_(i+1)j, G_ji = -X_j(i-1) beta - X_j(i+1) alpha
+                G[i * M + j] = ns++;
+                mixed.push_back({G[i * M + j], -1, T.de[i - 1], G[(i - 1) * M + j], up ? T.ga[i + 1] : -1,
+                                 up ? G[(i + 1) * M + j] : -1, -1.0f, -1.0f, 0});
+                G[j * M + i] = ns++;
+                mixed.push_back({G[j * M + i], -1, G[j * M + i - 1], T.be[i - 1], up ? G[j * M + i + 1] : -1,
+                                 up ? T.al[i + 1] : -1, -1.0f, -1.0f, 0});
+            }
+        }
+        for (int i = 1; i < M; i += 2)
+            for (int j = 1; j < M; j += 2) {
+                const bool up = i + 1 < M;
+                G[i * M + j] = ns++;
+                odd.push_back({G[i * M + j], i == j ? T.D[i] : -1, T.de[i - 1], G[(i - 1) * M + j],
+                               up ? T.ga[i + 1] : -1, up ? G[(i + 1) * M + j] : -1, -1.0f, -1.0f, 0});
+            }
+        P.tg.push_back(mixed);
+        P.tg.push_back(odd);
+        X = G;
+    }
+    if (P.tail_n) std::copy(X.begin(), X.end(), P.tail.begin());
     P.n_slots = ns;
     P.n_vecs = nv;
-    // layout: header | dls | per level inv, g1, g2, fwd, bwd | final op | slots | vecs
+    // layout: header | dls | per level inv, g1, g2 | per level fwd, bwd | final op | tail products, table | slots | vecs
     int64_t off = 256;
     P.off_dls = off;
     off = al256b(off + 4 * (int64_t)P.dls.size());
@@ -1118,6 +1297,8 @@ static void bcr_plan(int nx, int n, BcrPlan& P) {
         off = al256b(off + (int64_t)sizeof(BcrGemmOp) * P.g1[lv].size());
         P.off_g2.push_back(off);
         off = al256b(off + (int64_t)sizeof(BcrGemmOp) * P.g2[lv].size());
+    }
+    for (size_t lv = 0; lv < P.fwd.size(); ++lv) {
         P.off_fwd.push_back(off);
         off = al256b(off + (int64_t)sizeof(BcrVecOp) * P.fwd[lv].size());
         P.off_bwd.push_back(off);
@@ -1125,6 +1306,12 @@ static void bcr_plan(int nx, int n, BcrPlan& P) {
     }
     P.off_final = off;
     off = al256b(off + sizeof(BcrVecOp) + 4);
+    for (const auto& g : P.tg) {
+        P.off_tg.push_back(off);
+        off = al256b(off + (int64_t)sizeof(BcrGemmOp) * g.size());
+    }
+    P.off_tail = off;
+    off = al256b(off + 4 * (int64_t)P.tail.size());
     P.off_slots = off;
     off = al256b(off + (int64_t)P.n_slots * n * n * 8);
     P.off_vecs = off;
@@ -1171,7 +1358,16 @@ int bcr_apply_batch(const cv_fdfd_desc& dh, int nb, const void* const* factors, 
             }
         };
         for (size_t lv = 0; lv < P.fwd.size(); ++lv) launch(P.off_fwd[lv], (int)P.fwd[lv].size(), kVecReduce);
-        launch(P.off_final, 1, kVecGeneral);
+        if (P.tail_n) {
+            const int* tab = (const int*)(base0 + P.off_tail);
+            if (transpose)
+                k_bcr_tail<true><<<dim3(P.tail_n * ((n + kTailCols - 1) / kTailCols), cnt), 1024, 0, s>>>(
+                    B, tab, P.tail_n, n);
+            else
+                k_bcr_tail<false><<<dim3((P.tail_n * n + 3) / 4, cnt), 256, 0, s>>>(B, tab, P.tail_n, n);
+        } else {
+            launch(P.off_final, 1, kVecGeneral);
+        }
         for (size_t lv = P.bwd.size(); lv-- > 0;)
             launch(P.off_bwd[lv], (int)P.bwd[lv].size(), lv == 0 ? kVecDiag : kVecGeneral);
         CV_LAUNCH_CHECK();
@@ -1229,11 +1425,15 @@ static int bcr_factor_batch(int nb, const cv_fdfd_desc* const* desc, const cv_fd
         put(P.off_inv[lv], P.inv[lv].data(), 4 * P.inv[lv].size());
         put(P.off_g1[lv], P.g1[lv].data(), sizeof(BcrGemmOp) * P.g1[lv].size());
         put(P.off_g2[lv], P.g2[lv].data(), sizeof(BcrGemmOp) * P.g2[lv].size());
+    }
+    for (size_t lv = 0; lv < P.fwd.size(); ++lv) {
         put(P.off_fwd[lv], P.fwd[lv].data(), sizeof(BcrVecOp) * P.fwd[lv].size());
         put(P.off_bwd[lv], P.bwd[lv].data(), sizeof(BcrVecOp) * P.bwd[lv].size());
     }
     put(P.off_final, &P.final_op, sizeof(BcrVecOp));
     put(P.off_final + sizeof(BcrVecOp), &P.final_slot, 4);
+    for (size_t q = 0; q < P.tg.size(); ++q) put(P.off_tg[q], P.tg[q].data(), sizeof(BcrGemmOp) * P.tg[q].size());
+    put(P.off_tail, P.tail.data(), 4 * P.tail.size());
     for (int q = 0; q < nb; ++q) {
         char* base = (char*)factor[q];
         CV_HIP(hipMemcpyAsync(base, host.data(), host.size(), hipMemcpyHostToDevice, s));
@@ -1266,6 +1466,8 @@ static int bcr_factor_batch(int nb, const cv_fdfd_desc* const* desc, const cv_fd
                 launch_gemm(S, (const BcrGemmOp*)(base0 + P.off_g2[lv]), (int)P.g2[lv].size(), cnt, n, lv == 0, s);
         }
         k_bcr_inv<<<dim3(1, cnt), inv_threads, 0, s>>>(S, (const int*)(base0 + P.off_final + sizeof(BcrVecOp)), n);
+        for (size_t q = 0; q < P.tg.size(); ++q)
+            launch_gemm(S, (const BcrGemmOp*)(base0 + P.off_tg[q]), (int)P.tg[q].size(), cnt, n, false, s);
         CV_LAUNCH_CHECK();
     }
     std::vector<int> st(nb, 0);

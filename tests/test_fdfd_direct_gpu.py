@@ -83,6 +83,32 @@ def test_factor_and_sweep_invert_the_block_tridiagonal_part(pol, shape, npml, bl
             np.testing.assert_allclose(S[1], S1, rtol=0, atol=1e-4 * np.abs(S1).max())
 
 
+@pytest.mark.parametrize('nx,ny', [(3, 32), (5, 33), (7, 64), (8, 65), (9, 81), (11, 97), (13, 16), (15, 128),
+                                   (16, 127), (17, 31), (33, 5)])
+def test_cyclic_reduction_tail_of_every_block_count(nx, ny):
+    """Tails of 2 to 8 blocks, block sizes around the 16- and 32-wide tiles: one
+    application against spsolve.  Elimination in complex64 is off by the order
+    of c 2^-24, c the condition number of the system; 100 of that is allowed
+    for the growth over the levels."""
+    from ceviche_amd._fdfd_op import Direct
+    print('tail', nx, ny, flush=True)
+    rng = np.random.default_rng(nx * 131 + ny)
+    eps = rng.uniform(1, 12.25, (nx, ny))
+    npml = (0, min(ny // 4, 8))
+    op = _op('ez', (nx, ny), npml)
+    m0, m1 = op.materials(torch.from_numpy(eps.ravel()))
+    D = Direct(op, m0, m1, kind='bcr')
+    Anw = _without_x_wrap(_scaled_A(op, 'ez', eps, npml, (0.0, 0.0)), nx, ny)
+    c = np.linalg.cond(Anw.toarray())
+    v = rng.standard_normal(nx * ny) + 1j * rng.standard_normal(nx * ny)
+    for tr in (False, True):
+        z = D.apply(torch.from_numpy(v).cuda(), transpose=tr).cpu().numpy()
+        ref = spl.spsolve((Anw.T if tr else Anw).tocsc(), v)
+        err = np.linalg.norm(z - ref) / np.linalg.norm(ref)
+        print('  transpose', tr, 'error %.2e' % err, 'condition %.1e' % c, flush=True)
+        assert err <= 10 * c * 2.0 ** -24
+
+
 @pytest.mark.parametrize('kind', ['btd', 'bcr'])
 @pytest.mark.parametrize('pol,shape,npml,bloch', CASES_BCR)
 def test_direct_solves_match_spsolve(pol, shape, npml, bloch, kind):
