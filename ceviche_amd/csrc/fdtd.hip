@@ -183,6 +183,18 @@ __device__ __forceinline__ void stv(R* p, const Vec<R, V>& x) {
     *reinterpret_cast<Vec<R, V>*>(p) = x;
 }
 
+// Workgroups go round the 8 XCDs in turn: here workgroup b takes block
+// b / 8 of the (b mod 8)-th of eight equal ranges, so that the lines beside
+// and the slices before and after a block's are in the same L2.  The D phase
+// takes 114 us instead of 126 at 256^3 (15.5 instead of 17.6 at 131 x 117 x
+// 142), the adjoint's two phases 23 and 39 us instead of 24 and 40; the H
+// phase, whose D and eps planes of two slices fill an L2 (180 us against
+// 164), keeps the plain order.
+__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t blocks) {
+    const uint32_t per = blocks / 8, rest = blocks - per * 8, x = b & 7;
+    return x * per + min(x, rest) + (b >> 3);
+}
+
 // The cells of this thread: line (i, j), z = k0 .. k0 + V - 1.  Threads past
 // the end repeat the last group (lane shifts need every lane) and store nothing.
 template <typename R, int V>
@@ -191,9 +203,9 @@ struct ZGroup {
     bool live, lo, hi;     // lo / hi: the neighbour below / above is not in the lane beside
     int klo, khi;          // z of the cells below and above the group
 
-    __device__ __forceinline__ explicit ZGroup(const Fdtd<R>& f) : nz(f.nz), ny(f.ny) {
+    __device__ __forceinline__ ZGroup(const Fdtd<R>& f, uint32_t block) : nz(f.nz), ny(f.ny) {
         const int64_t total = f.n / V;
-        int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+        int64_t g = (int64_t)block * blockDim.x + threadIdx.x;
         live = g < total;
         if (!live) g = total - 1;
         if (total <= (int64_t)0xffffffffLL) {
@@ -318,7 +330,7 @@ __device__ __forceinline__ void pml_update(const Fdtd<R>& f, const Pml1<R>& x, c
 // H += curl E (fdtd.py:77-101) with E = D / eps_aa formed from D and eps.
 template <typename R, int V>
 __global__ void __launch_bounds__(256) k_h(Fdtd<R> f, const R* __restrict__ D) {
-    const ZGroup<R, V> g(f);
+    const ZGroup<R, V> g(f, blockIdx.x);
     const int64_t n = f.n;
     const int i = g.i, j = g.j, ip = wrapp(i, f.nx), jp = wrapp(j, f.ny), im = wrapm(i, f.nx), jm = wrapm(j, f.ny);
     const int64_t l = g.line(i, j), c = l + g.k0, l_jp = g.line(i, jp), l_ip = g.line(ip, j);
@@ -447,7 +459,7 @@ struct PointSrc {
 template <typename R, int V>
 __global__ void __launch_bounds__(256) k_d(Fdtd<R> f, const R* Din, R* Dout, const R* __restrict__ Jx,
                                            const R* __restrict__ Jy, const R* __restrict__ Jz, R jscale, PointSrc ps) {
-    const ZGroup<R, V> g(f);
+    const ZGroup<R, V> g(f, xcd_block(blockIdx.x, gridDim.x));
     const int64_t n = f.n;
     const int i = g.i, j = g.j;
     const int64_t l = g.line(i, j), c = l + g.k0, c_im = g.line(wrapm(i, f.nx), j) + g.k0,
@@ -641,7 +653,7 @@ __device__ __forceinline__ void adj_h_update(const Pml1<R>& x, const Pml1<R>& y,
 template <typename R, int V>
 __global__ void __launch_bounds__(256) k_adj_a(Fdtd<R> f, R* __restrict__ lam, R* __restrict__ T, int src_comp,
                                                int64_t src_cell, R* __restrict__ g_src) {
-    const ZGroup<R, V> g(f);
+    const ZGroup<R, V> g(f, xcd_block(blockIdx.x, gridDim.x));
     const int64_t n = f.n;
     const int i = g.i, j = g.j, ip = wrapp(i, f.nx), jp = wrapp(j, f.ny);
     const int64_t l = g.line(i, j), c = l + g.k0, c_jp = g.line(i, jp) + g.k0, c_ip = g.line(ip, j) + g.k0;
@@ -738,7 +750,7 @@ __device__ __forceinline__ void adj_d_update(const Pml1<R>& x, const Pml1<R>& y,
 template <typename R, int V>
 __global__ void __launch_bounds__(256) k_adj_b(Fdtd<R> f, R* __restrict__ lam, const R* __restrict__ T,
                                                const R* __restrict__ Dprev, R* __restrict__ gmE) {
-    const ZGroup<R, V> g(f);
+    const ZGroup<R, V> g(f, xcd_block(blockIdx.x, gridDim.x));
     const int64_t n = f.n;
     const int i = g.i, j = g.j, im = wrapm(i, f.nx), jm = wrapm(j, f.ny);
     const int64_t l = g.line(i, j), c = l + g.k0, c_jm = g.line(i, jm) + g.k0, c_im = g.line(im, j) + g.k0;
