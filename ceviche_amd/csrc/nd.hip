@@ -63,10 +63,12 @@ constexpr int kLuPanel = 16;      // columns per panel of the blocked Gauss-Jord
 constexpr int kLuMin = 64;        // interior blocks above this size take the blocked Gauss-Jordan ...
 constexpr int kLuMaxRows = 2048;  // ... up to this size (the panel kernels hold 1024 threads x 2 rows)
 
-struct NdGroup {               // (parent, child) pairs whose child sits at one level, one child slot
-    int child_level = 0, slot = 0;
-    std::vector<int32_t> parent, child, map;   // map: per pair, the child level's bmax entries
-    int64_t off_parent = 0, off_child = 0, off_map = 0;
+// A child of a node: its ring sums start at index t0 (of those of all levels),
+// its Schur complement at entry S of the factor buffer, mc entries per column.
+struct NdKid {
+    int32_t level = 0, node = 0;   // host only
+    int32_t t0 = 0, mc = 0;
+    int64_t S = 0;
 };
 
 struct NdLevel {
@@ -76,13 +78,13 @@ struct NdLevel {
     // whose couplings this node assembles (-1: outside the grid or eliminated
     // below this node)
     std::vector<int32_t> anbr;
-    std::vector<NdGroup> groups;           // children's Schur complements, extend-added slot by slot
+    std::vector<NdKid> kids;               // two per node (none at the level of the leaves)
     // per node and [I; B] position the entries of its two children's ring sums
     // that fall on it (indices into the sums of all levels, -1: none)
     std::vector<int32_t> up;
     int64_t t0 = 0;                        // first ring sum of the level
     // byte offsets of the device copies (plan buffer) and of the numeric data (factor buffer)
-    int64_t off_icells = 0, off_bcells = 0, off_anbr = 0, off_up = 0;
+    int64_t off_icells = 0, off_bcells = 0, off_anbr = 0, off_up = 0, off_kids = 0;
     int64_t off_F = 0, off_piv = 0, info_first = 0;
 };
 
@@ -251,23 +253,14 @@ extern "C" cv_nd_plan* cv_nd_plan_create(int nx, int ny) {
                     L.anbr[((size_t)e * L.kmax + p) * 4 + d] = nbv[d] >= 0 ? pos[nbv[d]] : -1;
             }
             if (b.c0 >= 0) {
+                if (L.kids.empty()) L.kids.resize((size_t)L.nb * 2);
                 for (int side = 0; side < 2; ++side) {
                     const int cq = side == 0 ? b.c0 : b.c1;
                     const int ch = nodes[cq].height;
                     const NdLevel& CL = P->L[ch];
-                    NdGroup* g = nullptr;
-                    for (auto& gg : L.groups)
-                        if (gg.child_level == ch && gg.slot == side) g = &gg;
-                    if (!g) {
-                        L.groups.push_back(NdGroup());
-                        g = &L.groups.back();
-                        g->child_level = ch;
-                        g->slot = side;
-                    }
-                    g->parent.push_back(e);
-                    g->child.push_back(level_index[cq]);
-                    const size_t base = g->map.size();
-                    g->map.resize(base + CL.bmax, -1);
+                    NdKid& kid = L.kids[(size_t)e * 2 + side];
+                    kid.level = ch;
+                    kid.node = level_index[cq];
                     for (size_t p = 0; p < nodes[cq].B.size(); ++p) {
                         const int32_t ps = pos[nodes[cq].B[p]];
                         if (ps < 0) {   // a child's ring lies on its parent's separator or ring
@@ -275,7 +268,6 @@ extern "C" cv_nd_plan* cv_nd_plan_create(int nx, int ny) {
                             delete P;
                             return nullptr;
                         }
-                        g->map[base + p] = ps;
                         L.up[((size_t)e * L.m + ps) * 2 + side] =
                             (int32_t)(CL.t0 + (int64_t)level_index[cq] * CL.bmax + (int64_t)p);
                     }
@@ -284,10 +276,6 @@ extern "C" cv_nd_plan* cv_nd_plan_create(int nx, int ny) {
             for (int32_t c : b.I) pos[c] = -1;
             for (int32_t c : b.B) pos[c] = -1;
         }
-        // the groups of one child level: slot 0 before slot 1 (extend-add order)
-        std::stable_sort(L.groups.begin(), L.groups.end(), [](const NdGroup& x, const NdGroup& y) {
-            return x.child_level != y.child_level ? x.child_level < y.child_level : x.slot < y.slot;
-        });
     }
     // device layouts: index arrays in the plan buffer, numeric data in the factor buffer
     int64_t po = 0, fo = 0, rmax = 0, r2max = 0, info_first = 0;
@@ -300,13 +288,15 @@ extern "C" cv_nd_plan* cv_nd_plan_create(int nx, int ny) {
         L.off_icells = take(po, 4 * (int64_t)L.icells.size());
         L.off_bcells = take(po, 4 * (int64_t)L.bcells.size());
         L.off_anbr = take(po, 4 * (int64_t)L.anbr.size());
-        for (auto& g : L.groups) {
-            g.off_parent = take(po, 4 * (int64_t)g.parent.size());
-            g.off_child = take(po, 4 * (int64_t)g.child.size());
-            g.off_map = take(po, 4 * (int64_t)g.map.size());
-        }
         L.off_up = take(po, 4 * (int64_t)L.up.size());
+        L.off_kids = take(po, (int64_t)(sizeof(NdKid) * L.kids.size()));
         L.off_F = take(fo, 8 * (int64_t)L.nb * L.m * L.m);
+        for (NdKid& q : L.kids) {
+            const NdLevel& C = P->L[q.level];
+            q.t0 = (int32_t)(C.t0 + (int64_t)q.node * C.bmax);
+            q.mc = C.m;
+            q.S = C.off_F / 8 + (int64_t)q.node * C.m * C.m + (int64_t)C.kmax * C.m + C.kmax;
+        }
         L.off_piv = take(fo, 4 * (int64_t)L.nb * std::max(1, L.kmax));
         L.info_first = info_first;
         info_first += L.nb;
@@ -358,9 +348,9 @@ extern "C" int cv_nd_plan_upload(const cv_nd_plan* p, void* plan_dev, int64_t pl
         if ((rc = up(L.off_icells, L.icells)) || (rc = up(L.off_bcells, L.bcells)) || (rc = up(L.off_anbr, L.anbr)) ||
             (rc = up(L.off_up, L.up)))
             return rc;
-        for (const auto& g : L.groups)
-            if ((rc = up(g.off_parent, g.parent)) || (rc = up(g.off_child, g.child)) || (rc = up(g.off_map, g.map)))
-                return rc;
+        if (!L.kids.empty())
+            CV_HIP(hipMemcpyAsync(base + L.off_kids, L.kids.data(), sizeof(NdKid) * L.kids.size(),
+                                  hipMemcpyHostToDevice, s));
     }
     // the host vectors are read by the copies above: wait for them before returning
     CV_HIP(hipStreamSynchronize(s));
@@ -411,25 +401,41 @@ k_nd_assemble(const cv_fdfd_desc* __restrict__ desc, const cx<float>* __restrict
     }
 }
 
-// children's Schur complements (the bottom-right bc x bc block of their F)
-// added into the parents' F at the mapped positions (one child slot per
-// launch, so every parent entry has one writer); one thread per entry of a
-// child's block, rows fastest (the reads of a wave are contiguous)
+// F of a level above the leaves' = the sum of its two children's Schur
+// complements (the bottom-right blocks of their F) at the positions `up` gives,
+// zero elsewhere.  Every entry of F is formed and written once, rows fastest
+// (runs of a wave's reads are contiguous): clearing F and adding the children
+// one after the other wrote it three times over (25 + 57 + 57 us for a level
+// of 1024^2 cells with 200 MB of fronts, now 65 to 79: 2.2 -> 0.9 ms of a
+// factorisation).  A thread takes
+// four columns of a row, so that it looks up its row and divides once.
+constexpr int kGatherPer = 4;
+
 __global__ void __launch_bounds__(256)
-k_nd_extend(const cx<float>* __restrict__ Fc, int mc, int kc, int bc, int npairs, const int32_t* __restrict__ parent,
-            const int32_t* __restrict__ child, const int32_t* __restrict__ map, cx<float>* __restrict__ F, int m) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t per = (int64_t)bc * bc;
-    if (t >= (int64_t)npairs * per) return;
-    const int pr = (int)(t / per);
-    const int r = (int)(t - (int64_t)pr * per);
-    const int jj = r / bc, ii = r - jj * bc;
-    const int32_t* mp = map + (int64_t)pr * bc;
-    const int pj = mp[jj], pi = mp[ii];
-    if (pj < 0 || pi < 0) return;
-    const cx<float> v = Fc[(int64_t)child[pr] * mc * mc + (int64_t)(kc + jj) * mc + kc + ii];
-    cx<float>* dst = F + (int64_t)parent[pr] * m * m + (int64_t)pj * m + pi;
-    *dst = *dst + v;
+k_nd_gather(const cx<float>* __restrict__ factor, const int2* __restrict__ up, const NdKid* __restrict__ kids,
+            cx<float>* __restrict__ F, int m, int blocks_per_node) {
+    const int e = blockIdx.x / blocks_per_node;
+    const int r = (blockIdx.x - e * blocks_per_node) * 256 + threadIdx.x;
+    const int jg = r / m, i = r - jg * m, j0 = jg * kGatherPer;
+    if (j0 >= m) return;
+    const NdKid a = kids[2 * (int64_t)e], b = kids[2 * (int64_t)e + 1];
+    up += (int64_t)e * m;
+    F += (int64_t)e * m * m + (int64_t)j0 * m + i;
+    const int2 ui = up[i];
+    const cx<float> *Sa = factor + a.S + (ui.x - a.t0), *Sb = factor + b.S + (ui.y - b.t0);
+    int2 uj[kGatherPer];
+#pragma unroll
+    for (int q = 0; q < kGatherPer; ++q) uj[q] = j0 + q < m ? up[j0 + q] : make_int2(-1, -1);
+    cx<float> v[kGatherPer];
+#pragma unroll
+    for (int q = 0; q < kGatherPer; ++q) {
+        const cx<float> x = (ui.x >= 0 && uj[q].x >= 0) ? Sa[(int64_t)(uj[q].x - a.t0) * a.mc] : czero<float>();
+        const cx<float> y = (ui.y >= 0 && uj[q].y >= 0) ? Sb[(int64_t)(uj[q].y - b.t0) * b.mc] : czero<float>();
+        v[q] = x + y;
+    }
+#pragma unroll
+    for (int q = 0; q < kGatherPer; ++q)
+        if (j0 + q < m) F[(int64_t)q * m] = v[q];
 }
 
 // Pivot search keys: one 64-bit word per candidate whose maximum is the
@@ -1383,17 +1389,14 @@ extern "C" int cv_nd_factor(const cv_nd_plan* P, const void* plan_dev, const cv_
         const NdLevel& L = P->L[l];
         rc_t* F = (rc_t*)(fb + L.off_F);
         const rocblas_stride sF = (rocblas_stride)L.m * L.m;
-        CV_HIP(hipMemsetAsync(F, 0, 8 * (size_t)L.nb * L.m * L.m, s));
-        // frontal matrix: the children's Schur complements (extend-add, one
-        // child slot per launch), then the node's own couplings of A
-        for (const auto& g : L.groups) {
-            const NdLevel& C = P->L[g.child_level];
-            if (C.bmax == 0 || g.parent.empty()) continue;
-            const int npairs = (int)g.parent.size();
-            k_nd_extend<<<nblk((int64_t)npairs * C.bmax * C.bmax), 256, 0, s>>>(
-                (const cx<float>*)(fb + C.off_F), C.m, C.kmax, C.bmax, npairs, (const int32_t*)(pb + g.off_parent),
-                (const int32_t*)(pb + g.off_child), (const int32_t*)(pb + g.off_map), (cx<float>*)F, L.m);
-            CV_LAUNCH_CHECK();
+        // frontal matrix: the children's Schur complements, then the node's
+        // own couplings of A
+        if (L.kids.empty()) {
+            CV_HIP(hipMemsetAsync(F, 0, 8 * (size_t)L.nb * L.m * L.m, s));
+        } else {
+            const int per = (int)(((int64_t)L.m * ((L.m + kGatherPer - 1) / kGatherPer) + 255) / 256);
+            k_nd_gather<<<(unsigned)(L.nb * per), 256, 0, s>>>((const cx<float>*)fb, (const int2*)(pb + L.off_up),
+                                                              (const NdKid*)(pb + L.off_kids), (cx<float>*)F, L.m, per);
         }
         if (L.kmax > 0)
             k_nd_assemble<<<nblk((int64_t)L.nb * L.kmax), 256, 0, s>>>(
