@@ -1260,7 +1260,8 @@ using rc_t = rocblas_float_complex;
 
 // Tile of an A x product: a lane per output row where the level has rows
 // enough for 256 workgroups, else down to 16 rows (128-byte runs), and threads
-// for at most 32 loads each.
+// for at most 32 loads each.  With 64 rows everywhere the products of a 1024^2
+// solve take 4.99 ms instead of 4.54, of a 301 x 219 one 1.79 instead of 1.70.
 template <bool UP>
 void launch_mv(const NdProduct& a, int nb, hipStream_t s) {
     int tr = a.nout <= 8 ? 8 : a.nout <= 16 ? 16 : a.nout <= 32 ? 32 : 64;
@@ -1280,7 +1281,10 @@ void launch_mv(const NdProduct& a, int nb, hipStream_t s) {
 }
 
 // Tile of an A^T x product: lanes along a column up to a wave, four columns a
-// group while that leaves 512 workgroups, else one.
+// group (the input's chunk is read once for them) while that leaves 512
+// workgroups, else one.  Four everywhere take 3.07 ms of a 301 x 219 gradient
+// instead of 2.48; one everywhere takes the same there, whose leaves have 2048
+// nodes.
 template <bool UP>
 void launch_mvt(const NdProduct& a, int nb, hipStream_t s) {
     const int gs = a.nin <= 8 ? 8 : a.nin <= 16 ? 16 : a.nin <= 32 ? 32 : 64;
