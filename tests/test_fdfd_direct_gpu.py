@@ -258,6 +258,32 @@ def test_nested_dissection_factor_inverts_the_unwrapped_operator(pol, shape, npm
         assert err <= tol
 
 
+@pytest.mark.parametrize('shape', [(8, 4), (9, 33), (31, 65), (64, 64), (65, 129), (5, 300), (200, 131), (257, 256)])
+def test_nested_dissection_application_at_tile_edges(shape):
+    """One application for A and A^T on grids whose levels cross the product
+    tiles' edges (8 to 64 rows or columns, one and four columns a group, levels
+    of one node to hundreds, from one leaf up).  Backward error: the sweeps of
+    at most 12 levels multiply with blocks of at most 257 columns in complex64,
+    12 * 257 * 2^-24 = 1.8e-4 of |A| |x| at most; a wrong or missing entry gives
+    errors of order one."""
+    from ceviche_amd._fdfd_op import NdDirect
+    print('nd tiles', shape, flush=True)
+    npml = (min(shape[0] // 4, 8), min(shape[1] // 4, 8))
+    op = _op('ez', shape, npml)
+    rng = np.random.default_rng(shape[0] * 1000 + shape[1])
+    eps = rng.uniform(1, 12.25, shape)
+    m0, m1 = op.materials(torch.from_numpy(eps.ravel()))
+    nd = NdDirect(op, m0, m1)
+    An = _nowrap(_scaled_A(op, 'ez', eps, npml, (0.0, 0.0)), *shape)
+    norm = np.sqrt(spl.norm(An, 1) * spl.norm(An, np.inf))
+    v = rng.standard_normal(eps.size) + 1j * rng.standard_normal(eps.size)
+    for tr in (False, True):
+        x = nd.apply(torch.from_numpy(v).cuda(), transpose=tr).cpu().numpy().astype(np.complex128)
+        back = np.linalg.norm(v - (An.T if tr else An) @ x) / (norm * np.linalg.norm(x))
+        print('  transpose', tr, 'backward error %.2e' % back, flush=True)
+        assert back <= 12 * 257 * 2.0 ** -24
+
+
 @pytest.mark.parametrize('pol', ['ez', 'hz'])
 def test_wide_grids_take_the_nested_dissection_path(pol):
     """A grid wider than 128 in both directions: method 'auto' (and
