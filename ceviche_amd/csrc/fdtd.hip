@@ -990,10 +990,16 @@ constexpr unsigned short kTmNoProbe = 0xffff;
 template <int RR, int NT>
 __device__ __forceinline__ bool tm_probe_slots(const TmProbes& pr, int nx, int ny, int i0, int j0,
                                                unsigned short (*s_slot)[RR][64], unsigned short* s_next, int* s_any) {
+    // component, row and column of each probe in the region (kTmNoProbe: none):
+    // the search for probes of one cell reads these, 8 at a time (reading comp
+    // and cell of 240 probes one after the other took 50 us a launch)
+    __shared__ __attribute__((aligned(16))) unsigned short s_key[kTmMaxProbes];
+    static_assert(RR <= 64, "6 bits per row");
     if (pr.n == 0) return false;
     if (threadIdx.x == 0) *s_any = 0;
     __syncthreads();
-    int pi = 0, pj = 0;
+    int pi = 0, pj = 0, kk = 0;
+    unsigned key = kTmNoProbe;
     bool mine = false;
     const int p = threadIdx.x;
     static_assert(NT >= kTmMaxProbes, "one thread per probe");
@@ -1006,25 +1012,33 @@ __device__ __forceinline__ bool tm_probe_slots(const TmProbes& pr, int nx, int n
             pi = (int)(c / ny);
             pj = (int)(c - (int64_t)pi * ny);
         }
-        mine = pmod(pi - i0, nx) < RR && pmod(pj - j0, ny) < 64;
-        if (mine) *s_any = 1;
+        const int r = pmod(pi - i0, nx), col = pmod(pj - j0, ny), k = pr.comp[p];
+        mine = r < RR && col < 64;
+        kk = k == 2 ? 0 : k - 5;
+        if (mine) {
+            *s_any = 1;
+            key = (unsigned)(kk << 12 | r << 6 | col);
+        }
     }
+    if (p < kTmMaxProbes) s_key[p] = (unsigned short)key;
     __syncthreads();
     if (!*s_any) return false;   // uniform
     for (int q = threadIdx.x; q < 3 * RR * 64; q += NT) (&s_slot[0][0][0])[q] = kTmNoProbe;
     __syncthreads();
     if (mine) {
-        const int k = pr.comp[p];
-        const int64_t c = pr.cell[p];
         int before = kTmNoProbe;
         bool head = true;
-        for (int m = 0; m < pr.n; ++m) {
-            if (pr.comp[m] != k || pr.cell[m] != c) continue;
-            if (m < p) before = m;
-            if (m > p) head = false;
+        for (int m = 0; m < pr.n; m += 8) {
+            const uint4 v = *reinterpret_cast<const uint4*>(s_key + m);
+            const unsigned word[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int h = 0; h < 8; ++h) {
+                const bool same = ((word[h / 2] >> (16 * (h & 1))) & 0xffffu) == key;
+                if (same && m + h < p) before = m + h;
+                if (same && m + h > p) head = false;
+            }
         }
         s_next[p] = (unsigned short)before;
-        const int kk = k == 2 ? 0 : k - 5;
         if (head)
             for (int r = pmod(pi - i0, nx); r < RR; r += nx)
                 for (int col = pmod(pj - j0, ny); col < 64; col += ny) s_slot[kk][r][col] = (unsigned short)p;
@@ -1188,6 +1202,15 @@ __global__ void __launch_bounds__(64 * WV) k_tm_block(TmArgs<R> a) {
                 if (__ballot(s_slot[k][w * RPT + q][lane] != kTmNoProbe)) pmask |= 1ull << (q * 3 + k);
             }
     }
+    // Ez probes: each row's last probe, and the rows with a cell of several
+    int last_ez[RPT];
+    unsigned several = 0;
+#pragma unroll
+    for (int q = 0; q < RPT; ++q) {
+        last_ez[q] = probes ? s_slot[0][w * RPT + q][lane] : kTmNoProbe;
+        if (__ballot(last_ez[q] != kTmNoProbe && s_next[last_ez[q] & (kTmMaxProbes - 1)] != kTmNoProbe))
+            several |= 1u << q;
+    }
     const int src_i = a.src_i, src_j = a.src_j;
     bool src_row = false;   // the source's row is one of this wave's
 #pragma unroll
@@ -1262,6 +1285,10 @@ __global__ void __launch_bounds__(64 * WV) k_tm_block(TmArgs<R> a) {
                     for (int k = 0; k < 3; ++k) {
                         if (!(pmask >> (q * 3 + k) & 1)) continue;
                         const R v = k == 0 ? ez[q] : k == 1 ? hx[q] : hy[q];
+                        if (k == 0) {
+                            if (last_ez[q] != kTmNoProbe) row[last_ez[q]] = v;
+                            if (!(several >> q & 1)) continue;
+                        }
                         for (int p = s_slot[k][w * RPT + q][lane]; p != kTmNoProbe; p = s_next[p]) row[p] = v;
                     }
             }
