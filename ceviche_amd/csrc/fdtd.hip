@@ -1025,6 +1025,17 @@ __device__ __forceinline__ bool tm_probe_slots(const TmProbes& pr, int nx, int n
     if (!*s_any) return false;   // uniform
     for (int q = threadIdx.x; q < 3 * RR * 64; q += NT) (&s_slot[0][0][0])[q] = kTmNoProbe;
     __syncthreads();
+    auto enter = [&] {
+        for (int r = pmod(pi - i0, nx); r < RR; r += nx)
+            for (int col = pmod(pj - j0, ny); col < 64; col += ny) s_slot[kk][r][col] = (unsigned short)p;
+    };
+    if (mine) {
+        s_next[p] = kTmNoProbe;
+        enter();
+    }
+    __syncthreads();
+    const bool other = mine && s_slot[kk][pmod(pi - i0, nx)][pmod(pj - j0, ny)] != p;
+    if (!__syncthreads_or(other)) return true;   // one probe per cell: no search
     if (mine) {
         int before = kTmNoProbe;
         bool head = true;
@@ -1039,9 +1050,7 @@ __device__ __forceinline__ bool tm_probe_slots(const TmProbes& pr, int nx, int n
             }
         }
         s_next[p] = (unsigned short)before;
-        if (head)
-            for (int r = pmod(pi - i0, nx); r < RR; r += nx)
-                for (int col = pmod(pj - j0, ny); col < 64; col += ny) s_slot[kk][r][col] = (unsigned short)p;
+        if (head) enter();
     }
     __syncthreads();
     return true;
@@ -1286,8 +1295,12 @@ __global__ void __launch_bounds__(64 * WV) k_tm_block(TmArgs<R> a) {
                         if (!(pmask >> (q * 3 + k) & 1)) continue;
                         const R v = k == 0 ? ez[q] : k == 1 ? hx[q] : hy[q];
                         if (k == 0) {
-                            if (last_ez[q] != kTmNoProbe) row[last_ez[q]] = v;
-                            if (!(several >> q & 1)) continue;
+                            const int last = last_ez[q];
+                            if (last != kTmNoProbe) row[last] = v;
+                            if (several >> q & 1)
+                                for (int p = last != kTmNoProbe ? s_next[last] : last; p != kTmNoProbe; p = s_next[p])
+                                    row[p] = v;
+                            continue;
                         }
                         for (int p = s_slot[k][w * RPT + q][lane]; p != kTmNoProbe; p = s_next[p]) row[p] = v;
                     }
