@@ -22,6 +22,12 @@
 
 namespace cv {
 
+// the constants of coef4 that no cell changes
+template <typename R>
+struct YeeConst {
+    R dt, c0, e0, e2, inv_dt, inv_e0, inv_e2;
+};
+
 template <typename R>
 struct Fdtd {
     int nx, ny, nz;
@@ -33,6 +39,7 @@ struct Fdtd {
     R* st;             // 18 * n
     // interior coefficients (sigma = 0): m1 and m2 for H and D
     R h1, h2, d1, d2;
+    YeeConst<R> yee;
     R cdt, c0dt, half_dt, dL_r;   // c0 dt / dL, c0 dt, dt / (2 eps0), dL
 };
 
@@ -167,8 +174,8 @@ __device__ __forceinline__ double recip(double v) { return 1.0 / v; }
 // Cache).  Neighbours along z are the next element or the next lane; lanes at
 // the end of a line or a wave read that one element from memory.  V divides
 // nz and every base pointer is aligned to it (step_width).  At 256^3 float32
-// with PML on all faces a step takes 164 + 114 us (H, D phase; 198 + 156 with
-// one cell per thread), 40 + 36 B per cell at 4.1 and 5.3 TB/s; the adjoint of
+// with PML on all faces a step takes 173 + 115 us (H, D phase; 198 + 156 with
+// one cell per thread), 40 + 36 B per cell at 3.9 and 5.3 TB/s; the adjoint of
 // a step of 131 x 117 x 142 takes 23 + 39 us (57 + 71).
 template <typename R, int V>
 struct alignas(V * sizeof(R)) Vec {
@@ -189,10 +196,11 @@ __device__ __forceinline__ void stv(R* p, const Vec<R, V>& x) {
 // Workgroups go round the 8 XCDs in turn: here workgroup b takes block
 // b / 8 of the (b mod 8)-th of eight equal ranges, so that the lines beside
 // and the slices before and after a block's are in the same L2.  The D phase
-// takes 114 us instead of 126 at 256^3 (15.5 instead of 17.6 at 131 x 117 x
+// takes 115 us instead of 118 at 256^3 (17.4 instead of 18.9 at 131 x 117 x
 // 142), the adjoint's two phases 23 and 39 us instead of 24 and 40; the H
-// phase, whose D and eps planes of two slices fill an L2 (180 us against
-// 164), keeps the plain order.
+// phase, whose D and eps planes of two slices fill an L2, takes the same in
+// either order (173 and 174 us; 23.1 plain and 22.1 in ranges at 131 x 117 x
+// 142) and keeps the plain one.
 __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t blocks) {
     const uint32_t per = blocks / 8, rest = blocks - per * 8, x = b & 7;
     return x * per + min(x, rest) + (b >> 3);
@@ -257,7 +265,38 @@ __device__ __forceinline__ Vec<R, V> e_vec(const Vec<R, V>& d, const Vec<R, V>& 
     return y;
 }
 
-// PML profile values b = sigma dt / (2 eps0) and r = 1 / (1 + b) of an axis.
+__device__ __forceinline__ float fused(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fused(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// 1 / v, rounded to nearest like the division (float32: two Newton steps on the
+// hardware's estimate round correctly, Markstein 1990; compared with the
+// division for every mantissa), and a / d by rd = 1 / d rounded to nearest.
+// With divisions instead, a step at 256^3 takes 188 + 121 us.
+__device__ __forceinline__ float recip_rn(float v) {
+    float r = __builtin_amdgcn_rcpf(v);
+    r = fused(fused(-v, r, 1.0f), r, r);
+    r = fused(fused(-v, r, 1.0f), r, r);
+    return __builtin_amdgcn_div_fixupf(r, v, 1.0f);
+}
+__device__ __forceinline__ double recip_rn(double v) { return 1.0 / v; }
+template <typename R>
+__device__ __forceinline__ R quot_rn(R a, R d, R rd) {
+#pragma clang fp contract(off)
+    R q = a * rd;
+    q = fused(fused(-d, q, a), rd, q);
+    return fused(fused(-d, q, a), rd, q);
+}
+
+// 1 / eps_aa
+template <typename R, int V>
+__device__ __forceinline__ Vec<R, V> inv_eps(const Vec<R, V>& e, const Vec<R, V>& em) {
+    Vec<R, V> y;
+#pragma unroll
+    for (int q = 0; q < V; ++q) y[q] = recip_rn((e[q] + em[q]) / R(2));
+    return y;
+}
+
+// PML profile values for the adjoint, b = sigma dt / (2 eps0) and r = 1 / (1 + b) of an axis.
 // The coefficients of fdtd.py:272-311 separate into them: for a component
 // with own axis a and the others b, c
 //   m1 = (1 - b_b - b_c - b_b b_c) r_b r_c,  m2 = +-c0 dt r_b r_c,
@@ -297,42 +336,77 @@ __device__ __forceinline__ void pml_axes(const Pml1<R>& x, const Pml1<R>& y, con
     r = (A == 0 ? y.r : x.r) * (A == 2 ? y.r : z.r[q]);
 }
 
-// One component's update in the PML: u = m1 u + m2 dc + m3 ic + m4 iu with the
-// undivided curl difference dc (1 / dL folded into cdt = +-c0 dt / dL).  ic and
-// iu (at this thread's cells) advance where their coefficient is non-zero.
+// One component's step u += curl ch of this thread's cells, with the
+// reference's coefficients formed cell by cell (coef4) where a sigma is
+// non-zero and i1, i2 (those of sigma = 0) elsewhere; sx, sy, sz the sigmas of
+// the axes, sign -1 for H, +1 for D.  ic and iu (at this thread's cells)
+// advance where their coefficient is non-zero.
+// The roundings are written out (no contraction but the fused products named
+// here): a field that a pulse leaves behind is static, its curl cancels and
+// what remains of H is rounding, so that any other order of these operations
+// gives another H in a few cells (up to 2e-11 of its rms in float64 and 9e-3
+// in float32, over runs of 300 steps on grids of 28 to 200 cells a side).
 template <int A, typename R, int V>
-__device__ __forceinline__ void pml_update(const Fdtd<R>& f, const Pml1<R>& x, const Pml1<R>& y, const PmlZ<R, V>& z,
-                                           R cdt, Vec<R, V>& u, const Vec<R, V>& dc, R* ic, R* iu, bool live) {
-    const bool has_ic = A == 0 ? x.b != R(0) : A == 1 ? y.b != R(0) : z.any;
-    const bool has_iu = A == 0 ? y.b != R(0) && z.any : A == 1 ? x.b != R(0) && z.any : x.b != R(0) && y.b != R(0);
-    Vec<R, V> i1, i2;
-    if (has_ic) i1 = ldv<R, V>(ic);
-    if (has_iu) i2 = ldv<R, V>(iu);
+__device__ __forceinline__ void yee_update(const Fdtd<R>& f, R sign, R i1, R i2, R sx, R sy, const Vec<R, V>& sz,
+                                           bool z_any, Vec<R, V>& u, const Vec<R, V>& ch, R* ic, R* iu, bool live) {
+#pragma clang fp contract(off)
+    const bool has_ic = A == 0 ? sx != R(0) : A == 1 ? sy != R(0) : z_any;
+    const bool has_iu = A == 0 ? sy != R(0) && z_any : A == 1 ? sx != R(0) && z_any : sx != R(0) && sy != R(0);
+    const YeeConst<R> k = f.yee;
+    Vec<R, V> c1, c2;
+    if (has_ic) c1 = ldv<R, V>(ic);
+    if (has_iu) c2 = ldv<R, V>(iu);
 #pragma unroll
     for (int q = 0; q < V; ++q) {
-        R ba, bb, bc, r;
-        pml_axes<A>(x, y, z, q, ba, bb, bc, r);
-        const R p = bb * bc;
-        R t = dc[q];
-        if (has_ic && ba != R(0)) {
-            i1[q] += dc[q] * f.inv_dL;
-            t += R(2) * ba * f.dL_r * i1[q];
+        const R sa = A == 0 ? sx : A == 1 ? sy : sz[q], sb = A == 0 ? sy : sx, sc = A == 2 ? sy : sz[q];
+        // coef4, operation by operation
+        const R s1 = quot_rn((sb + sc) / R(2), k.e0, k.inv_e0), s2 = quot_rn(sb * sc * k.dt / R(4), k.e2, k.inv_e2);
+        const R im0 = recip_rn(k.inv_dt + s1 + s2), m2 = sign * im0 * k.c0;
+        const R h = u[q], c = ch[q];
+        R v = fused(im0 * (k.inv_dt - s1 - s2), h, m2 * c);
+        if (has_ic && sa != R(0)) {
+            c1[q] = c1[q] + c;
+            v = fused(quot_rn(m2 * k.dt * sa, k.e0, k.inv_e0), c1[q], v);
         }
-        R v = ((R(1) - bb - bc - p) * r) * u[q] + (cdt * r) * t;
-        if (has_iu && p != R(0)) {
-            i2[q] += u[q];
-            v += (R(-4) * p * r) * i2[q];
+        if (has_iu && sb != R(0) && sc != R(0)) {
+            c2[q] = c2[q] + h;
+            v = fused(-im0 * k.dt * sb * sc / k.e2, c2[q], v);
         }
-        u[q] = v;
+        u[q] = sa == R(0) && sb == R(0) && sc == R(0) ? fused(i2, c, i1 * h) : v;
     }
-    if (live && has_ic) stv(ic, i1);
-    if (live && has_iu) stv(iu, i2);
+    if (live && has_ic) stv(ic, c1);
+    if (live && has_iu) stv(iu, c2);
+}
+
+// the three components
+template <typename R, int V>
+__device__ __forceinline__ void yee_update3(const Fdtd<R>& f, R sign, R i1, R i2, R sx, R sy, const R* sig_z,
+                                            Vec<R, V> (&u)[3], const Vec<R, V> (&ch)[3], R* ic, R* iu, bool live) {
+#pragma clang fp contract(off)
+    Vec<R, V> sz;
+    bool z_any = false;
+#pragma unroll
+    for (int q = 0; q < V; ++q) {
+        sz[q] = sig_z[q];
+        z_any = z_any || sz[q] != R(0);
+    }
+    if (sx != R(0) || sy != R(0) || z_any) {
+        yee_update<0>(f, sign, i1, i2, sx, sy, sz, z_any, u[0], ch[0], ic, iu, live);
+        yee_update<1>(f, sign, i1, i2, sx, sy, sz, z_any, u[1], ch[1], ic + f.n, iu + f.n, live);
+        yee_update<2>(f, sign, i1, i2, sx, sy, sz, z_any, u[2], ch[2], ic + 2 * f.n, iu + 2 * f.n, live);
+    } else {
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int q = 0; q < V; ++q) u[a][q] = fused(i2, ch[a][q], i1 * u[a][q]);
+    }
 }
 
 // ----------------------------------------------------------------- H phase
 // H += curl E (fdtd.py:77-101) with E = D / eps_aa formed from D and eps.
 template <typename R, int V>
 __global__ void __launch_bounds__(256) k_h(Fdtd<R> f, const R* __restrict__ D) {
+#pragma clang fp contract(off)
     const ZGroup<R, V> g(f, blockIdx.x);
     const int64_t n = f.n;
     const int i = g.i, j = g.j, ip = wrapp(i, f.nx), jp = wrapp(j, f.ny), im = wrapm(i, f.nx), jm = wrapm(j, f.ny);
@@ -347,7 +421,7 @@ __global__ void __launch_bounds__(256) k_h(Fdtd<R> f, const R* __restrict__ D) {
                     dx_jp = ldv<R, V>(Dx + l_jp + g.k0), dz_jp = ldv<R, V>(Dz + l_jp + g.k0),
                     dy_ip = ldv<R, V>(Dy + l_ip + g.k0), dz_ip = ldv<R, V>(Dz + l_ip + g.k0);
     Vec<R, V> h[3] = {ldv<R, V>(H), ldv<R, V>(H + n), ldv<R, V>(H + 2 * n)};
-    R e_lo = R(0), e_jplo = R(0), e_iplo = R(0), ex_hi = R(0), ey_hi = R(0);
+    R e_lo = R(0), e_jplo = R(0), e_iplo = R(0), ix_hi = R(0), iy_hi = R(0), dx_hi = R(0), dy_hi = R(0);
     if (g.nz != V) {
         if (g.lo) {
             e_lo = eps[l + g.klo];
@@ -356,36 +430,27 @@ __global__ void __launch_bounds__(256) k_h(Fdtd<R> f, const R* __restrict__ D) {
         }
         if (g.hi) {
             const R eh = eps[l + g.khi];
-            ex_hi = recip((eh + eps[g.line(im, j) + g.khi]) / R(2)) * Dx[l + g.khi];
-            ey_hi = recip((eh + eps[g.line(i, jm) + g.khi]) / R(2)) * Dy[l + g.khi];
+            ix_hi = recip_rn((eh + eps[g.line(im, j) + g.khi]) / R(2));
+            iy_hi = recip_rn((eh + eps[g.line(i, jm) + g.khi]) / R(2));
+            dx_hi = Dx[l + g.khi];
+            dy_hi = Dy[l + g.khi];
         }
     }
-    const Vec<R, V> ex = e_vec(dx, e, e_im), ey = e_vec(dy, e, e_jm), ez = e_vec(dz, e, g.below(e, e_lo));
-    const Vec<R, V> ex_jp = e_vec(dx_jp, e_jp, e_jpim), ez_jp = e_vec(dz_jp, e_jp, g.below(e_jp, e_jplo));
-    const Vec<R, V> ey_ip = e_vec(dy_ip, e_ip, e_ipjm), ez_ip = e_vec(dz_ip, e_ip, g.below(e_ip, e_iplo));
-    const Vec<R, V> ex_kp = g.above(ex, ex_hi), ey_kp = g.above(ey, ey_hi);
-    Vec<R, V> dc[3];   // dL curl_E, ceviche/derivatives.py:16-22 (forward differences, periodic)
+    const Vec<R, V> ix = inv_eps(e, e_im), iy = inv_eps(e, e_jm), iz = inv_eps(e, g.below(e, e_lo));
+    const Vec<R, V> ix_jp = inv_eps(e_jp, e_jpim), iz_jp = inv_eps(e_jp, g.below(e_jp, e_jplo));
+    const Vec<R, V> iy_ip = inv_eps(e_ip, e_ipjm), iz_ip = inv_eps(e_ip, g.below(e_ip, e_iplo));
+    const Vec<R, V> ix_kp = g.above(ix, ix_hi), iy_kp = g.above(iy, iy_hi), dx_kp = g.above(dx, dx_hi),
+                    dy_kp = g.above(dy, dy_hi);
+    Vec<R, V> ce[3];   // curl_E, ceviche/derivatives.py:16-22 (forward differences, periodic)
 #pragma unroll
     for (int q = 0; q < V; ++q) {
-        dc[0][q] = (ez_jp[q] - ez[q]) - (ey_kp[q] - ey[q]);
-        dc[1][q] = (ex_kp[q] - ex[q]) - (ez_ip[q] - ez[q]);
-        dc[2][q] = (ey_ip[q] - ey[q]) - (ex_jp[q] - ex[q]);
+        const R ex = ix[q] * dx[q], ey = iy[q] * dy[q], ez = iz[q] * dz[q];
+        ce[0][q] = (fused(iz_jp[q], dz_jp[q], -ez) - fused(iy_kp[q], dy_kp[q], -ey)) * f.inv_dL;
+        ce[1][q] = (fused(ix_kp[q], dx_kp[q], -ex) - fused(iz_ip[q], dz_ip[q], -ez)) * f.inv_dL;
+        ce[2][q] = (fused(iy_ip[q], dy_ip[q], -ey) - fused(ix_jp[q], dx_jp[q], -ex)) * f.inv_dL;
     }
-    const R sx = sigH(f, 0)[i], sy = sigH(f, 1)[j];
-    PmlZ<R, V> z;
-    z.load(sigH(f, 2) + g.k0, f.half_dt);
-    if (sx != R(0) || sy != R(0) || z.any) {
-        z.recips();
-        const Pml1<R> x(sx, f.half_dt), y(sy, f.half_dt);
-        pml_update<0>(f, x, y, z, -f.cdt, h[0], dc[0], H + 6 * n, H + 9 * n, g.live);
-        pml_update<1>(f, x, y, z, -f.cdt, h[1], dc[1], H + 7 * n, H + 10 * n, g.live);
-        pml_update<2>(f, x, y, z, -f.cdt, h[2], dc[2], H + 8 * n, H + 11 * n, g.live);
-    } else {
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-#pragma unroll
-            for (int q = 0; q < V; ++q) h[a][q] -= f.cdt * dc[a][q];
-    }
+    yee_update3(f, R(-1), f.h1, f.h2, sigH(f, 0)[i], sigH(f, 1)[j], sigH(f, 2) + g.k0, h, ce, H + 6 * n, H + 9 * n,
+                g.live);
     if (!g.live) return;
     stv(H, h[0]);
     stv(H + n, h[1]);
@@ -462,6 +527,7 @@ struct PointSrc {
 template <typename R, int V>
 __global__ void __launch_bounds__(256) k_d(Fdtd<R> f, const R* Din, R* Dout, const R* __restrict__ Jx,
                                            const R* __restrict__ Jy, const R* __restrict__ Jz, R jscale, PointSrc ps) {
+#pragma clang fp contract(off)
     const ZGroup<R, V> g(f, xcd_block(blockIdx.x, gridDim.x));
     const int64_t n = f.n;
     const int i = g.i, j = g.j;
@@ -478,29 +544,16 @@ __global__ void __launch_bounds__(256) k_d(Fdtd<R> f, const R* Din, R* Dout, con
         hy_lo = Hy[l + g.klo];
     }
     const Vec<R, V> hx_km = g.below(hx, hx_lo), hy_km = g.below(hy, hy_lo);
-    Vec<R, V> dc[3];   // dL curl_H, ceviche/derivatives.py:24-30 (backward differences, periodic)
+    Vec<R, V> ch[3];   // curl_H, ceviche/derivatives.py:24-30 (backward differences, periodic)
 #pragma unroll
     for (int q = 0; q < V; ++q) {
-        dc[0][q] = (hz[q] - hz_jm[q]) - (hy[q] - hy_km[q]);
-        dc[1][q] = (hx[q] - hx_km[q]) - (hz[q] - hz_im[q]);
-        dc[2][q] = (hy[q] - hy_im[q]) - (hx[q] - hx_jm[q]);
+        ch[0][q] = ((hz[q] - hz_jm[q]) - (hy[q] - hy_km[q])) * f.inv_dL;
+        ch[1][q] = ((hx[q] - hx_km[q]) - (hz[q] - hz_im[q])) * f.inv_dL;
+        ch[2][q] = ((hy[q] - hy_im[q]) - (hx[q] - hx_jm[q])) * f.inv_dL;
     }
-    const R sx = sigD(f, 0)[i], sy = sigD(f, 1)[j];
-    PmlZ<R, V> z;
-    z.load(sigD(f, 2) + g.k0, f.half_dt);
-    if (sx != R(0) || sy != R(0) || z.any) {
-        z.recips();
-        const Pml1<R> x(sx, f.half_dt), y(sy, f.half_dt);
-        R* aux = f.st + c;
-        pml_update<0>(f, x, y, z, f.cdt, d[0], dc[0], aux + 12 * n, aux + 15 * n, g.live);
-        pml_update<1>(f, x, y, z, f.cdt, d[1], dc[1], aux + 13 * n, aux + 16 * n, g.live);
-        pml_update<2>(f, x, y, z, f.cdt, d[2], dc[2], aux + 14 * n, aux + 17 * n, g.live);
-    } else {
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-#pragma unroll
-            for (int q = 0; q < V; ++q) d[a][q] += f.cdt * dc[a][q];
-    }
+    R* aux = f.st + c;
+    yee_update3(f, R(1), f.d1, f.d2, sigD(f, 0)[i], sigD(f, 1)[j], sigD(f, 2) + g.k0, d, ch, aux + 12 * n,
+                aux + 15 * n, g.live);
     if (!g.live) return;
     const R* J[3] = {Jx, Jy, Jz};
     const int64_t at = ps.cell - c;
@@ -508,7 +561,7 @@ __global__ void __launch_bounds__(256) k_d(Fdtd<R> f, const R* Din, R* Dout, con
     for (int a = 0; a < 3; ++a) {
         if (J[a])
 #pragma unroll
-            for (int q = 0; q < V; ++q) d[a][q] += jscale * J[a][c + q];
+            for (int q = 0; q < V; ++q) d[a][q] = fused(jscale, J[a][c + q], d[a][q]);
         if (ps.comp == a && at >= 0 && at < V) {
             const R amp = R(ps.amp_dev ? *ps.amp_dev : ps.amp);
 #pragma unroll
@@ -2522,6 +2575,14 @@ static int make_fdtd(const cv_fdtd_desc* d, const void* sig, const void* eps, vo
     f.c0dt = R(d->c0 * d->dt);
     f.half_dt = R(d->dt / (2.0 * d->eps0));
     f.dL_r = R(d->dL);
+    YeeConst<R>& y = f.yee;
+    y.dt = R(d->dt);
+    y.c0 = R(d->c0);
+    y.e0 = R(d->eps0);
+    y.e2 = y.e0 * y.e0;
+    y.inv_dt = R(1) / y.dt;
+    y.inv_e0 = R(1) / y.e0;
+    y.inv_e2 = R(1) / y.e2;
     f.sig = (const R*)sig;
     f.eps = (const R*)eps;
     f.st = (R*)state;

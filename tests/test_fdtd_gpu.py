@@ -549,3 +549,85 @@ def test_step_kernels_of_every_width_match_oracle(shape, npml, precision, tol):
         scale = float(np.abs(wt * trc.imag).sum() / h)
         got = float((ge.detach().cpu().double().numpy() * d).sum() + (ga.numpy() * da).sum())
         assert abs(got - want) <= 20 * tol * scale, (got, want)
+
+
+def _fused(dtype):
+    """a * b + c with one rounding, elementwise (the C library's fma / fmaf)."""
+    import ctypes
+    import ctypes.util
+    libm = ctypes.CDLL(ctypes.util.find_library('m') or 'libm.so.6')
+    fn, ct = (libm.fmaf, ctypes.c_float) if dtype == np.float32 else (libm.fma, ctypes.c_double)
+    fn.restype, fn.argtypes = ct, [ct] * 3
+    each = np.frompyfunc(lambda a, b, c: fn(a, b, c), 3, 1)
+    return lambda a, b, c: each(a, b, c).astype(dtype)
+
+
+def _rounded_steps(eps, dL, dt, sig, src, amp, dtype):
+    """Yee steps in ``dtype`` with the roundings the framework promises: the
+    reference's coefficients (fdtd.py:272-311) operation by operation, a
+    neighbour's E product fused into the difference, m1 u fused onto m2 curl in
+    the PML and m2 curl onto m1 u elsewhere.  Returns (D, H)."""
+    from ceviche_amd.constants import C_0, EPSILON_0
+    R, fma = dtype, _fused(dtype)
+    shape = eps.shape
+    eps = eps.astype(dtype)
+    dt, c0, e0, inv_dL = R(dt), R(C_0), R(EPSILON_0), R(1.0 / dL)
+    inv = [R(1) / ((eps + np.roll(eps, 1, a)) / R(2)) for a in range(3)]
+    axis = np.split(sig.astype(dtype), np.cumsum(list(shape) * 2)[:-1])
+    full = lambda k, a: np.broadcast_to(axis[3 * k + a].reshape([-1 if b == a else 1 for b in range(3)]), shape)
+    H, D = ([np.zeros(shape, dtype) for _ in range(3)] for _ in range(2))
+    integrals = [[np.zeros(shape, dtype) for _ in range(6)] for _ in range(2)]
+
+    def update(k, sign, a, u, curl):
+        sa = full(k, a)
+        sb, sc = (full(k, b) for b in range(3) if b != a)
+        s1, s2 = (sb + sc) / R(2) / e0, sb * sc * dt / R(4) / (e0 * e0)
+        m0 = R(1) / dt + s1 + s2
+        m1, m2 = R(1) / m0 * (R(1) / dt - s1 - s2), R(sign) / m0 * c0
+        m3, m4 = m2 * dt * sa / e0, R(-1) / m0 * dt * sb * sc / (e0 * e0)
+        ic, iu = integrals[k][a], integrals[k][3 + a]
+        v = fma(m1, u, m2 * curl)
+        ic[sa != 0] += curl[sa != 0]
+        v = np.where(sa != 0, fma(m3, ic, v), v)
+        both = (sb != 0) & (sc != 0)
+        iu[both] += u[both]
+        v = np.where(both, fma(m4, iu, v), v)
+        return np.where((sa == 0) & (sb == 0) & (sc == 0), fma(m2, curl, m1 * u), v)
+
+    for t in range(len(amp)):
+        E = [inv[a] * D[a] for a in range(3)]
+        ahead = lambda a, b: fma(np.roll(inv[a], -1, b), np.roll(D[a], -1, b), -E[a])     # E_a one cell up b, less E_a
+        curl = [(ahead(2, 1) - ahead(1, 2)) * inv_dL, (ahead(0, 2) - ahead(2, 0)) * inv_dL,
+                (ahead(1, 0) - ahead(0, 1)) * inv_dL]
+        H = [update(0, -1, a, H[a], curl[a]) for a in range(3)]
+        behind = lambda a, b: H[a] - np.roll(H[a], 1, b)
+        curl = [(behind(2, 1) - behind(1, 2)) * inv_dL, (behind(0, 2) - behind(2, 0)) * inv_dL,
+                (behind(1, 0) - behind(0, 1)) * inv_dL]
+        D = [update(1, 1, a, D[a], curl[a]) for a in range(3)]
+        D[2][src] += R(amp[t])
+    return D, H
+
+
+@pytest.mark.parametrize('precision', ['float32', 'float64'])
+@pytest.mark.parametrize('shape,npml', [((6, 5, 8), [1, 1, 2]), ((4, 7, 66), [2, 0, 4]), ((5, 6, 37), [1, 2, 3]),
+                                        ((3, 5, 4), [0, 1, 1]), ((3, 2, 264), [0, 0, 9])])
+def test_step_kernels_keep_their_roundings(shape, npml, precision):
+    """The fields of the per-step kernels bit for bit, for every width a thread
+    can have along z, groups that a PML edge divides, single-group lines and
+    lines longer than a wave.  Fields that a pulse leaves behind are static and
+    H is what rounding leaves of their curl, so kernels that round in another
+    order differ by far more than roundings there: nothing but equality holds
+    over long runs."""
+    import ceviche_amd as cv
+    print('roundings', shape, npml, precision, flush=True)
+    dtype = np.float32 if precision == 'float32' else np.float64
+    rng = np.random.default_rng(sum(shape))
+    eps = rng.uniform(1, 12.25, shape).astype(dtype)
+    amp = rng.standard_normal(12)
+    src = tuple(n // 2 for n in shape)
+    F = cv.fdtd(eps, 25e-9, npml, precision=precision)
+    F.run(len(amp), src, amp, [('Ez', src)], kernel='generic')
+    D, H = _rounded_steps(eps, 25e-9, F.dt, F._grid.sig_host, src, amp, dtype)
+    got = F.fields
+    for a, c in enumerate('xyz'):
+        assert np.array_equal(got['D' + c], D[a]) and np.array_equal(got['H' + c], H[a]), c
