@@ -360,12 +360,16 @@ class FdtdRun(torch.autograd.Function):
         # The amplitude series is read by the temporally blocked and fused
         # kernels and by the reverse sweep from device memory (a float64
         # device tensor is used as it is, anything else is uploaded once) and
-        # by the per-step kernels from host memory (copied once, only for those).
+        # by the per-step kernels from host memory (copied once, only for
+        # those).  The reverse sweep replays the steps: it keeps amplitudes of
+        # its own, which the caller cannot write between forward and backward.
         a = amp.detach()
         amp_dev = amp_h = None
         need_grad = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
         if tm_config != 'generic' or need_grad:
             amp_dev = a.to(grid.device, torch.float64).contiguous().reshape(-1)
+            if need_grad and amp_dev.data_ptr() == a.data_ptr():
+                amp_dev = amp_dev.clone()
         if tm_config in ('generic', 'fused'):
             amp_h = a.to('cpu', torch.float64).numpy()
         state = state0.detach().clone()

@@ -631,3 +631,27 @@ def test_step_kernels_keep_their_roundings(shape, npml, precision):
     got = F.fields
     for a, c in enumerate('xyz'):
         assert np.array_equal(got['D' + c], D[a]) and np.array_equal(got['H' + c], H[a]), c
+
+
+@pytest.mark.parametrize('shape,kernel', [((24, 20, 1), 'auto'), ((24, 20, 1), 'generic'), ((24, 20, 1), 'fused'),
+                                          ((8, 7, 6), 'generic'), ((8, 7, 6), 'fused')])
+def test_amplitudes_written_after_the_run_do_not_change_its_gradient(shape, kernel):
+    """The reverse sweep replays the steps; a float64 device tensor of
+    amplitudes that the caller refills before backward() must not reach it."""
+    import ceviche_amd as cv
+    rng = np.random.default_rng(4)
+    eps0, amp0 = rng.uniform(1, 6, shape), rng.standard_normal(30)
+    src = tuple(n // 2 for n in shape)
+    grads = []
+    for refill in (False, True):
+        eps = torch.tensor(eps0, device='cuda', requires_grad=True)
+        amp = torch.tensor(amp0, device='cuda', requires_grad=True)
+        F = cv.fdtd(eps, 25e-9, [2, 2, 2 if shape[2] > 1 else 0])
+        loss = (F.run(len(amp0), src, amp, [('Ez', src), ('Hx', (1, 1, 0))], checkpoint_every=7, kernel=kernel) ** 2).sum()
+        if refill:
+            with torch.no_grad():
+                amp.mul_(-3.0)
+        loss.backward()
+        grads.append((eps.grad, amp.grad))
+    for x, y in zip(*grads):
+        assert torch.equal(x, y)
