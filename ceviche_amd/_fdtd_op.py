@@ -365,7 +365,7 @@ class FdtdRun(torch.autograd.Function):
         # its own, which the caller cannot write between forward and backward.
         a = amp.detach()
         amp_dev = amp_h = None
-        need_grad = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
+        need_grad = ctx.needs_input_grad[0] or ctx.needs_input_grad[1] or ctx.needs_input_grad[3]
         if tm_config != 'generic' or need_grad:
             amp_dev = a.to(grid.device, torch.float64).contiguous().reshape(-1)
             if need_grad and amp_dev.data_ptr() == a.data_ptr():

@@ -655,3 +655,35 @@ def test_amplitudes_written_after_the_run_do_not_change_its_gradient(shape, kern
         grads.append((eps.grad, amp.grad))
     for x, y in zip(*grads):
         assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize('final', [False, True])
+@pytest.mark.parametrize('shape,kernel', [((40, 30, 1), 'auto'), ((40, 30, 1), 8), ((40, 30, 1), 'generic'),
+                                          ((40, 30, 1), 'fused'), ((9, 8, 7), 'generic'), ((9, 8, 7), 'fused')])
+def test_gradient_passes_through_a_run_that_only_continues(shape, kernel, final):
+    """The second of two runs has plain amplitudes and a plain eps: its start
+    state alone carries the gradient of the first one's amplitudes.  Against
+    one run over all steps, which forms the same sums of O(steps) terms: 40
+    roundings a step."""
+    import ceviche_amd as cv
+    print('continued run', shape, kernel, final, flush=True)
+    rng = np.random.default_rng(6)
+    eps, amp0 = torch.from_numpy(rng.uniform(1, 6, shape)).cuda(), rng.standard_normal(45)
+    src, n1 = tuple(n // 2 for n in shape), 19
+    probes = [('Ez', (shape[0] // 2 + 2, shape[1] // 2, shape[2] // 2)), ('Hx', src)]
+    npml = [3, 3, 2 if shape[2] > 1 else 0]
+
+    def loss(F, rec):
+        out = (rec[-(len(amp0) - n1):] ** 2).sum()
+        return out + (F.fields['Ez'] ** 2).sum() + (F.fields['Hy'] ** 3).sum() if final else out
+
+    one = torch.tensor(amp0, requires_grad=True)
+    F = cv.fdtd(eps, 25e-9, npml)
+    loss(F, F.run(len(amp0), src, one, probes, checkpoint_every=8, kernel=kernel)).backward()
+    first = torch.tensor(amp0[:n1], requires_grad=True)
+    F = cv.fdtd(eps, 25e-9, npml)
+    F.run(n1, src, first, probes, checkpoint_every=8, kernel=kernel)
+    loss(F, F.run(len(amp0) - n1, src, amp0[n1:], probes, checkpoint_every=8, kernel=kernel)).backward()
+    want = one.grad[:n1]
+    assert float(want.norm()) > 0
+    assert float((first.grad - want).norm()) <= 40 * len(amp0) * 2.0 ** -52 * float(one.grad.norm())
