@@ -385,12 +385,12 @@ k_lu_tri(int n, const cx<double>* __restrict__ LU, cx<double>* __restrict__ B, i
     __shared__ cx<double> s_t[kTri][kTri + 1];   // [column][row] of a block (as stored), padded against conflicts
     __shared__ cx<double> s_part[4][kTri];
     __shared__ cx<double> s_y[kTri];
-    cx<double>* b = B + (int64_t)blockIdx.y * n;
+    cx<double>* b = B + (int64_t)blockIdx.x * n;   // right-hand sides along x, which has room for any number
     const int nblk = (n + kTri - 1) / kTri;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int next = kForward ? blk + 1 : blk - 1;
-    const int mine = kForward ? next + (int)blockIdx.x : next - (int)blockIdx.x;   // in range by the grid
-    const bool solve = blockIdx.x == 0;
+    const int mine = kForward ? next + (int)blockIdx.y : next - (int)blockIdx.y;   // in range by the grid
+    const bool solve = blockIdx.y == 0;
     const bool update = blk >= 0 && blk < nblk;
     const int row = mine * kTri + lane;   // the unknown of this lane
     // block (br, bc) of LU as s_t[column][row]
@@ -593,7 +593,7 @@ extern "C" int cv_dense_lu_solve(int n, const void* LU, const int32_t* piv, void
         else k_lu_permute_seq<<<nrhs, 1, 0, s>>>(n, piv, b, forward);
     };
     // the first launch of a sweep only solves its own block
-    auto groups = [&](int left, bool first) { return dim3(first ? 1 : left, nrhs); };
+    auto groups = [&](int left, bool first) { return dim3(nrhs, first ? 1 : left); };
     if (trans == 0) {
         permute(1);
         for (int q = -1; q < nblk - 1; ++q) k_lu_tri<0><<<groups(nblk - 1 - q, q < 0), 256, 0, s>>>(n, Z, b, q, 0);

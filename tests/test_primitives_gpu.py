@@ -224,3 +224,22 @@ def test_segsum_batches_and_unit_segments(lengths):
            alpha=2.0 - 1.0j)
     want = torch.stack([(2.0 - 1.0j) * (u[iu[p[s]:p[s + 1]]] * v[iv[p[s]:p[s + 1]]].conj()).sum() for s in range(n_seg)])
     assert float((out.cpu() - want).abs().max()) <= 1e-14 * max(1, max(lengths or [1]))
+
+
+@pytest.mark.parametrize('n', [3, 70])
+def test_dense_lu_solves_more_right_hand_sides_than_a_grid_has_rows(n):
+    """65600 right-hand sides, beyond the 65535 workgroups of a launch's second
+    and third dimension: backward error of the worst of them, 50 n^(1/2)
+    roundings as above."""
+    from ceviche_amd._lib import lib, ptr, stream_ptr, check
+    g = torch.Generator().manual_seed(n)
+    A = torch.randn(n, n, generator=g, dtype=torch.complex128)
+    B = torch.randn(65600, n, generator=g, dtype=torch.complex128)
+    dev, x = A.t().contiguous().cuda(), B.cuda()
+    piv = torch.empty(n, dtype=torch.int32, device='cuda')
+    info = torch.zeros(1, dtype=torch.int32, device='cuda')
+    check(lib().cv_dense_lu(n, ptr(dev), ptr(piv), ptr(info), stream_ptr()), 'lu')
+    check(lib().cv_dense_lu_solve(n, ptr(dev), ptr(piv), ptr(x), B.shape[0], 0, stream_ptr()), 'solve')
+    X = x.cpu()
+    r = (X @ A.t() - B).norm(dim=1)
+    assert float((r / X.norm(dim=1)).max()) <= 50 * n ** 0.5 * 2.2e-16 * float(A.norm())
