@@ -991,7 +991,7 @@ __global__ void __launch_bounds__(256) k_efields_grad(Fdtd<R> f, const R* __rest
 // us with every neighbour through LDS, 30 operations a cell and an amplitude
 // load in each step).
 struct TmProbes {
-    const int32_t* comp;       // 2 Ez, 6 Hx, 7 Hy
+    const int32_t* comp;       // 2 Ez, 6 Hx, any other Hy
     const int64_t* cell;       // flat cells
     int n;
 };
@@ -1066,8 +1066,9 @@ __device__ __forceinline__ bool tm_probe_slots(const TmProbes& pr, int nx, int n
             pj = (int)(c - (int64_t)pi * ny);
         }
         const int r = pmod(pi - i0, nx), col = pmod(pj - j0, ny), k = pr.comp[p];
-        mine = r < RR && col < 64;
-        kk = k == 2 ? 0 : k - 5;
+        // a cell outside the grid is no tile's; s_slot has three components
+        mine = (uint64_t)c < (uint64_t)((int64_t)nx * ny) && r < RR && col < 64;
+        kk = k == 2 ? 0 : k == 6 ? 1 : 2;
         if (mine) {
             *s_any = 1;
             key = (unsigned)(kk << 12 | r << 6 | col);

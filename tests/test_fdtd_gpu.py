@@ -687,3 +687,30 @@ def test_gradient_passes_through_a_run_that_only_continues(shape, kernel, final)
     want = one.grad[:n1]
     assert float(want.norm()) > 0
     assert float((first.grad - want).norm()) <= 40 * len(amp0) * 2.0 ** -52 * float(one.grad.norm())
+
+
+@pytest.mark.parametrize('cfg', [0, 7])
+def test_tm_probes_beyond_the_grid_or_the_components_stay_in_bounds(cfg):
+    """Probe arrays are read on the device only: a component that is neither Ez
+    nor Hx records Hy, a cell outside the grid records nothing, and neither
+    touches another probe's record."""
+    import ceviche_amd as cv
+    print('tm probe bounds', cfg, flush=True)
+    nx, ny, steps = 40, 33, 20
+    rng = np.random.default_rng(2)
+    F = cv.fdtd(torch.from_numpy(rng.uniform(1, 6, (nx, ny, 1))).cuda(), 25e-9, [4, 4, 0])
+    g = F._grid
+    amp = torch.from_numpy(rng.standard_normal(steps)).cuda()
+    src, at = 20 * ny + 16, 21 * ny + 17
+    comp = [2, 6, 7, 8, 0, 5, 1000, -3, 2, 6, 7, 2]
+    cell = [at, at, at, at, at, at, at, at, -1, nx * ny, nx * ny + at, 1 << 40]
+    pt = (torch.tensor(comp, dtype=torch.int32, device='cuda'), torch.tensor(cell, dtype=torch.int64, device='cuda'))
+    rec = torch.full((steps, len(comp)), -77.0, dtype=torch.float64, device='cuda')
+    g.run_tm(g.new_state(), F._eps_dev, src, amp, 0, steps, pt, rec, 0, cfg)
+    want = F.run(steps, (20, 16, 0), amp, [('Ez', (21, 17, 0)), ('Hx', (21, 17, 0)), ('Hy', (21, 17, 0))], kernel='generic')
+    for p in range(len(comp)):
+        if p >= 8:
+            assert bool((rec[:, p] == -77.0).all()), p
+        else:
+            col = want[:, min(p, 2)]
+            assert float((rec[:, p] - col).norm()) <= 1e-12 * float(col.norm()), p
