@@ -148,6 +148,7 @@ _SIGS = {
     'cv_fdtd_tm_configs': (I, [P, P, P, I]),
     'cv_fdtd_run_fused': (I, [I, P, P, P, P, P, I, I64, P, I, I, P, P, I, P, I, P]),
     'cv_segsum': (I, [I64, P, P, P, P, P, I, I, D, D, P, I, P, P]),
+    'cv_segsum_unit': (I, [I64, P, P, P, P, I, I, D, D, P, I, P, P]),
     'cv_csr_solve_workspace_bytes': (I64, [I64]),
     'cv_csr_solve': (I, [I64, I, P, P, P, P, P, D, I, I, P, I64, P, P]),
     'cv_nd_plan_create': (P, [I, I]),

@@ -14,8 +14,8 @@
 namespace cv {
 
 // out[o(s)] (+)= alpha * sum_{q in [ptr[s], ptr[s+1])} opu(u[iu[q]]) * opv(v[iv[q]])
-// with o(s) = oidx ? oidx[s] : s and opu / opv optional conjugation; without
-// ptr (UNIT) segment s is entry s alone.  One thread per segment; the sum
+// with o(s) = oidx ? oidx[s] : s and opu / opv optional conjugation; UNIT:
+// segment s is entry s alone, no ptr.  One thread per segment; the sum
 // runs in storage order (deterministic).  Bound by the latency of index and
 // gather loads that follow each other, so four entries are in flight at a
 // time (1.3 million entries in 262144 rows: 52 -> 49 us; as unit segments,
@@ -525,20 +525,37 @@ __global__ void k_zero_i32(int32_t* p) { *p = 0; }
 
 using namespace cv;
 
-extern "C" int cv_segsum(int64_t n_seg, const int64_t* ptr, const int64_t* iu, const int64_t* iv, const void* u,
-                         const void* v, int conj_u, int conj_v, double alpha_re, double alpha_im,
-                         const int64_t* oidx, int accumulate, void* out, void* stream) {
+namespace cv {
+
+template <bool UNIT>
+static int segsum_impl(int64_t n_seg, const int64_t* ptr, const int64_t* iu, const int64_t* iv, const void* u,
+                       const void* v, int conj_u, int conj_v, double alpha_re, double alpha_im, const int64_t* oidx,
+                       int accumulate, void* out, hipStream_t s) {
     CV_CHECK(n_seg >= 0, "n_seg < 0");
-    CV_CHECK(u && v && out, "null pointer argument");
+    CV_CHECK((UNIT || ptr) && u && v && out, "null pointer argument");
     if (n_seg == 0) return CV_OK;
     const int64_t nb = (n_seg + 255) / 256;
     CV_CHECK(nb < (1ll << 31), "too many segments");
-    auto* kern = ptr ? k_segsum<false> : k_segsum<true>;
-    kern<<<(unsigned)nb, 256, 0, as_stream(stream)>>>(n_seg, ptr, iu, iv, (const cx<double>*)u, (const cx<double>*)v,
-                                                      conj_u, conj_v, mk(alpha_re, alpha_im), oidx, accumulate,
-                                                      (cx<double>*)out);
+    k_segsum<UNIT><<<(unsigned)nb, 256, 0, s>>>(n_seg, ptr, iu, iv, (const cx<double>*)u, (const cx<double>*)v, conj_u,
+                                                conj_v, mk(alpha_re, alpha_im), oidx, accumulate, (cx<double>*)out);
     CV_LAUNCH_CHECK();
     return CV_OK;
+}
+
+}  // namespace cv
+
+extern "C" int cv_segsum(int64_t n_seg, const int64_t* ptr, const int64_t* iu, const int64_t* iv, const void* u,
+                         const void* v, int conj_u, int conj_v, double alpha_re, double alpha_im,
+                         const int64_t* oidx, int accumulate, void* out, void* stream) {
+    return segsum_impl<false>(n_seg, ptr, iu, iv, u, v, conj_u, conj_v, alpha_re, alpha_im, oidx, accumulate, out,
+                              as_stream(stream));
+}
+
+extern "C" int cv_segsum_unit(int64_t n_seg, const int64_t* iu, const int64_t* iv, const void* u, const void* v,
+                              int conj_u, int conj_v, double alpha_re, double alpha_im, const int64_t* oidx,
+                              int accumulate, void* out, void* stream) {
+    return segsum_impl<true>(n_seg, nullptr, iu, iv, u, v, conj_u, conj_v, alpha_re, alpha_im, oidx, accumulate, out,
+                             as_stream(stream));
 }
 
 extern "C" int cv_dense_lu(int n, void* A, int32_t* piv, int32_t* info_dev, void* stream) {

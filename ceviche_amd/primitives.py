@@ -115,9 +115,13 @@ class Pattern:
 
 
 def segsum(n_seg, ptr_t, iu, iv, u, v, out, conj_u=False, conj_v=False, alpha=1.0, oidx=None, accumulate=False):
-    check(lib().cv_segsum(int(n_seg), ptr(ptr_t), ptr(iu), ptr(iv), ptr(u), ptr(v), int(conj_u), int(conj_v),
-                          float(np.real(alpha)), float(np.imag(alpha)), ptr(oidx), int(accumulate), ptr(out),
-                          stream_ptr()), 'segsum')
+    """Segmented product sum; ptr_t None: segments of one entry each."""
+    rest = (ptr(iu), ptr(iv), ptr(u), ptr(v), int(conj_u), int(conj_v), float(np.real(alpha)), float(np.imag(alpha)),
+            ptr(oidx), int(accumulate), ptr(out), stream_ptr())
+    if ptr_t is None:
+        check(lib().cv_segsum_unit(int(n_seg), *rest), 'segsum')
+    else:
+        check(lib().cv_segsum(int(n_seg), ptr(ptr_t), *rest), 'segsum')
     return out
 
 

@@ -443,17 +443,20 @@ int cv_fdtd_eps_grad(int dtype, const cv_fdtd_desc* d, const void* sig, const vo
 /* ---------------------------------------------------- generic sparse (COO) */
 /* Segmented product sum over complex128 vectors:
  *   out[o(s)] (+)= alpha * sum_{q = ptr[s]}^{ptr[s+1]-1} opu(u[iu[q]]) * opv(v[iv[q]])
- * o(s) = oidx[s] (or s when oidx is NULL), iu / iv NULL mean the identity, ptr
- * NULL segments of one entry (segment s holds entry s),
+ * o(s) = oidx[s] (or s when oidx is NULL), iu / iv NULL mean the identity,
  * opu / opv conjugate when conj_u / conj_v.  Deterministic (storage order).
  * With host-built groupings of the COO entries this is the CSR SpMV of
  * sp_mult (primitives.py:58-72), its A^T / A^H products and the gather
  * v[i]*x[j] (:74-86), the SpGEMM numerics of spsp_mult (:153-176) and its
  * VJP/JVP rules (:178-257), and the duplicate summation of make_sparse
- * (utils.py:13-25). */
+ * (utils.py:13-25).  cv_segsum_unit: segments of one entry each (segment s
+ * holds entry s), without a ptr. */
 int cv_segsum(int64_t n_seg, const int64_t* ptr, const int64_t* iu, const int64_t* iv,
               const void* u, const void* v, int conj_u, int conj_v, double alpha_re, double alpha_im,
               const int64_t* oidx, int accumulate, void* out, void* stream);
+int cv_segsum_unit(int64_t n_seg, const int64_t* iu, const int64_t* iv, const void* u, const void* v, int conj_u,
+                   int conj_v, double alpha_re, double alpha_im, const int64_t* oidx, int accumulate, void* out,
+                   void* stream);
 
 /* Solves A x = b for a general sparse complex128 matrix in CSR form
  * (indptr[n+1], indices, data: the arrays of a scipy.sparse.csr_matrix, int32

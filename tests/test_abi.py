@@ -33,3 +33,11 @@ def test_python_binding_covers_the_header():
 def test_version_string():
     from ceviche_amd import _lib
     assert b'gfx950' in _lib.lib().cv_version()
+
+
+def test_segsum_refuses_a_missing_segment_pointer():
+    from ceviche_amd import _lib
+    one = ctypes.cast(ctypes.create_string_buffer(64), ctypes.c_void_p)     # never read: the call ends at its checks
+    null = ctypes.c_void_p(0)
+    rc = _lib.lib().cv_segsum(2, null, null, null, one, one, 0, 0, 1.0, 0.0, null, 0, one, null)
+    assert rc != _lib.CV_OK and b'null pointer' in _lib.lib().cv_last_error()
