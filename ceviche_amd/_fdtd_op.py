@@ -336,14 +336,22 @@ def autotune_tm(grid, eps, steps=64, reps=2):
 
 def _probe_tensors(grid, probes):
     """(component int32, flat cell int64) device tensors of point probes."""
-    names, pos = zip(*probes) if probes else ((), ())
-    code = {c: COMPONENTS[c] if isinstance(c, str) else int(c) for c in set(names)}
+    names, pos = zip(*probes) if len(probes) else ((), ())
+    try:
+        kinds = set(names)
+    except TypeError:             # 0-d arrays
+        names = [c if isinstance(c, str) else int(c) for c in names]
+        kinds = set(names)
+    code = {c: COMPONENTS[c] if isinstance(c, str) else int(c) for c in kinds}
     comps = np.fromiter(map(code.__getitem__, names), np.int32, len(names))
     if set(map(len, pos)) - {3}:
         pos = [tuple(p) + (0,) * (3 - len(p)) for p in pos]
         if max(map(len, pos)) > 3:
             raise ValueError('a probe position has at most three indices')
-    xyz = np.fromiter(map(int, chain.from_iterable(pos)), np.int64, 3 * len(pos)).reshape(-1, 3)
+    try:
+        xyz = np.fromiter(map(int, chain.from_iterable(pos)), np.int64, 3 * len(pos)).reshape(-1, 3)
+    except OverflowError:
+        raise ValueError('a probe position is outside the grid %s' % (grid.shape,)) from None
     bad = ((xyz < 0) | (xyz >= np.array(grid.shape))).any(axis=1)
     if bad.any():
         raise ValueError('probe position %s outside the grid %s' % (tuple(pos[int(bad.argmax())]), grid.shape))

@@ -165,3 +165,27 @@ def test_value_and_shape_helpers():
     assert U.get_shape(1.0) == (1,) and U.get_shape(3) == (1,)
     assert U.get_shape([1, 2, 3]) == (3,) and U.get_shape((1, 2)) == (2,)
     assert U.get_shape(np.zeros((2, 7))) == (2, 7) and U.get_shape(torch.zeros(4, 1)) == (4, 1)
+
+
+def test_probe_positions_in_every_accepted_form():
+    """The probe list's conversion against one probe at a time: names as text,
+    codes and 0-d arrays, positions of one to three indices in lists, tuples,
+    arrays and floats, object arrays as the list; positions outside the grid
+    raise ValueError however large."""
+    import types
+    from ceviche_amd._fdtd_op import COMPONENTS, _probe_tensors
+    g = types.SimpleNamespace(nx=5, ny=6, nz=7, shape=(5, 6, 7), device='cpu')
+    table = np.empty((2, 2), dtype=object)
+    table[0, 0], table[0, 1], table[1, 0], table[1, 1] = 'Ez', (1, 2, 3), 'Hx', (2, 2)
+    for probes in ([], [('Ez', (1, 2, 3)), ('Hx', [0, 0, 0])], [('Ez', (1, 2)), ('Hy', (4,)), ('Ex', ())],
+                   [(2, (1, 2, 3)), (np.int64(6), [1, 1, 1])], [(np.array(2), (1, 2, 3)), ('Dz', (0, 5))],
+                   [(torch.tensor(7), (torch.tensor(1), 2, 3))], [('Ez', np.array([1, 2, 3])), ('Ez', (1.9, 2.2))], table):
+        pc, pl = _probe_tensors(g, probes)
+        assert pc.dtype == torch.int32 and pl.dtype == torch.int64
+        for k, (name, p) in enumerate(probes):
+            i, j, l = (int(v) for v in tuple(p) + (0,) * (3 - len(p)))
+            assert pc[k] == (COMPONENTS[name] if isinstance(name, str) else int(name))
+            assert pl[k] == (i * 6 + j) * 7 + l
+    for bad in ((5, 0, 0), (0, 0, 7), (-1, 0, 0), (10 ** 30, 0, 0), (1, 2, 3, 0)):
+        with pytest.raises(ValueError):
+            _probe_tensors(g, [('Ez', bad)])
