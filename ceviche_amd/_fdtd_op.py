@@ -390,7 +390,8 @@ class FdtdRun(torch.autograd.Function):
         if need_grad and isinstance(tm_config, int) and n_steps > 0:
             # whole launches per segment: the next lower multiple of the steps
             # a launch takes (a checkpoint is a third of a full state)
-            ts = tm_configs()[tm_config][2]
+            configs = tm_configs()
+            ts = configs[tm_config][2] if 0 <= tm_config < len(configs) else 1   # an unknown one is refused below
             ck = min(ck - ck % ts if ck > ts else ck, n_steps)
             checkpoints = grid.run_tm_checkpoints(state, eps, src[1], amp_dev, n_steps, ck, probes, rec, tm_config)
             t = n_steps

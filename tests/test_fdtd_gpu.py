@@ -714,3 +714,13 @@ def test_tm_probes_beyond_the_grid_or_the_components_stay_in_bounds(cfg):
         else:
             col = want[:, min(p, 2)]
             assert float((rec[:, p] - col).norm()) <= 1e-12 * float(col.norm()), p
+
+
+@pytest.mark.parametrize('cfg', [-1, 12, 99])
+@pytest.mark.parametrize('grad', [False, True])
+def test_unknown_tm_configuration_is_refused(cfg, grad):
+    import ceviche_amd as cv
+    from ceviche_amd._lib import CevicheError
+    F = cv.fdtd(torch.ones(30, 30, 1, dtype=torch.float64, device='cuda', requires_grad=grad), 25e-9, [3, 3, 0])
+    with pytest.raises(CevicheError):
+        F.run(5, (15, 15, 0), np.ones(5), [('Ez', (1, 1, 0))], kernel=cfg)
