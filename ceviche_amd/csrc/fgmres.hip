@@ -22,7 +22,7 @@
 namespace cv {
 
 constexpr int kFgMaxM = 64;                  // longest restart cycle
-constexpr int kFgSumFirst = 4096;            // workgroups above which the norm's partials are summed apart
+constexpr int kFgSumFirst = 3072;            // workgroups above which the norm's partials are summed apart
 
 // Cells per thread of the vector kernels: one below half a million cells,
 // where four leave most of the GPU idle and put four stencils in a row (28 us
@@ -387,8 +387,11 @@ static int fgmres_core(const cv_fdfd_desc* desc, const cv_fdfd_desc& dh, const v
             k_fg_reduce<<<2 * (j + 1), kBlock, 0, s>>>(w.partial, n_wg, 2 * (j + 1), h2, 0);
             (cpt == 1 ? k_fg_axpy<false, 1> : k_fg_axpy<false, 4>)<<<n_wg, kBlock, 0, s>>>(w.V, j + 1, h2, wv, n,
                                                                                           w.partial);
-            // each workgroup sums the partials of all: from 4096 workgroups
-            // on that would read more than the vector, so they are summed first
+            // Each workgroup sums the partials of all, out of its L2: from the
+            // second pass to the normalised vector 7.0 us at 1024 workgroups
+            // and 12.4 at 2198, where a launch of its own for the sum makes it
+            // 11.1 and 13.7; at 4089 it is 22.8 against 20.2, at 4307 25.3
+            // against 21.5.  The two meet near 3000.
             const bool sum_first = n_wg > kFgSumFirst;
             if (sum_first) k_fg_reduce<<<1, kBlock, 0, s>>>(w.partial, n_wg, 1, nrm + 1, 0);
             (cpt == 1 ? k_fg_normalize<1> : k_fg_normalize<4>)<<<n_wg, kBlock, 0, s>>>(

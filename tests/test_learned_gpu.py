@@ -200,7 +200,7 @@ def test_fgmres_steps_minimise_the_residual_at_every_vector_width(N):
     """Three Arnoldi steps: the residual must be the least over span{b, Ab,
     A^2 b}, which a complex128 least-squares problem gives.  One cell per
     thread up to 724^2 < 2^19 cells, four from 725^2 on; at 2100^2 the norm's
-    partials (more than 4096) are summed by a launch of their own.  The basis
+    partials (more than 3072) are summed by a launch of their own.  The basis
     is complex64: each of its vectors, orthogonalised twice, is off by a few
     2^-24 relative to the rest, and so are their images in the residual (norm
     at most |b|), so 3 * 8 * 2^-24 < 2e-6 bounds the difference."""
