@@ -427,3 +427,40 @@ def test_nested_dissection_root_above_1024_cells():
     print('  method', info['method'], 'iterations', info['iterations'], 'residual %.2e' % info['rel_residual'],
           flush=True)
     assert info.get('factor') == 'nd' and info['rel_residual'] <= 1e-10 and info['iterations'] <= 40
+
+
+@pytest.mark.parametrize('pol,shape', [('ez', (1201, 905)), ('hz', (905, 1201))])
+def test_large_odd_grids_satisfy_the_assembled_equations(pol, shape):
+    """Grids of more than a million cells, whose upper levels hold the largest
+    fronts and the products with the longest inputs: the returned field against
+    the oracle's matrix in FP64, the other components against the oracle's
+    differences of it, and the gradient of a linear functional with respect to
+    the source against the transposed matrix.  Residuals within the requested
+    1e-8 (one part in a thousand for the oracle's own rounding), in at most 40
+    FGMRES steps, which a factor with wrong entries would not do."""
+    import ceviche_amd as cv
+    print('large odd grid', pol, shape, flush=True)
+    dL, npml, tol = 50e-9, [20, 20], 1e-8
+    rng = np.random.default_rng(31)
+    eps = np.ones(shape)
+    eps[shape[0] // 3:2 * shape[0] // 3, shape[1] // 3:2 * shape[1] // 3] = rng.uniform(
+        1, 4, (2 * shape[0] // 3 - shape[0] // 3, 2 * shape[1] // 3 - shape[1] // 3))
+    src = np.zeros(shape, dtype=np.complex128)
+    src[shape[0] // 4, shape[1] // 2 - 10:shape[1] // 2 + 10] = 1.0
+    s = torch.from_numpy(src).cuda().requires_grad_(True)
+    F = (cv.fdfd_ez if pol == 'ez' else cv.fdfd_hz)(OMEGA, dL, torch.from_numpy(eps).cuda(), npml,
+                                                   solver_options=cv.SolverOptions(tol=tol, method='direct'))
+    fx, fy, fz = F.solve(s)
+    assert F.last_solve_info.get('factor') == 'nd' and F.last_solve_info['iterations'] <= 40
+    c = torch.from_numpy(rng.standard_normal(shape) + 1j * rng.standard_normal(shape)).cuda()
+    g, = torch.autograd.grad((c * fz).sum().real, s)
+    A = (R.make_A_ez if pol == 'ez' else R.make_A_hz)(OMEGA, dL, eps, npml)
+    z = fz.detach().cpu().numpy()
+    b = 1j * OMEGA * src.ravel()
+    assert np.linalg.norm(A @ z.ravel() - b) <= 1.001 * tol * np.linalg.norm(b)
+    mu = g.cpu().numpy().conj().ravel() / (1j * OMEGA)
+    cn = c.cpu().numpy().ravel()
+    assert np.linalg.norm(A.T @ mu - cn) <= 1.001 * tol * np.linalg.norm(cn)
+    want = (R.ez_to_hx_hy(OMEGA, dL, shape, npml, z) if pol == 'ez' else R.hz_to_ex_ey(OMEGA, dL, eps, npml, z))
+    for x, y in zip((fx, fy), want):
+        assert np.linalg.norm(x.detach().cpu().numpy().ravel() - y.ravel()) <= 1e-12 * np.linalg.norm(y)
