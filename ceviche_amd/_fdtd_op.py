@@ -196,17 +196,11 @@ class FdtdGrid:
             self._tmp = torch.empty((3,) + self.shape, dtype=self.dtype, device=self.device)
         return self._tmp
 
-    def adjoint(self, lam, eps, D_prev, gmE, probes=None, g_probe=None, D_t=None, src=None, g_src=None):
-        """Reverse one step in place (lam: after step t -> before step t).
-        With src = (comp, cell) and g_src (a one-element device tensor of the
-        grid dtype), g_src receives the cotangent of the point-source
-        amplitude added at this step."""
-        pc, pl = (None, None) if probes is None else probes
-        npb = 0 if probes is None else int(pc.numel())
-        comp, cell = (-1, 0) if src is None else (int(src[0]), int(src[1]))
+    def adjoint(self, lam, eps, D_prev, gmE):
+        """Reverse one step in place (lam: after the step -> before it)."""
         check(lib().cv_fdtd_adjoint_step(self.code, self._d(), ptr(self.sig), ptr(eps), ptr(lam), ptr(self.tmp()),
-                                         ptr(D_prev), ptr(gmE), ptr(pc), ptr(pl), npb, ptr(g_probe), ptr(D_t),
-                                         comp, cell, ptr(g_src), stream_ptr()), 'fdtd adjoint')
+                                         ptr(D_prev), ptr(gmE), None, None, 0, None, None, -1, 0, None,
+                                         stream_ptr()), 'fdtd adjoint')
 
     def step_history(self, state, hist, eps, src, amp_dev, n_steps):
         """Advance ``state`` (all but its D) n_steps with D of every step kept:

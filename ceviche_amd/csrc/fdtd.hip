@@ -11,7 +11,8 @@
 //
 // Coefficients (fdtd.py:265-311) are functions of the per-axis sigma profiles
 // sigH_a[n_a], sigD_a[n_a] (fdtd.py:224-263) and are formed in-kernel with the
-// reference's formula; interior cells (all sigma zero) use host-computed
+// reference's formula, in the adjoint and the temporally blocked 2D kernels
+// separated by axis; interior cells (all sigma zero) use host-computed
 // constants.
 #include "common.h"
 
@@ -1797,8 +1798,9 @@ __global__ void __launch_bounds__(256) k_fused(Fdtd<R> f, const R* __restrict__ 
 // Reads come from the old state A only and writes go to B (ping-pong), so
 // workgroup order does not matter; a chunk starts by recomputing H(i0-1).
 // DRAM traffic per cell-step: H, D, eps read and H, D written (52 B in
-// float32) plus the 1 / 14 and 1 / 62 halo fractions.  Same arithmetic as
-// h_cell / d_cell.
+// float32) plus the 1 / 14 and 1 / 62 halo fractions.  The update and its
+// coefficients (coef4) are those of k_h and k_d; which products are fused is
+// left to the compiler here, so single roundings differ.
 constexpr int kMRows = 16, kMLanes = 64;
 constexpr int kMOwnY = kMRows - 2, kMOwnZ = kMLanes - 2;
 
@@ -2046,8 +2048,9 @@ __global__ void __launch_bounds__(64 * kMRows / kMRpt) k_march(Fdtd<R> f, const 
 // recomputing H(i0-1).  HBM traffic per cell-step: H, D, eps read, H, D
 // written (52 B in float32, plus the PML integrals inside the PML); the halo
 // rows are re-read by the neighbouring band on the same XCD (consecutive
-// bands of a chunk are mapped to one XCD).  Same arithmetic as h_cell /
-// d_cell, term by term.
+// bands of a chunk are mapped to one XCD).  The update and its coefficients
+// (coef4) are those of k_h and k_d; which products are fused is left to the
+// compiler here, so single roundings differ.
 constexpr int kSlabMaxNz = 256;
 
 // Load / store at a 32-bit byte offset through a raw buffer resource over

@@ -1056,9 +1056,9 @@ k_nd_block_copy(const cx<float>* __restrict__ src, int64_t src_stride, int src_l
 //   down: input the work vector at the ring cells (x_B); x = y - output.
 // Bound by latency: index, gather and matrix loads of a launch follow each
 // other, so the first matrix loads are issued before the gather, and the tile
-// of a workgroup is chosen (nd_product) to keep many of them in flight.  The
-// 32 partial-sum and ring-sum launches these kernels used to need took a
-// third of an application at 1024^2.
+// of a workgroup is chosen (launch_mv, launch_mvt) to keep many of them in
+// flight.  The 32 partial-sum and ring-sum launches these kernels used to need
+// took a third of an application at 1024^2.
 struct NdProduct {
     const cx<float>* F;
     int m, row0, col0, nout, nin, k, b;

@@ -88,8 +88,8 @@ def test_factor_and_sweep_invert_the_block_tridiagonal_part(pol, shape, npml, bl
 def test_cyclic_reduction_tail_of_every_block_count(nx, ny):
     """Tails of 2 to 8 blocks, block sizes around the 16- and 32-wide tiles: one
     application against spsolve.  Elimination in complex64 is off by the order
-    of c 2^-24, c the condition number of the system; 100 of that is allowed
-    for the growth over the levels."""
+    of c 2^-24, c the condition number of the system; 10 of that is allowed
+    for the growth over the at most 6 levels."""
     from ceviche_amd._fdfd_op import Direct
     print('tail', nx, ny, flush=True)
     rng = np.random.default_rng(nx * 131 + ny)
