@@ -90,7 +90,8 @@ class fdtd:
         self._grid.desc.dt = self.dt
         self._as_torch = isinstance(new_eps, torch.Tensor)
         if self._as_torch:
-            self._eps_dev = new_eps.to(self._grid.device, self._tdtype)
+            # the kernels read it as a dense array: a transposed or expanded view is copied
+            self._eps_dev = new_eps.to(self._grid.device, self._tdtype).contiguous()
         else:
             self._eps_dev = torch.from_numpy(np.ascontiguousarray(new_eps, dtype=np.float64)).to(
                 self._grid.device, self._tdtype)

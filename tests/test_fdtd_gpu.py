@@ -725,3 +725,34 @@ def test_unknown_tm_configuration_is_refused(cfg, grad):
     F = cv.fdtd(torch.ones(30, 30, 1, dtype=torch.float64, device='cuda', requires_grad=grad), 25e-9, [3, 3, 0])
     with pytest.raises(CevicheError):
         F.run(5, (15, 15, 0), np.ones(5), [('Ez', (1, 1, 0))], kernel=cfg)
+
+
+@pytest.mark.parametrize('view', ['transposed', 'strided', 'expanded'])
+@pytest.mark.parametrize('shape', [(14, 11, 1), (9, 8, 6)])
+def test_eps_given_as_a_view_is_read_by_its_strides(shape, view):
+    """A transposed, a strided and an expanded eps against a dense copy of it:
+    records and gradients equal bit for bit."""
+    import ceviche_amd as cv
+    print('eps view', shape, view, flush=True)
+    rng = np.random.default_rng(8)
+    amp, src = rng.standard_normal(15), tuple(n // 2 for n in shape)
+    full = torch.from_numpy(rng.uniform(1, 6, (2 * shape[0], 2 * shape[1], shape[2]))).cuda()
+    out = []
+    for dense in (True, False):
+        if view == 'transposed':
+            base = full[:shape[1], :shape[0]].contiguous().requires_grad_(True)
+            eps = base.transpose(0, 1)
+        elif view == 'strided':
+            base = full.clone().requires_grad_(True)
+            eps = base[::2, ::2]
+        else:
+            base = full[:1, :1].contiguous().requires_grad_(True)
+            eps = base.expand(shape)
+        assert tuple(eps.shape) == shape and not eps.is_contiguous()
+        F = cv.fdtd(eps.contiguous() if dense else eps, 25e-9, [2, 2, 2 if shape[2] > 1 else 0])
+        rec = F.run(len(amp), src, amp, [('Ez', src), ('Hx', (3, 3, 0))], checkpoint_every=4)
+        f = F.forward()
+        g, = torch.autograd.grad((rec ** 2).sum() + (f['Ez'] ** 2).sum(), base)
+        out.append((rec.detach(), f['Hy'].detach(), g))
+    for x, y in zip(*out):
+        assert torch.equal(x, y)
