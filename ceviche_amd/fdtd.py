@@ -174,7 +174,8 @@ class fdtd:
         (nz == 1, Jz source, TE fields zero, Ez/Hx/Hy probes, <= 256 probes;
         tile shape from the autotuner) and the two-phase per-step kernels
         otherwise (measured faster than the single-pass kernels at 256^3:
-        280 us per step against 420 us for the slab-marching kernel);
+        301 us per step, recording included, against 433 us for the
+        slab-marching kernel);
         'generic' forces the two-phase kernels, 'fused' the single-pass
         kernel (slab-marching when nz is a multiple of 64 up to 256,
         x-marching tiles otherwise in 3D), an int a TM tile configuration."""
